@@ -41,6 +41,7 @@
 //
 // 16-bit NN with rows not in 16-byte groups (L % 8 != 0 or unaligned) uses an
 // LDS-transposing kernel with a separate split-K reduction.
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <functional>
@@ -55,6 +56,21 @@ namespace {
 
 constexpr int NTHR = 256;
 
+// 16-byte accesses of operands at any element alignment (an odd leading
+// dimension leaves every column at another offset): global_load_dwordx4 /
+// global_store_dwordx4 take element-aligned addresses, so ragged shapes run the
+// same kernels as aligned ones; a lane's word then straddles two lines now and
+// then.  NMF-HALS 20011 x 9973, k = 50: the element-wise loads that this
+// replaces made the products 833 and 777 us.
+typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef unsigned uintx4h __attribute__((ext_vector_type(4), aligned(2)));
+__device__ inline floatx4 ldf4(const float *p) { return *(const floatx4u *)p; }
+__device__ inline void stf4(float *p, floatx4 v) { *(floatx4u *)p = v; }
+__device__ inline uint4 ldh8(const uint16_t *p) {
+  const uintx4h v = *(const uintx4h *)p;
+  return uint4{v[0], v[1], v[2], v[3]};
+}
+
 // ---------------------------------------------------------------------------
 // Thin operand: B(g, c) for g < K, c < k.
 struct ThinDev {
@@ -66,7 +82,7 @@ struct ThinDev {
   unsigned dim[6];
   long ld[6];
   int k;
-  int vec;  // 16-byte loads valid at 4-aligned g (alignment and shape checked on the host)
+  int vec;  // one 16-byte load (times one entry per further KRP factor) gives four rows at 4-aligned g
 };
 
 __device__ inline float thin_at(const ThinDev &t, unsigned g, int c) {
@@ -96,7 +112,7 @@ __device__ inline floatx4 thin4(const ThinDev &t, long kb, long kend, int c) {
   if (c >= t.k) return v;
   if (t.vec && kb + 3 < kend) {
     if (t.nf == 0) {
-      v = *(const floatx4 *)(t.B + kb + t.ldb * c);
+      v = ldf4(t.B + kb + t.ldb * c);
     } else {
       unsigned rest = (unsigned)kb / t.dim[0];
       unsigned d0 = (unsigned)kb - rest * t.dim[0];
@@ -110,14 +126,14 @@ __device__ inline floatx4 thin4(const ThinDev &t, long kb, long kend, int c) {
           s *= t.f[q][d + t.ld[q] * c];
         }
       }
-      v = *(const floatx4 *)(t.f[0] + d0 + t.ld[0] * c);
+      v = ldf4(t.f[0] + d0 + t.ld[0] * c);
       v[0] *= s;
       v[1] *= s;
       v[2] *= s;
       v[3] *= s;
     }
     if (t.rowscale) {
-      floatx4 r = *(const floatx4 *)(t.rowscale + kb);
+      floatx4 r = ldf4(t.rowscale + kb);
       v[0] *= r[0];
       v[1] *= r[1];
       v[2] *= r[2];
@@ -187,8 +203,7 @@ struct StreamParams {
   long kchunk;  // k range of one blockIdx.y (multiple of the k step)
   int nsplit;
   float *part;
-  int avec;   // 16-byte loads of A valid (lda and base aligned)
-  int cvec;   // 16-byte stores of C valid
+  int shift;  // FP32 NN: the last four-row group of an L that is no multiple of 4 is rows L - 4 .. L - 1
   float oscale;  // every output element is multiplied by it (1: none; 16-bit products only)
 };
 
@@ -248,8 +263,8 @@ __device__ inline void store_acc_tn(const StreamParams &p, long l0, int a, float
   v[2] *= sc;
   v[3] *= sc;
   const int c = 16 * t + 4 * lg;
-  if (p.cmajor && p.cvec && c + 3 < p.th.k) {
-    *(floatx4 *)(p.C + c + p.ldc * l) = v;
+  if (p.cmajor && c + 3 < p.th.k) {
+    stf4(p.C + c + p.ldc * l, v);
   } else {
 #pragma unroll
     for (int u = 0; u < 4; ++u)
@@ -257,8 +272,11 @@ __device__ inline void store_acc_tn(const StreamParams &p, long l0, int a, float
   }
 }
 
+// First row of the FP32 NN four-row group at l (l % 4 == 0, l < L).
+__device__ inline long first_row(const StreamParams &p, long l) { return p.shift && l + 4 > p.L ? p.L - 4 : l; }
+
 // NN accumulator a = t*4 + j of a group starting at row l0:
-// v[u] = C(l0 + 16lg + 4u + j, 16t + lc).
+// v[u] = C(l0 + 16lg + 4u + j, 16t + lc) (first_row for a last partial group).
 __device__ inline void store_acc_nn(const StreamParams &p, long l0, int a, floatx4 v) {
   const int lane = threadIdx.x & 63, lc = lane & 15, lg = lane >> 4;
   const int t = a / 4, j = a % 4;
@@ -266,7 +284,9 @@ __device__ inline void store_acc_nn(const StreamParams &p, long l0, int a, float
   if (c >= p.th.k) return;
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
-    const long l = l0 + 16 * lg + 4 * u + j;
+    const long lq = l0 + 16 * lg + 4 * u;
+    if (lq >= p.L) continue;
+    const long l = first_row(p, lq) + j;
     if (l >= p.L) continue;
     if (p.cmajor)
       p.C[c + p.ldc * l] = v[u];
@@ -312,7 +332,7 @@ constexpr int EP_LD = 68;
 template <int NT>
 __device__ inline void epilogue_nn(const StreamParams &p, floatx4 (&acc)[4 * NT], long l0, float *ep) {
   const int lane = threadIdx.x & 63, lc = lane & 15, lg = lane >> 4;
-  if (ep && !p.cmajor && p.cvec && l0 + 63 < p.L) {
+  if (ep && !p.cmajor && l0 + 63 < p.L) {
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
 #pragma unroll
@@ -327,7 +347,7 @@ __device__ inline void epilogue_nn(const StreamParams &p, floatx4 (&acc)[4 * NT]
         const int cl = 4 * q + lg;  // column of this lane's 16 bytes
         const floatx4 o = *(const floatx4 *)(ep + cl * EP_LD + 4 * lc);
         const int c = 16 * t + cl;
-        if (c < p.th.k) *(floatx4 *)(p.C + l0 + 4 * lc + p.ldc * c) = o;
+        if (c < p.th.k) stf4(p.C + l0 + 4 * lc + p.ldc * c, o);
       }
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
@@ -342,16 +362,17 @@ __device__ inline void epilogue_nn(const StreamParams &p, floatx4 (&acc)[4 * NT]
     for (int v = 0; v < 4; ++v) {
       const long l = l0 + 16 * lg + 4 * v;
       floatx4 o = {acc[t * 4 + 0][v], acc[t * 4 + 1][v], acc[t * 4 + 2][v], acc[t * 4 + 3][v]};
-      if (!p.cmajor && p.cvec && l + 3 < p.L) {
-        *(floatx4 *)(p.C + l + p.ldc * c) = o;
+      if (!p.cmajor && l + 3 < p.L) {
+        stf4(p.C + l + p.ldc * c, o);
       } else {
+        const long ls = first_row(p, l);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          if (l + j >= p.L) continue;
+          if (l >= p.L || ls + j >= p.L) continue;
           if (p.cmajor)
-            p.C[c + p.ldc * (l + j)] = o[j];
+            p.C[c + p.ldc * (ls + j)] = o[j];
           else
-            p.C[l + j + p.ldc * c] = o[j];
+            p.C[ls + j + p.ldc * c] = o[j];
         }
       }
     }
@@ -425,7 +446,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_nn_kernel(StreamParams p, i
   for (; sp < p.nsplit; ++sp)
 #pragma unroll
     for (int h = 0; h < JW; ++h) s[h] += src[(long)sp * split_stride + 4 * 64 * h];
-  const bool fast = !p.cmajor && p.cvec && l0 + G <= p.L;  // uniform over the block
+  const bool fast = !p.cmajor && l0 + G <= p.L;  // uniform over the block
   if (!fast) {
 #pragma unroll
     for (int h = 0; h < JW; ++h) {
@@ -459,7 +480,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_nn_kernel(StreamParams p, i
 #pragma unroll
       for (int e = 0; e < 4; ++e) o[e] = o[e] * ((p.colscale ? p.colscale[l + e] : 1.0f) * p.oscale);
     }
-    *(floatx4 *)(p.C + l + p.ldc * c) = o;
+    stf4(p.C + l + p.ldc * c, o);
   }
 }
 
@@ -523,13 +544,13 @@ __device__ inline void thin_step(const ThinDev &th, long kb, const float *const 
                                  const float *const (&tf1)[NT], floatx4 (&a)[NT], float (&sc)[NT]) {
   if (TM == THIN_PLAIN) {
 #pragma unroll
-    for (int t = 0; t < NT; ++t) a[t] = *(const floatx4 *)(tb[t] + kb);
+    for (int t = 0; t < NT; ++t) a[t] = ldf4(tb[t] + kb);
   } else if (TM == THIN_KRP2) {
     const unsigned r = (unsigned)kb / th.dim[0];
     const unsigned d0 = (unsigned)kb - r * th.dim[0];
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      a[t] = *(const floatx4 *)(tb[t] + d0);
+      a[t] = ldf4(tb[t] + d0);
       sc[t] = tf1[t][r];
     }
   } else {
@@ -598,7 +619,7 @@ __global__ __launch_bounds__(NTHR) void tn_f32_kernel(StreamParams p) {
 #pragma unroll
     for (int cw = 0; cw < CW; ++cw) {
       if (TM != THIN_SAFE) {
-        b.x[cw] = *(const floatx4 *)(col[cw] + kb);
+        b.x[cw] = ldf4(col[cw] + kb);
       } else {
 #pragma unroll
         for (int u = 0; u < 4; ++u) b.x[cw][u] = col[cw][kb + u];
@@ -685,8 +706,8 @@ __global__ __launch_bounds__(NTHR) void tn_f32d_kernel(StreamParams p) {
     const long kb = kbeg + (kph + i * p.wk) * STEP + 8 * lg;
 #pragma unroll
     for (int cw = 0; cw < CW; ++cw) {
-      b.x[cw][0] = *(const floatx4 *)(col[cw] + kb);
-      b.x[cw][1] = *(const floatx4 *)(col[cw] + kb + 4);
+      b.x[cw][0] = ldf4(col[cw] + kb);
+      b.x[cw][1] = ldf4(col[cw] + kb + 4);
     }
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -772,6 +793,13 @@ __device__ inline void pack8(const floatx4 &lo, const floatx4 &hi, uint4 (&w)[NP
   }
 }
 
+// The thin operand written out: out(g, c) = B(g, c), K x k, ld K.
+__global__ __launch_bounds__(256) void form_thin_kernel(ThinDev th, long K, float *out) {
+  const int c = blockIdx.y;
+  for (long g = (long)blockIdx.x * 256 + threadIdx.x; g < K; g += (long)gridDim.x * 256)
+    out[g + K * c] = thin_at(th, (unsigned)g, c);
+}
+
 // One thread per (S, t, lane): both halves h of its column's 16 rows 64 S +
 // 16 (lane >> 4) .. + 15 (64 contiguous bytes: a wave reads whole 256-byte
 // column segments).
@@ -834,17 +862,17 @@ struct ThinProducer16 {
     if (krp2) {
       const unsigned q = (unsigned)kb / dim0;
       const unsigned d0 = (unsigned)kb - q * dim0;
-      r.a0 = *(const floatx4 *)(tb + d0);
-      r.a1 = *(const floatx4 *)(tb + d0 + 4);
+      r.a0 = ldf4(tb + d0);
+      r.a1 = ldf4(tb + d0 + 4);
       r.sc = tf1[q];
     } else {
-      r.a0 = *(const floatx4 *)(tb + kb);
-      r.a1 = *(const floatx4 *)(tb + kb + 4);
+      r.a0 = ldf4(tb + kb);
+      r.a1 = ldf4(tb + kb + 4);
       r.sc = 1.0f;
     }
     if (rs) {
-      r.r0 = *(const floatx4 *)(rs + kb);
-      r.r1 = *(const floatx4 *)(rs + kb + 4);
+      r.r0 = ldf4(rs + kb);
+      r.r1 = ldf4(rs + kb + 4);
     }
   }
   template <typename TA, int NT, int NP>
@@ -865,7 +893,7 @@ struct ThinProducer16 {
 // 16-bit TN.  DUAL = 0: step = 32 k, a lane reads 8 consecutive k of a
 // column (16 bytes); DUAL = 1: step = 64 k, a lane reads 16 consecutive k
 // (two 16-byte words, a full 128-byte line per column across the four lane
-// groups) feeding two MFMAs.  SAFE: scalar loads of A (unaligned lda/base).
+// groups) feeding two MFMAs.
 template <int NT, int CW, int NS, int NP>
 struct BufH {
   uint4 x[CW][NS];
@@ -874,7 +902,7 @@ struct BufH {
 
 // NP == 2: the compensated thin operand (two planes, both contracted with
 // the same A words into one accumulator).
-template <typename TA, int NT, int CW, int SAFE, int DUAL, int NP>
+template <typename TA, int NT, int CW, int DUAL, int NP>
 __global__ __launch_bounds__(NTHR) void tn_h_kernel(StreamParams p) {
   constexpr int NS = DUAL ? 2 : 1, STEP = 32 * NS, PD = DUAL ? 2 : 3, NA = CW * NT;
   constexpr int LW = 8 * NS;  // k per lane per step
@@ -922,14 +950,7 @@ __global__ __launch_bounds__(NTHR) void tn_h_kernel(StreamParams p) {
     for (int cw = 0; cw < CW; ++cw)
 #pragma unroll
       for (int h = 0; h < NS; ++h) {
-        if (!SAFE) {
-          b.x[cw][h] = *(const uint4 *)(col[cw] + kb + 8 * h);
-        } else {
-          uint16_t v[8];
-#pragma unroll
-          for (int u = 0; u < 8; ++u) v[u] = col[cw][kb + 8 * h + u];
-          b.x[cw][h] = __builtin_bit_cast(uint4, v);
-        }
+        b.x[cw][h] = ldh8(col[cw] + kb + 8 * h);
       }
     load_thin(kb, b);
   };
@@ -959,8 +980,9 @@ __global__ __launch_bounds__(NTHR) void tn_h_kernel(StreamParams p) {
 
 // ---------------------------------------------------------------------------
 // FP32 NN.  Step = 16 k; a wave owns 64 rows.  acc[t*4 + j][v] holds
-// C(l0 + 16lg + 4v + j, 16t + lc).  Fast modes need L % 4 == 0 (a lane's
-// four rows are in or out together; rows past L re-read rows L-4..L-1).
+// C(l0 + 16lg + 4v + j, 16t + lc).  Fast modes need L >= 4: a lane whose four
+// rows would pass L takes rows L-4 .. L-1 instead (with L % 4 != 0 those
+// overlap the lane before it: the same sums, stored twice; StreamParams::shift).
 template <int NT>
 struct BufNN {
   floatx4 x[4];
@@ -983,10 +1005,12 @@ __global__ __launch_bounds__(NTHR) void nn_f32_kernel(StreamParams p) {
   const long nfull = kend > kbeg ? (kend - kbeg) / STEP : 0;
   const float *A = (const float *)p.A;
   const long lr = l0 + 4 * lc;  // first of this lane's 4 rows
-  const float *base = A + (TM != THIN_SAFE ? (lr < p.L - 4 ? lr : p.L - 4) : 0);
+  // Fast modes (L >= 4): a lane past L - 4 takes rows L - 4 .. L - 1.
+  const long rb = lr < p.L - 4 ? lr : p.L - 4;
+  const float *base = A + (TM != THIN_SAFE ? rb : 0);
   long rows[4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) rows[j] = lr + j < p.L ? lr + j : p.L - 1;
+  for (int j = 0; j < 4; ++j) rows[j] = TM != THIN_SAFE ? rb + j : (lr + j < p.L ? lr + j : p.L - 1);
   const float *tb[NT], *tf1[NT];
   thin_cols<NT>(p.th, tb, tf1);
   floatx4 acc[NA];
@@ -1006,7 +1030,7 @@ __global__ __launch_bounds__(NTHR) void nn_f32_kernel(StreamParams p) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       if (TM != THIN_SAFE) {
-        b.x[u] = *(const floatx4 *)(base + p.lda * (kb + u));
+        b.x[u] = ldf4(base + p.lda * (kb + u));
       } else {
 #pragma unroll
         for (int j = 0; j < 4; ++j) b.x[u][j] = A[rows[j] + p.lda * (kb + u)];
@@ -1121,10 +1145,10 @@ struct ThinProducerF32 {
     if (TM == THIN_KRP2) {
       const unsigned q = (unsigned)kb / dim0;
       const unsigned d0 = (unsigned)kb - q * dim0;
-      r.a = *(const floatx4 *)(tb + d0);
+      r.a = ldf4(tb + d0);
       r.sc = tf1[q];
     } else {
-      r.a = *(const floatx4 *)(tb + kb);
+      r.a = ldf4(tb + kb);
       r.sc = 1.0f;
     }
   }
@@ -1158,7 +1182,8 @@ __global__ __launch_bounds__(NTHR) void nn_f32_sh_kernel(StreamParams p) {
   const long nfull = kend > kbeg ? (kend - kbeg) / STEP : 0;
   const float *A = (const float *)p.A;
   const long lr = l0 + 4 * lc;
-  const float *base = A + (lr < p.L - 4 ? lr : p.L - 4);
+  const long rb = lr < p.L - 4 ? lr : p.L - 4;  // a lane past L - 4 takes rows L - 4 .. L - 1
+  const float *base = A + rb;
   floatx4 acc[NA];
 #pragma unroll
   for (int a = 0; a < NA; ++a) acc[a] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -1169,7 +1194,7 @@ __global__ __launch_bounds__(NTHR) void nn_f32_sh_kernel(StreamParams p) {
   auto loadA = [&](long s, BufA &b) {
     const long kb = kbeg + s * STEP + 4 * lg;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) b.x[u] = *(const floatx4 *)(base + p.lda * (kb + u));
+    for (int u = 0; u < 4; ++u) b.x[u] = ldf4(base + p.lda * (kb + u));
   };
   auto rload = [&](long s, RawF32 &r) { prod.load(kbeg + s * STEP, r); };
   auto rstore = [&](const RawF32 &r, int stage) { prod.template store<NT>(r, ts, stage); };
@@ -1191,7 +1216,7 @@ __global__ __launch_bounds__(NTHR) void nn_f32_sh_kernel(StreamParams p) {
     // The partial last step, masked.
     long rows[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) rows[j] = lr + j < p.L ? lr + j : p.L - 1;
+    for (int j = 0; j < 4; ++j) rows[j] = rb + j;
     BufA b;
     const long kb = kbeg + nfull * STEP + 4 * lg;
 #pragma unroll
@@ -1247,7 +1272,7 @@ __global__ __launch_bounds__(NTHR) void tn_f32_sh_kernel(StreamParams p) {
   auto loadA = [&](long s, BufA &b) {
     const long kb = kbeg + s * STEP + 4 * lg;
 #pragma unroll
-    for (int cw = 0; cw < CW; ++cw) b.x[cw] = *(const floatx4 *)(col[cw] + kb);
+    for (int cw = 0; cw < CW; ++cw) b.x[cw] = ldf4(col[cw] + kb);
   };
   auto rload = [&](long s, RawF32 &r) { prod.load(kbeg + s * STEP, r); };
   auto rstore = [&](const RawF32 &r, int stage) { prod.template store<NT>(r, ts, stage); };
@@ -1335,7 +1360,7 @@ __global__ __launch_bounds__(NTHR) void tn_h_sh_kernel(StreamParams p) {
 #pragma unroll
     for (int cw = 0; cw < CW; ++cw)
 #pragma unroll
-      for (int h = 0; h < NS; ++h) b.x[cw][h] = *(const uint4 *)(col[cw] + kb + 8 * h);
+      for (int h = 0; h < NS; ++h) b.x[cw][h] = ldh8(col[cw] + kb + 8 * h);
   };
   auto rload = [&](long s, RawH &r) {
 #pragma unroll
@@ -1470,7 +1495,7 @@ __global__ __launch_bounds__(NTHR) void nn16_kernel(StreamParams p) {
   auto load = [&](long i, BufNN16<NT, NP> &b) {
     const long kb = kbeg + i * STEP + 8 * lg;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) b.w[u] = *(const uint4 *)(base + p.lda * (kb + u));
+    for (int u = 0; u < 8; ++u) b.w[u] = ldh8(base + p.lda * (kb + u));
 #pragma unroll
     for (int q = 0; q < NP; ++q)
 #pragma unroll
@@ -1491,7 +1516,7 @@ __global__ __launch_bounds__(NTHR) void nn16_kernel(StreamParams p) {
     auto loadA = [&](long i, BufA &b) {
       const long kb = kbeg + i * STEP + 8 * lg;
 #pragma unroll
-      for (int u = 0; u < 8; ++u) b.w[u] = *(const uint4 *)(base + p.lda * (kb + u));
+      for (int u = 0; u < 8; ++u) b.w[u] = ldh8(base + p.lda * (kb + u));
     };
     auto mma_st = [&](BufA &b, int stage) {
       uint4 bt[NP][NT];
@@ -1592,8 +1617,8 @@ __global__ __launch_bounds__(NTHR) void nn16_kernel(StreamParams p) {
 #pragma unroll
           for (int e = 0; e < 4; ++e) o[e] *= l + e < p.L ? p.colscale[l + e] : 1.0f;
         }
-        if (!p.cmajor && p.cvec && l + 3 < p.L) {
-          *(floatx4 *)(p.C + l + p.ldc * c) = o;
+        if (!p.cmajor && l + 3 < p.L) {
+          stf4(p.C + l + p.ldc * c, o);
         } else {
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
@@ -1843,6 +1868,16 @@ std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K,
   const long ksteps = (K + step - 1) / step;
   const int esz = dtype == PLANC_F32 ? 4 : 2;
   const double abytes = (double)L * (double)K * esz;
+  // K splits: the partial tiles' round trip may be 10% of A's bytes, or 8 MB
+  // (they stay in L2) where A is small and one pass of its few groups leaves
+  // most CUs idle; each wave keeps 8 k steps, 2 there (2000 x 1000, k = 20:
+  // 37 and 21 us products with one split of 32 waves).
+  const bool small = abytes <= (double)(64L << 20);
+  const long min_steps = small ? 2 : 8;
+  auto partials_fit = [&](const Geometry &g, double share) {
+    const double b = 2.0 * g.nsplit * g.groups * g.tile_bytes;
+    return b <= share * abytes || (small && b <= (double)(8L << 20));
+  };
   if (!trans && dtype != PLANC_F32) {
     // Streaming 16-bit NN: one k phase, K splits only; per-wave or
     // block-shared thin operand.
@@ -1854,8 +1889,8 @@ std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K,
       bool skipped = false, split_added = false;
       for (long ns = 1; ns <= 4096; ns *= 2) {
         Geometry g = make_geometry(L, K, trans, dtype, NT, 1, 1, ns, 0, sh);
-        if (ns > 1 && (g.nsplit < ns || ksteps / g.nsplit < 8)) break;
-        if (ns > 1 && 2.0 * g.nsplit * g.groups * g.tile_bytes > 0.10 * abytes) break;
+        if (ns > 1 && (g.nsplit < ns || ksteps / g.nsplit < min_steps)) break;
+        if (ns > 1 && !partials_fit(g, 0.10)) break;
         const long waves = g.blocks_x * 4 * g.nsplit;
         if (ns > 1 && waves > 16L * 1024) break;
         if (!out.empty() && waves < 2L * ctx->num_cu && ns < 4096) {
@@ -1889,7 +1924,7 @@ std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K,
     long ns = 1;
     while (g.blocks_x * 4 * ns < 4L * ctx->num_cu) {
       Geometry h = make_geometry(L, K, trans, dtype, NT, cw, wk, ns * 2);
-      if (2.0 * h.nsplit * h.groups * h.tile_bytes > 0.06 * abytes || ksteps / ((long)h.nsplit * wk) < 8) break;
+      if (!partials_fit(h, 0.06) || ksteps / ((long)h.nsplit * wk) < min_steps) break;
       ns *= 2;
       g = h;
     }
@@ -1903,8 +1938,8 @@ std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K,
       if (wk > 1 && ksteps < 8L * wk * (dual ? 2 : 1)) break;
       for (long ns = 1; ns <= 4096; ns *= 2) {
         Geometry g = make_geometry(L, K, trans, dtype, NT, cw, wk, ns, dual);
-        if (ns > 1 && (g.nsplit < ns || ksteps / ((long)g.nsplit * wk * (dual ? 2 : 1)) < 8)) break;
-        if (ns > 1 && 2.0 * g.nsplit * g.groups * g.tile_bytes > 0.10 * abytes) break;
+        if (ns > 1 && (g.nsplit < ns || ksteps / ((long)g.nsplit * wk * (dual ? 2 : 1)) < min_steps)) break;
+        if (ns > 1 && !partials_fit(g, 0.10)) break;
         const long waves = g.blocks_x * 4 * g.nsplit;
         if (ns > 1 && waves > 16L * 1024) break;
         if (waves < 2L * ctx->num_cu && ns < 4096) continue;  // too few waves: try more splits
@@ -1919,8 +1954,8 @@ std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K,
       const long sk = (K + sstep - 1) / sstep;
       for (long ns = 1; ns <= 4096; ns *= 2) {
         Geometry g = make_geometry(L, K, trans, dtype, NT, cw, 1, ns, 1, 1);
-        if (ns > 1 && (g.nsplit < ns || sk / g.nsplit < 8)) break;
-        if (ns > 1 && 2.0 * g.nsplit * g.groups * g.tile_bytes > 0.10 * abytes) break;
+        if (ns > 1 && (g.nsplit < ns || sk / g.nsplit < min_steps)) break;
+        if (ns > 1 && !partials_fit(g, 0.10)) break;
         const long waves = g.blocks_x * 4 * g.nsplit;
         if (ns > 1 && waves > 16L * 1024) break;
         if (waves < 2L * ctx->num_cu && ns < 4096) continue;
@@ -1930,8 +1965,8 @@ std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K,
   return out;
 }
 
-int thin_mode(const ThinDev &th, bool avec, const float *rowscale) {
-  if (!avec || rowscale || !th.vec) return THIN_SAFE;
+int thin_mode(const ThinDev &th, const float *rowscale) {
+  if (rowscale || !th.vec) return THIN_SAFE;
   if (th.nf <= 1) return THIN_PLAIN;
   if (th.nf == 2) return THIN_KRP2;
   return THIN_SAFE;
@@ -1960,13 +1995,11 @@ void launch_nn_f32(int tm, dim3 grid, hipStream_t st, const StreamParams &p) {
     nn_f32_kernel<NT, THIN_SAFE><<<grid, NTHR, 0, st>>>(p);
 }
 template <typename TA, int NT, int NP>
-void launch_tn_h(bool safe, int dual, dim3 grid, hipStream_t st, const StreamParams &p) {
-  if (safe)
-    tn_h_kernel<TA, NT, 4, 1, 0, NP><<<grid, NTHR, 0, st>>>(p);
-  else if (dual)
-    tn_h_kernel<TA, NT, 4, 0, 1, NP><<<grid, NTHR, 0, st>>>(p);
+void launch_tn_h(int dual, dim3 grid, hipStream_t st, const StreamParams &p) {
+  if (dual)
+    tn_h_kernel<TA, NT, 4, 1, NP><<<grid, NTHR, 0, st>>>(p);
   else
-    tn_h_kernel<TA, NT, 4, 0, 0, NP><<<grid, NTHR, 0, st>>>(p);
+    tn_h_kernel<TA, NT, 4, 0, NP><<<grid, NTHR, 0, st>>>(p);
 }
 template <int NT, int CW>
 void launch_tn_f32_sh(int tm, dim3 grid, hipStream_t st, const StreamParams &p) {
@@ -2021,17 +2054,16 @@ void launch_tn16(int dtype, int NT, const Geometry &g, dim3 grid, hipStream_t st
     }
     return;
   }
-  const bool safe = !p.avec;
   if (dtype == PLANC_BF16) {
-    if (NT == 1) launch_tn_h<bf16_t, 1, NP>(safe, g.dual, grid, st, p);
-    else if (NT == 2) launch_tn_h<bf16_t, 2, NP>(safe, g.dual, grid, st, p);
-    else if (NT == 3) launch_tn_h<bf16_t, 3, NP>(safe, g.dual, grid, st, p);
-    else launch_tn_h<bf16_t, 4, NP>(safe, g.dual, grid, st, p);
+    if (NT == 1) launch_tn_h<bf16_t, 1, NP>(g.dual, grid, st, p);
+    else if (NT == 2) launch_tn_h<bf16_t, 2, NP>(g.dual, grid, st, p);
+    else if (NT == 3) launch_tn_h<bf16_t, 3, NP>(g.dual, grid, st, p);
+    else launch_tn_h<bf16_t, 4, NP>(g.dual, grid, st, p);
   } else {
-    if (NT == 1) launch_tn_h<f16_t, 1, NP>(safe, g.dual, grid, st, p);
-    else if (NT == 2) launch_tn_h<f16_t, 2, NP>(safe, g.dual, grid, st, p);
-    else if (NT == 3) launch_tn_h<f16_t, 3, NP>(safe, g.dual, grid, st, p);
-    else launch_tn_h<f16_t, 4, NP>(safe, g.dual, grid, st, p);
+    if (NT == 1) launch_tn_h<f16_t, 1, NP>(g.dual, grid, st, p);
+    else if (NT == 2) launch_tn_h<f16_t, 2, NP>(g.dual, grid, st, p);
+    else if (NT == 3) launch_tn_h<f16_t, 3, NP>(g.dual, grid, st, p);
+    else launch_tn_h<f16_t, 4, NP>(g.dual, grid, st, p);
   }
 }
 template <int NT, int CW>
@@ -2137,7 +2169,7 @@ bool stream_capturing(hipStream_t st) {
 
 // Picks the geometry of a product shape: cached per context; otherwise
 // every candidate is timed on the live operands (one warm-up launch and two
-// timed launches each; the products are idempotent) unless tuning is off
+// or eight timed launches each; the products are idempotent) unless tuning is off
 // (PLANC_AUTOTUNE=0) or the stream is being captured into a graph, where the
 // static choice is used.  PLANC_TUNE_LOG=1 prints each candidate's time.
 // fly_ok: the shared 16-bit NN kernel may form its thin operand on the fly
@@ -2155,7 +2187,7 @@ int pick_geometry(planc_ctx *ctx, int dtype, int trans, int NT, int tm, const St
   const char *venv = getenv("PLANC_STREAM_VARIANT");
   const std::string vs = venv ? venv : "";
   const int smode = vs == "plain" ? 0 : (vs == "shared" ? 1 : (vs == "dual" ? 3 : (vs == "fly" ? 4 : 2)));
-  const std::vector<long> key = {dtype, trans, NT, tm, p.L, p.K, p.lda, p.th.k, p.avec, p.cmajor, smode, p.np,
+  const std::vector<long> key = {dtype, trans, NT, tm, p.L, p.K, p.lda, p.th.k, p.cmajor, smode, p.np,
                                  fly_ok ? 1 : 0};
   for (const auto &e : ctx->gemm_tuned)
     if (e.first == key) {
@@ -2163,7 +2195,7 @@ int pick_geometry(planc_ctx *ctx, int dtype, int trans, int NT, int tm, const St
       *out = make_geometry(p.L, p.K, trans, dtype, NT, (int)v[0], (int)v[1], v[2], (int)v[3], (int)v[4]);
       return PLANC_OK;
     }
-  const bool shared_ok = (dtype == PLANC_F32 ? tm != THIN_SAFE : p.avec != 0) && smode != 0 && smode != 3;
+  const bool shared_ok = (dtype != PLANC_F32 || tm != THIN_SAFE) && smode != 0 && smode != 3;
   std::vector<Geometry> cands = candidate_geometries(ctx, p.L, p.K, trans, dtype, NT, shared_ok,
                                                      dtype == PLANC_F32 && tm != THIN_SAFE, fly_ok && shared_ok);
   if (smode != 2) {
@@ -2172,6 +2204,16 @@ int pick_geometry(planc_ctx *ctx, int dtype, int trans, int NT, int tm, const St
       if (smode == 4 ? g.shared == 2
                      : smode == 1 ? g.shared != 0 : (g.shared == 0 && (smode == 3) == (g.dual != 0)))
         sel.push_back(g);
+    if (!sel.empty()) cands.swap(sel);
+  }
+  // FP32 operands off the 16-byte grid: chains of at most 1024 k per
+  // accumulator where the candidates have them (one 4986-k chain per row of a
+  // 20011 x 9973 product was 12% faster than sixteen of 623, and left NMF-HALS
+  // factors five times as far from FP64 as those did).
+  if (dtype == PLANC_F32 && (p.lda % 4 != 0 || (uintptr_t)p.A % 16 != 0)) {
+    std::vector<Geometry> sel;
+    for (const Geometry &g : cands)
+      if (g.kchunk <= 1024L * g.wk) sel.push_back(g);
     if (!sel.empty()) cands.swap(sel);
   }
   const char *env = getenv("PLANC_AUTOTUNE");
@@ -2183,7 +2225,10 @@ int pick_geometry(planc_ctx *ctx, int dtype, int trans, int NT, int tm, const St
     hipEvent_t e0, e1;
     PLANC_HIP_CHECK(ctx, hipEventCreate(&e0));
     PLANC_HIP_CHECK(ctx, hipEventCreate(&e1));
-    float pack_ms = 0.0f;  // two pack launches, as each candidate is timed over two launches
+    // Launches timed per candidate: two of a large product, eight of one that
+    // takes microseconds (A up to 64 MB).
+    const int reps = (double)p.L * (double)p.K * (dtype == PLANC_F32 ? 4 : 2) <= (double)(64L << 20) ? 8 : 2;
+    float pack_ms = 0.0f;  // as many pack launches
     if (dtype != PLANC_F32) {
       int prc = pack();
       if (prc) return prc;
@@ -2191,7 +2236,7 @@ int pick_geometry(planc_ctx *ctx, int dtype, int trans, int NT, int tm, const St
       for (const Geometry &g : cands) any_fly = any_fly || g.shared == 2;
       if (any_fly) {
         PLANC_HIP_CHECK(ctx, hipEventRecord(e0, ctx->stream));
-        for (int r = 0; r < 2 && !prc; ++r) prc = pack();
+        for (int r = 0; r < reps && !prc; ++r) prc = pack();
         if (prc) return prc;
         PLANC_HIP_CHECK(ctx, hipEventRecord(e1, ctx->stream));
         PLANC_HIP_CHECK(ctx, hipEventSynchronize(e1));
@@ -2204,7 +2249,7 @@ int pick_geometry(planc_ctx *ctx, int dtype, int trans, int NT, int tm, const St
       int rc = launch_stream(ctx, dtype, trans, NT, tm, p, g);  // warm-up (and workspace growth)
       if (rc) return rc;
       PLANC_HIP_CHECK(ctx, hipEventRecord(e0, ctx->stream));
-      for (int r = 0; r < 2; ++r) {
+      for (int r = 0; r < reps; ++r) {
         rc = launch_stream(ctx, dtype, trans, NT, tm, p, g);
         if (rc) return rc;
       }
@@ -2213,10 +2258,13 @@ int pick_geometry(planc_ctx *ctx, int dtype, int trans, int NT, int tm, const St
       float ms = 0.0f;
       PLANC_HIP_CHECK(ctx, hipEventElapsedTime(&ms, e0, e1));
       if (g.shared != 2) ms += pack_ms;
+      // Launched back to back a reduction of the K splits costs less than in a
+      // loop of dependent small kernels: 2 us is what a launch more takes there.
+      if (g.nsplit > 1) ms += 0.002f * reps;
       if (log)
         fprintf(stderr,
                 "planc tune dtype %d trans %d L %ld K %ld k %d: cw %d wk %d nsplit %ld dual %d shared %d -> %.2f us\n",
-                dtype, trans, p.L, p.K, p.th.k, g.cw, g.wk, (long)g.nsplit, g.dual, g.shared, ms * 500.0f);
+                dtype, trans, p.L, p.K, p.th.k, g.cw, g.wk, (long)g.nsplit, g.dual, g.shared, ms * 1000.0f / reps);
       if (!have || ms < best_ms) {
         best_ms = ms;
         best = g;
@@ -2237,7 +2285,7 @@ int fill_thin(planc_ctx *ctx, ThinDev &th, const float *B, long ldb, const KrpDe
   th = ThinDev{};
   th.k = kc;
   th.rowscale = rowscale;
-  bool vec = rowscale == nullptr || ((uintptr_t)rowscale % 16 == 0);
+  bool vec = true;
   if (krp && krp->nf > 0) {
     if (krp->nf > 6) return set_error(ctx, PLANC_EINVAL, "thin_gemm: more than 6 KRP factors");
     long prod = 1;
@@ -2250,14 +2298,13 @@ int fill_thin(planc_ctx *ctx, ThinDev &th, const float *B, long ldb, const KrpDe
       th.dim[q] = (unsigned)krp->dim[q];
       th.ld[q] = krp->ld[q];
     }
-    vec = vec && krp->dim[0] % 4 == 0 && krp->ld[0] % 4 == 0 && ((uintptr_t)krp->f[0] % 16 == 0);
+    vec = krp->nf == 1 || krp->dim[0] % 4 == 0;  // four consecutive rows share the further factors' entries
   } else {
     if (!B) return set_error(ctx, PLANC_EINVAL, "thin_gemm: null B");
     if (K >= (1L << 32)) return set_error(ctx, PLANC_EINVAL, "thin_gemm: K too large");
     th.nf = 0;
     th.B = B + ldb * c0;
     th.ldb = ldb;
-    vec = vec && ldb % 4 == 0 && ((uintptr_t)B % 16 == 0);
   }
   th.vec = vec ? 1 : 0;
   return PLANC_OK;
@@ -2293,7 +2340,7 @@ int thin_gemm(planc_ctx *ctx, int dtype, int trans, const void *A, long lda, lon
                                             ctx->stream));
       continue;
     }
-    if (dtype != PLANC_F32 && !trans && !(avec && L % 8 == 0)) {
+    if (dtype != PLANC_F32 && !trans && L % 8 != 0) {
       // 16-bit NN with rows that do not come in 16-byte groups: the
       // LDS-transposing kernel.
       GemmParams p{};
@@ -2372,11 +2419,30 @@ int thin_gemm(planc_ctx *ctx, int dtype, int trans, const void *A, long lda, lon
     p.C = Cs;
     p.ldc = ldc;
     p.cmajor = cmajor;
-    p.avec = avec ? 1 : 0;
-    p.cvec = (ldc % 4 == 0 && ((uintptr_t)Cs % 16 == 0)) ? 1 : 0;
     p.oscale = oscale;
-    int tm = thin_mode(th, avec, rowscale);
-    if (!trans && L % 4 != 0) tm = THIN_SAFE;
+    // FP32 with a Khatri-Rao operand that the kernels cannot form from one
+    // 16-byte load per four rows (three or more factors, a ragged first one,
+    // row scales): the K x k operand is written out once in FP32, while that
+    // stays small beside A (or small outright), and read as a plain one.  Its
+    // entries are the products that the kernels would form element by element
+    // per use (61 x 53 x 47 x 35, k = 17: 205 and 45 us products).
+    if (dtype == PLANC_F32 && thin_mode(th, rowscale) == THIN_SAFE &&
+        (L >= 2L * kc || K * kc <= (4L << 20))) {
+      float *kr = (float *)ws_get(ctx, 6, sizeof(float) * (size_t)K * kc);
+      if (!kr) return set_error(ctx, PLANC_ENOMEM, "thin_gemm: Khatri-Rao operand");
+      form_thin_kernel<<<dim3((unsigned)std::min<long>((K + 255) / 256, 4096), (unsigned)kc), 256, 0, ctx->stream>>>(
+          th, K, kr);
+      PLANC_LAUNCH_CHECK(ctx);
+      th = ThinDev{};
+      th.k = kc;
+      th.B = kr;
+      th.ldb = K;
+      th.vec = 1;
+      p.th = th;
+    }
+    int tm = thin_mode(th, th.rowscale);
+    if (!trans && L < 4) tm = THIN_SAFE;
+    p.shift = dtype == PLANC_F32 && !trans && tm != THIN_SAFE && L % 4 != 0;
     // 16-bit TN / NN: the thin operand packed into the 16-bit MFMA operand
     // layout (8 consecutive k of one column per lane) once per product,
     // unless the chosen kernel forms it on the fly.
