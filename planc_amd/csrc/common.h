@@ -120,7 +120,8 @@ namespace planc {
 // 10 BPP per-column iteration counts, 11 BPP failure flag, 12 CP-loss scalar,
 // 13 CP-gradient float buffers, 14 CP-gradient Grams, 15 loop-graph counter,
 // 16 transposed 16-bit copy of A / X, 17 HALS grid-barrier counter and flag,
-// 18 NTF mode-update partials (two-launch form), 19/21 (unused), 20 (unused), 22 AO-ADMM factor / partials,
+// 18 NTF mode-update partials (two-launch form), 19 / 20 the pieces of A's / A^T's long rows and 21 their
+// partial sums (sparse.hip), 22 AO-ADMM factor / partials,
 // 23 GNSym CG vectors, 24..31 sparse path (sparse.hip: k-major factor
 // copies, error partials, transposed CSR, sort keys / entries / temporary
 // storage), 32 NTF AO-ADMM duals, 33 NMF AO-ADMM duals, 34 dual norms,
@@ -268,15 +269,24 @@ int cp_loss_forward(planc_ctx *ctx, const float *X, int N, const long *dims, con
                     int k, double *d_loss);
 // Sparse (CSR) products of the sparse-input NMF (sparse.hip).  SparseOps
 // holds the CSR of A^T built once per run.
+// The long rows of a CSR cut into pieces (sparse.hip): device counts and
+// descriptors, with what they can hold.
+struct SpmmPlan {
+  int *cnt = nullptr;
+  void *seg = nullptr;
+  long segs = 0, parts = 0;
+};
 struct SparseOps {
+  SpmmPlan plan, t_plan;  // of A and of A^T
   const long *t_indptr = nullptr;
   const int *t_indices = nullptr;
   const float *t_values = nullptr;
 };
 int csr_transpose(planc_ctx *ctx, long m, long n, long nnz, const long *indptr, const int *indices,
                   const float *values, long *out_indptr, int *out_indices, float *out_values);
-int spmm_csr(planc_ctx *ctx, long rows, const long *indptr, const int *indices, const float *values,
-             const float *F, long ldf, int k, float *out, long ors, long ocs);
+int spmm_plan(planc_ctx *ctx, int slot, long rows, const long *indptr, long nnz, SpmmPlan *plan);
+int spmm_csr(planc_ctx *ctx, const SpmmPlan &plan, long rows, const long *indptr, const int *indices,
+             const float *values, const float *F, long ldf, int k, float *out, long ors, long ocs);
 int spmm_colmajor(planc_ctx *ctx, long rows, long cols, const long *indptr, const int *indices,
                   const float *values, const float *F, long ldf, int k, float *out, long ldo);
 int sparse_fit_error(planc_ctx *ctx, long m, long n, const long *indptr, const int *indices,

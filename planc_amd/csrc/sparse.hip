@@ -6,9 +6,17 @@
 // analogue of the reference's At = A.t() in the constructors).
 //
 // Products: out(r, :) = sum_e val(e) F(col(e), :) over the entries of row r
-// (SpMM), one wavefront per row, lane c holding output column c; the dense
-// factor is read from a row-major (k-major) copy so every entry gathers one
-// contiguous row of F.  Entries are summed in CSR order in FP32.
+// (SpMM), FP32 sums; the dense factor is read from a row-major (k-major) copy
+// so every entry gathers one contiguous row of F, 16 bytes a lane.  Bound by
+// the gathers' latency and L2 rate, so what counts is entries in flight, on
+// rows whose lengths follow a power law: rows of up to SP_SHORT entries are
+// walked by a lane group each (several rows per wavefront), longer ones are
+// cut into segments of SP_SEG entries that a whole wavefront walks, its groups
+// taking entries in turn, and a row's segments are added in order.  Term-
+// document matrix 100000 x 40000, 2.6 M entries, k = 32 (its longest row has
+// 40000): a wavefront per row walking its entries one by one took 4983 us a
+// product, this takes 28 and 5.6 to add the pieces; a run of five MU
+// iterations 51.1 -> 0.97 ms.
 //
 // Also the sparse error helper of common/utils.hpp:190-241 (sum over the
 // non-zeros of (a_ij - w_i h_j)^2 and of (w_i h_j)^2, plus ||W H^T||_F^2).
@@ -19,7 +27,6 @@
 // After common.h: hipCUB picks its backend from the platform macro that
 // hip_runtime.h defines.
 #include <hipcub/device/device_radix_sort.hpp>
-#include <hipcub/device/device_scan.hpp>
 
 namespace planc {
 
@@ -39,48 +46,186 @@ __global__ void iota_kernel(long n, int *v) {
   if (e < n) v[e] = (int)e;
 }
 
-__global__ void col_count_kernel(long nnz, const int *indices, int *cnt) {
-  long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < nnz) atomicAdd(&cnt[indices[e]], 1);
-}
-
-__global__ void set_long_kernel(long *p, long v) { *p = v; }
-
-__global__ void csr_t_gather_kernel(long nnz, const int *ent, const int *rowid, const float *values,
-                                    int *out_indices, float *out_values) {
+// Entries of A^T in their sorted order, and its row pointers where the sorted
+// column changes (each thread writes those of the columns that begin at its
+// entry, empty ones among them; the last entry's thread the ones behind it).
+__global__ void csr_t_gather_kernel(long nnz, long n, const int *ent, const unsigned *key, const int *rowid,
+                                    const float *values, int *out_indices, float *out_values, long *out_indptr) {
   long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= nnz) return;
   const int e = ent[p];
   out_indices[p] = rowid[e];
   out_values[p] = values[e];
+  const long c = key[p];
+  for (long q = p > 0 ? (long)key[p - 1] + 1 : 0; q <= c; ++q) out_indptr[q] = p;
+  if (p == nnz - 1)
+    for (long q = c + 1; q <= n; ++q) out_indptr[q] = nnz;
 }
 
-// out(r, c) at out[r * ors + c * ocs] = sum over row r's entries of
-// val(e) * F(col(e), c), F k-major (element (j, c) at F[j * ldf + c]).
-__global__ __launch_bounds__(256) void spmm_rows_kernel(long rows, const long *indptr, const int *indices,
-                                                         const float *values, const float *F, long ldf,
-                                                         int k, float *out, long ors, long ocs) {
-  const long r = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+constexpr int SP_SHORT = 64;
+constexpr int SP_SEG = 512;
+
+// A piece of a row longer than SP_SHORT: entries part * SP_SEG .. of row
+// `row`; with nseg > 1 its sums go to partial row pslot, the row's pieces in
+// consecutive ones.
+struct SpSeg {
+  int row, part, nseg, pslot;
+};
+
+__global__ void spmm_plan_zero_kernel(int *cnt) {
+  if (threadIdx.x < 2) cnt[threadIdx.x] = 0;
+}
+
+// cnt[0] pieces and cnt[1] partial rows.  Their order depends on the atomics,
+// the values computed from them do not.
+__global__ void spmm_plan_kernel(long rows, const long *indptr, int *cnt, SpSeg *seg) {
+  const long r = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= rows) return;
-  const int lane = threadIdx.x & 63;
-  const long b = indptr[r], e = indptr[r + 1];
-  const bool active = lane < k;
-  float acc = 0.0f;
-  for (long base = b; base < e; base += 64) {
-    int j = 0;
-    float v = 0.0f;
-    if (base + lane < e) {
-      j = indices[base + lane];
-      v = values[base + lane];
+  const long len = indptr[r + 1] - indptr[r];
+  if (len <= SP_SHORT) return;
+  const int ns = (int)((len + SP_SEG - 1) / SP_SEG);
+  const int slot = atomicAdd(&cnt[0], ns);
+  const int ps = ns > 1 ? atomicAdd(&cnt[1], ns) : 0;
+  for (int p = 0; p < ns; ++p) seg[slot + p] = SpSeg{(int)r, p, ns, ps + p};
+}
+
+__device__ inline void spmm_store4(float *out, long r, int c, int k, long ors, long ocs, floatx4 v) {
+  if (ocs == 1 && c + 3 < k) {
+    typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
+    *(floatx4u *)(out + r * ors + c) = v;
+    return;
+  }
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+    if (c + u < k) out[r * ors + (c + u) * ocs] = v[u];
+}
+
+// out(r, c) at out[r * ors + c * ocs], F k-major (element (j, c) at F[j * ldf
+// + c], ldf a multiple of 4).  G lanes (4 G >= k) hold an output row, four
+// columns each.  PLAN: blocks below nsegb walk the pieces, the others the short
+// rows.  Without a plan (nsegb 0: a single product whose entry count the host
+// does not know) a block walks the long ones among its rows afterwards, its
+// four wavefronts together.
+template <int G, bool PLAN>
+__global__ __launch_bounds__(256) void spmm_kernel(long rows, const long *indptr, const int *indices,
+                                                   const float *values, const float *F, long ldf, int k, float *out,
+                                                   long ors, long ocs, int nsegb, const int *cnt, const SpSeg *seg,
+                                                   float *partial) {
+  constexpr int NG = 64 / G;  // groups per wavefront
+  constexpr int U = 4;        // entries in flight per group
+  const int lane = threadIdx.x & 63, gl = lane % G, grp = lane / G;
+  const int c = 4 * gl < ldf ? 4 * gl : 0;  // lanes past the row re-read its first columns (not stored)
+  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+  // Entries e0, e0 + st, ... below e1.
+  auto walk = [&](long e0, long e1, int st) {
+    long e = e0;
+    for (; e + (U - 1) * st < e1; e += U * st) {
+      int j[U];
+      float v[U];
+      floatx4 f[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        j[u] = indices[e + u * st];
+        v[u] = values[e + u * st];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) f[u] = *(const floatx4 *)(F + (long)j[u] * ldf + c);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[q] = fmaf(v[u], f[u][q], acc[q]);
     }
-    const int cnt = (int)((e - base) < 64 ? (e - base) : 64);
-    for (int t = 0; t < cnt; ++t) {
-      const int jt = __shfl(j, t, 64);
-      const float vt = __shfl(v, t, 64);
-      if (active) acc += vt * F[(long)jt * ldf + lane];
+    if (e < e1) {  // the rest, in flight together: entries past the end weigh nothing
+      int j[U - 1];
+      float v[U - 1];
+      floatx4 f[U - 1];
+#pragma unroll
+      for (int u = 0; u < U - 1; ++u) {
+        const long x = e + u * st < e1 ? e + u * st : e;
+        j[u] = indices[x];
+        v[u] = values[x];
+      }
+#pragma unroll
+      for (int u = 0; u < U - 1; ++u) f[u] = *(const floatx4 *)(F + (long)j[u] * ldf + c);
+#pragma unroll
+      for (int u = 0; u < U - 1; ++u)
+        if (e + u * st < e1)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) acc[q] = fmaf(v[u], f[u][q], acc[q]);
+    }
+  };
+  if ((int)blockIdx.x >= nsegb) {
+    const long r = ((long)blockIdx.x - nsegb) * (256 / G) + threadIdx.x / G;
+    const long b = r < rows ? indptr[r] : 0, e = r < rows ? indptr[r + 1] : 0;
+    const bool is_long = e - b > SP_SHORT;
+    if (r < rows && !is_long) {
+      walk(b, e, 1);
+      spmm_store4(out, r, 4 * gl, k, ors, ocs, acc);
+    }
+    if constexpr (!PLAN) {
+      __shared__ int nlong, lrow[256 / G];
+      __shared__ floatx4 red[4][G];
+      if (threadIdx.x == 0) nlong = 0;
+      __syncthreads();
+      if (is_long && gl == 0) lrow[atomicAdd(&nlong, 1)] = (int)r;
+      __syncthreads();
+      const int wave = threadIdx.x >> 6;
+      for (int i = 0; i < nlong; ++i) {
+        const long lr = lrow[i];
+        acc = floatx4{0.f, 0.f, 0.f, 0.f};
+        walk(indptr[lr] + wave * NG + grp, indptr[lr + 1], 4 * NG);
+#pragma unroll
+        for (int off = G; off < 64; off <<= 1)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) acc[q] += __shfl_xor(acc[q], off, 64);
+        if (grp == 0) red[wave][gl] = acc;
+        __syncthreads();
+        if (threadIdx.x < G) spmm_store4(out, lr, 4 * gl, k, ors, ocs, (red[0][gl] + red[1][gl]) + (red[2][gl] + red[3][gl]));
+        __syncthreads();
+      }
+    }
+    return;
+  }
+  const int n = cnt[0];
+  for (int s = blockIdx.x * 4 + (threadIdx.x >> 6); s < n; s += nsegb * 4) {
+    const SpSeg sg = seg[s];
+    const long b = indptr[sg.row] + (long)sg.part * SP_SEG;
+    const long e = min(b + SP_SEG, indptr[sg.row + 1]);
+    acc = floatx4{0.f, 0.f, 0.f, 0.f};
+    walk(b + grp, e, NG);
+#pragma unroll
+    for (int off = G; off < 64; off <<= 1)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) acc[q] += __shfl_xor(acc[q], off, 64);
+    if (grp == 0) {
+      if (sg.nseg == 1) spmm_store4(out, sg.row, 4 * gl, k, ors, ocs, acc);
+      else *(floatx4 *)(partial + ((long)sg.pslot * G + gl) * 4) = acc;
     }
   }
-  if (active) out[r * ors + (long)lane * ocs] = acc;
+}
+
+// Rows of more than one piece: their partial sums in piece order.
+template <int G>
+__global__ __launch_bounds__(256) void spmm_finish_kernel(const int *cnt, const SpSeg *seg, const float *partial, int k,
+                                                          float *out, long ors, long ocs) {
+  const int gl = threadIdx.x % G;
+  const int n = cnt[0];
+  for (int s = (blockIdx.x * 256 + threadIdx.x) / G; s < n; s += gridDim.x * (256 / G)) {
+    const SpSeg sg = seg[s];
+    if (sg.part != 0 || sg.nseg == 1) continue;
+    const floatx4 *p = (const floatx4 *)partial + (long)sg.pslot * G + gl;
+    floatx4 t = {0.f, 0.f, 0.f, 0.f};
+    int i = 0;
+    for (; i + 8 <= sg.nseg; i += 8) {
+      floatx4 v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = p[(long)(i + u) * G];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) t += v[u];
+    }
+    for (; i < sg.nseg; ++i) t += p[(long)i * G];
+    spmm_store4(out, sg.row, 4 * gl, k, ors, ocs, t);
+  }
 }
 
 // Per block: sum over the non-zeros of its rows of (a - t)^2 and t^2 with
@@ -147,11 +292,10 @@ int csr_transpose(planc_ctx *ctx, long m, long n, long nnz, const long *indptr, 
   while (bits < 31 && (1L << bits) < n) ++bits;
   int *rowid = (int *)ws_get(ctx, kSparseSlot0 + 4, sizeof(int) * (size_t)nnz);
   unsigned *keys = (unsigned *)ws_get(ctx, kSparseSlot0 + 5, sizeof(unsigned) * 2 * (size_t)nnz);
-  int *ent = (int *)ws_get(ctx, kSparseSlot0 + 6, sizeof(int) * 2 * (size_t)nnz + sizeof(int) * (size_t)(n + 1));
+  int *ent = (int *)ws_get(ctx, kSparseSlot0 + 6, sizeof(int) * 2 * (size_t)nnz);
   if (!rowid || !keys || !ent) return set_error(ctx, PLANC_ENOMEM, "csr_transpose: workspace");
   unsigned *keys_s = keys + nnz;
   int *ent_s = ent + nnz;
-  int *cnt = ent + 2 * nnz;
   csr_entry_rows_kernel<<<(unsigned)((m + 3) / 4), 256, 0, ctx->stream>>>(m, indptr, rowid);
   PLANC_LAUNCH_CHECK(ctx);
   iota_kernel<<<(unsigned)((nnz + 255) / 256), 256, 0, ctx->stream>>>(nnz, ent);
@@ -161,34 +305,67 @@ int csr_transpose(planc_ctx *ctx, long m, long n, long nnz, const long *indptr, 
   size_t bytes = 0;
   PLANC_HIP_CHECK(ctx, hipcub::DeviceRadixSort::SortPairs(nullptr, bytes, keys, keys_s, ent, ent_s, (int)nnz, 0,
                                                           bits, ctx->stream));
-  size_t scan_bytes = 0;
-  PLANC_HIP_CHECK(ctx, hipcub::DeviceScan::ExclusiveScan(nullptr, scan_bytes, cnt, out_indptr, hipcub::Sum(),
-                                                         0L, (int)n, ctx->stream));
-  void *temp = ws_get(ctx, kSparseSlot0 + 7, std::max(bytes, scan_bytes));
+  void *temp = ws_get(ctx, kSparseSlot0 + 7, bytes);
   if (!temp) return set_error(ctx, PLANC_ENOMEM, "csr_transpose: sort workspace");
   PLANC_HIP_CHECK(ctx, hipcub::DeviceRadixSort::SortPairs(temp, bytes, keys, keys_s, ent, ent_s, (int)nnz, 0,
                                                           bits, ctx->stream));
-  csr_t_gather_kernel<<<(unsigned)((nnz + 255) / 256), 256, 0, ctx->stream>>>(nnz, ent_s, rowid, values,
-                                                                              out_indices, out_values);
-  PLANC_LAUNCH_CHECK(ctx);
-  PLANC_HIP_CHECK(ctx, hipMemsetAsync(cnt, 0, sizeof(int) * (size_t)n, ctx->stream));
-  col_count_kernel<<<(unsigned)((nnz + 255) / 256), 256, 0, ctx->stream>>>(nnz, indices, cnt);
-  PLANC_LAUNCH_CHECK(ctx);
-  PLANC_HIP_CHECK(ctx, hipcub::DeviceScan::ExclusiveScan(temp, scan_bytes, cnt, out_indptr, hipcub::Sum(), 0L,
-                                                         (int)n, ctx->stream));
-  set_long_kernel<<<1, 1, 0, ctx->stream>>>(out_indptr + n, nnz);
+  csr_t_gather_kernel<<<(unsigned)((nnz + 255) / 256), 256, 0, ctx->stream>>>(nnz, n, ent_s, keys_s, rowid, values,
+                                                                              out_indices, out_values, out_indptr);
   PLANC_LAUNCH_CHECK(ctx);
   return PLANC_OK;
 }
 
-int spmm_csr(planc_ctx *ctx, long rows, const long *indptr, const int *indices, const float *values,
-             const float *F, long ldf, int k, float *out, long ors, long ocs) {
-  if (k <= 0 || k > 64) return set_error(ctx, PLANC_EUNSUPPORTED, "spmm: k must be 1..64");
+// The pieces of a CSR's long rows, in workspace slot `slot` (two counts, then
+// room for all that nnz entries can make).
+int spmm_plan(planc_ctx *ctx, int slot, long rows, const long *indptr, long nnz, SpmmPlan *plan) {
+  const long cap = nnz / SP_SHORT + nnz / SP_SEG + 1;
+  char *w = (char *)ws_get(ctx, slot, 256 + sizeof(SpSeg) * (size_t)cap);
+  if (!w) return set_error(ctx, PLANC_ENOMEM, "spmm: workspace");
+  plan->cnt = (int *)w;
+  plan->seg = w + 256;
+  plan->segs = cap - 1;
+  plan->parts = 2 * (nnz / SP_SEG);
   if (rows <= 0) return PLANC_OK;
-  spmm_rows_kernel<<<(unsigned)((rows + 3) / 4), 256, 0, ctx->stream>>>(rows, indptr, indices, values, F, ldf,
-                                                                        k, out, ors, ocs);
+  spmm_plan_zero_kernel<<<1, 64, 0, ctx->stream>>>(plan->cnt);
+  PLANC_LAUNCH_CHECK(ctx);
+  spmm_plan_kernel<<<(unsigned)((rows + 255) / 256), 256, 0, ctx->stream>>>(rows, indptr, plan->cnt,
+                                                                           (SpSeg *)plan->seg);
   PLANC_LAUNCH_CHECK(ctx);
   return PLANC_OK;
+}
+
+template <int G>
+static int spmm_launch(planc_ctx *ctx, const SpmmPlan &pl, long rows, const long *indptr, const int *indices,
+                       const float *values, const float *F, long ldf, int k, float *out, long ors, long ocs) {
+  if (!pl.cnt) {
+    spmm_kernel<G, false><<<(unsigned)((rows + 256 / G - 1) / (256 / G)), 256, 0, ctx->stream>>>(
+        rows, indptr, indices, values, F, ldf, k, out, ors, ocs, 0, nullptr, nullptr, nullptr);
+    PLANC_LAUNCH_CHECK(ctx);
+    return PLANC_OK;
+  }
+  float *partial = (float *)ws_get(ctx, 21, sizeof(float) * 4 * G * (size_t)std::max(pl.parts, 1L));
+  if (!partial) return set_error(ctx, PLANC_ENOMEM, "spmm: workspace");
+  const int nsegb = (int)std::min<long>((pl.segs + 3) / 4, 8L * ctx->num_cu);
+  const long nb = nsegb + (rows + 256 / G - 1) / (256 / G);
+  const SpSeg *seg = (const SpSeg *)pl.seg;
+  spmm_kernel<G, true><<<(unsigned)nb, 256, 0, ctx->stream>>>(rows, indptr, indices, values, F, ldf, k, out, ors, ocs,
+                                                              nsegb, pl.cnt, seg, partial);
+  PLANC_LAUNCH_CHECK(ctx);
+  if (pl.parts > 0) {
+    const long fb = std::min<long>((pl.segs + 256 / G - 1) / (256 / G), 4L * ctx->num_cu);
+    spmm_finish_kernel<G><<<(unsigned)fb, 256, 0, ctx->stream>>>(pl.cnt, seg, partial, k, out, ors, ocs);
+    PLANC_LAUNCH_CHECK(ctx);
+  }
+  return PLANC_OK;
+}
+
+int spmm_csr(planc_ctx *ctx, const SpmmPlan &plan, long rows, const long *indptr, const int *indices,
+             const float *values, const float *F, long ldf, int k, float *out, long ors, long ocs) {
+  if (k <= 0 || k > 64) return set_error(ctx, PLANC_EUNSUPPORTED, "spmm: k must be 1..64");
+  if (rows <= 0) return PLANC_OK;
+  if (k <= 16) return spmm_launch<4>(ctx, plan, rows, indptr, indices, values, F, ldf, k, out, ors, ocs);
+  if (k <= 32) return spmm_launch<8>(ctx, plan, rows, indptr, indices, values, F, ldf, k, out, ors, ocs);
+  return spmm_launch<16>(ctx, plan, rows, indptr, indices, values, F, ldf, k, out, ors, ocs);
 }
 
 // k-major copies of W (m x k) and H (n x k) in workspace slots; returns them.
@@ -199,12 +376,23 @@ static int kmajor(planc_ctx *ctx, int slot, const float *X, long rows, long ldx,
   return transpose_to_k_major(ctx, X, rows, ldx, k, p, k);
 }
 
+// Row pitch of the products' k-major copies: rows of whole 16-byte words (what
+// lies past k is read into lanes that are not stored).
+static long pitch4(int k) { return (k + 3) / 4 * 4; }
+
+static int kmajor4(planc_ctx *ctx, int slot, const float *X, long rows, long ldx, int k, float **out) {
+  float *p = (float *)ws_get(ctx, slot, sizeof(float) * (size_t)rows * pitch4(k));
+  if (!p) return set_error(ctx, PLANC_ENOMEM, "sparse: factor copy");
+  *out = p;
+  return transpose_to_k_major(ctx, X, rows, ldx, k, p, pitch4(k));
+}
+
 int spmm_colmajor(planc_ctx *ctx, long rows, long cols, const long *indptr, const int *indices,
                   const float *values, const float *F, long ldf, int k, float *out, long ldo) {
   float *Fk = nullptr;
-  int rc = kmajor(ctx, kSparseSlot0 + 1, F, cols, ldf, k, &Fk);
+  int rc = kmajor4(ctx, kSparseSlot0 + 1, F, cols, ldf, k, &Fk);
   if (rc) return rc;
-  return spmm_csr(ctx, rows, indptr, indices, values, Fk, k, k, out, 1, ldo);
+  return spmm_csr(ctx, SpmmPlan{}, rows, indptr, indices, values, Fk, pitch4(k), k, out, 1, ldo);
 }
 
 int sparse_fit_error(planc_ctx *ctx, long m, long n, const long *indptr, const int *indices,
@@ -240,22 +428,23 @@ int sparse_products(planc_ctx *ctx, long m, long n, long nnz, const long *indptr
   ops->t_indptr = tptr;
   ops->t_indices = tidx;
   ops->t_values = tval;
-  return PLANC_OK;
+  if ((rc = spmm_plan(ctx, 19, m, indptr, nnz, &ops->plan))) return rc;
+  return spmm_plan(ctx, 20, n, tptr, nnz, &ops->t_plan);
 }
 
 int sparse_wta(planc_ctx *ctx, const SparseOps &o, long m, long n, const float *W, int k, float *out) {
   float *Wk = nullptr;
-  int rc = kmajor(ctx, kSparseSlot0 + 0, W, m, m, k, &Wk);
+  int rc = kmajor4(ctx, kSparseSlot0 + 0, W, m, m, k, &Wk);
   if (rc) return rc;
-  return spmm_csr(ctx, n, o.t_indptr, o.t_indices, o.t_values, Wk, k, k, out, k, 1);
+  return spmm_csr(ctx, o.t_plan, n, o.t_indptr, o.t_indices, o.t_values, Wk, pitch4(k), k, out, k, 1);
 }
 
 int sparse_ah(planc_ctx *ctx, const SparseOps &o, long m, long n, const long *indptr, const int *indices,
               const float *values, const float *H, int k, float *out) {
   float *Hk = nullptr;
-  int rc = kmajor(ctx, kSparseSlot0 + 1, H, n, n, k, &Hk);
+  int rc = kmajor4(ctx, kSparseSlot0 + 1, H, n, n, k, &Hk);
   if (rc) return rc;
-  return spmm_csr(ctx, m, indptr, indices, values, Hk, k, k, out, 1, m);
+  return spmm_csr(ctx, o.plan, m, indptr, indices, values, Hk, pitch4(k), k, out, 1, m);
 }
 
 }  // namespace planc
