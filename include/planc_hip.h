@@ -290,7 +290,7 @@ int planc_csr_col_subset(planc_ctx *ctx, long m, long n, const long *d_indptr, c
  * Node seeds: initseed * index (rank 0); W from stream 0, H from stream 1,
  * the power-iteration start from normals of stream 2 (Philox).  Nodes are
  * processed in batches (all nodes of a batch as one block-diagonal matrix,
- * one hipGraph-captured iteration loop).
+ * three launches per iteration).
  *   desc->nodes <= 0: the complete tree of `depth` levels, level by level;
  *     h_nodes in level order (capacity 2^depth - 1).
  *   desc->nodes > 0: the reference's best-first frontier with that node

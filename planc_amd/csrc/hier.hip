@@ -17,8 +17,21 @@
 // so DistR2 sets that row of W to 0 at the first W update and it stays 0;
 // it contributes to W^T W only at iteration 0, whose Gram is taken over all
 // m rows of the initial W (drawn from the node's Philox stream).
-// The iteration loop of a level is captured once into a hipGraph and
-// launched as one graph.
+// An iteration is three launches, each over blocks that belong to one node:
+//   h_gram_kernel: a column per thread, its H row, and the block's partial H^T H;
+//   w_rows_kernel: 256 compacted rows per block -- rows of up to SHORT_ROW
+//     entries a thread each, up to LONG_ROW a group of 16 lanes -- with the
+//     block's partial W^T W; further blocks take the segments of longer rows
+//     (the power-law row popularity of term-document matrices puts a few very
+//     long rows next to millions of short ones);
+//   w_long_kernel: the long rows from their segments, and their part of W^T W.
+// A block that needs its node's 2 x 2 Gram sums the node's partials itself.  The
+// power iteration has the same three steps.  All of it is bound by latency:
+// dependent gathers, and the launches of a loop whose kernels take
+// microseconds.  Complete tree of 9 levels, 50000 x 200000, 1.9 M entries, 100
+// iterations: eight launches an iteration, with 16 lanes on every row, took
+// 97 us (41 of them the row kernel) and the power iteration 51 us; these take
+// 46 (22) and 33 us.
 #include <algorithm>
 #include <cstring>
 #include <map>
@@ -170,57 +183,101 @@ struct Chunk {
   long b, e;
 };
 
-// Partial Grams of 2-column factors over chunks of contiguous rows.
-__global__ void gram2_chunks(const Chunk *ch, const double *X, double *part) {
-  __shared__ double red[3][4];
-  Chunk c = ch[blockIdx.x];
-  double s00 = 0, s01 = 0, s11 = 0;
-  for (long r = c.b + threadIdx.x; r < c.e; r += blockDim.x) {
-    double x0 = X[2 * r], x1 = X[2 * r + 1];
-    s00 += x0 * x0;
-    s01 += x0 * x1;
-    s11 += x1 * x1;
-  }
+// Sums over a block of 256 threads (valid in thread 0), fixed order.
+__device__ inline void block_sum3(double &s0, double &s1, double &s2, double (*red)[4]) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
-    s00 += __shfl_xor(s00, off, 64);
-    s01 += __shfl_xor(s01, off, 64);
-    s11 += __shfl_xor(s11, off, 64);
+    s0 += __shfl_xor(s0, off, 64);
+    s1 += __shfl_xor(s1, off, 64);
+    s2 += __shfl_xor(s2, off, 64);
   }
-  int w = threadIdx.x >> 6;
+  const int w = threadIdx.x >> 6;
   if ((threadIdx.x & 63) == 0) {
-    red[0][w] = s00;
-    red[1][w] = s01;
-    red[2][w] = s11;
+    red[0][w] = s0;
+    red[1][w] = s1;
+    red[2][w] = s2;
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    double t0 = 0, t1 = 0, t2 = 0;
-    for (int q = 0; q < (int)(blockDim.x >> 6); ++q) {
-      t0 += red[0][q];
-      t1 += red[1][q];
-      t2 += red[2][q];
-    }
-    part[3 * blockIdx.x] = t0;
-    part[3 * blockIdx.x + 1] = t1;
-    part[3 * blockIdx.x + 2] = t2;
+    s0 = red[0][0] + red[0][1] + red[0][2] + red[0][3];
+    s1 = red[1][0] + red[1][1] + red[1][2] + red[1][3];
+    s2 = red[2][0] + red[2][1] + red[2][2] + red[2][3];
   }
 }
 
-// Node Gram (column-major 2x2) from its chunks [cb[t], cb[t+1]).
-__global__ void gram2_finalize(const double *part, const int *cb, int nn, double *G) {
-  int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nn) return;
-  double a = 0, b = 0, c = 0;
-  for (int q = cb[t]; q < cb[t + 1]; ++q) {
-    a += part[3 * q];
-    b += part[3 * q + 1];
-    c += part[3 * q + 2];
+// Partials of a node's 2 x 2 Gram (x0^2, x0 x1, x1^2): chunks [cb[t], cb[t+1])
+// of `part` and, with `extra`, entry t of it (the long rows' share).
+struct GramParts {
+  const double *part;
+  const int *cb;
+  const double *extra;
+};
+
+// Sum of entries b, b + st, ... < e in order, eight loads in flight.
+__device__ inline double ordered_sum(const double *part, long b, long e, long st) {
+  double s = 0;
+  for (; b + 7 * st < e; b += 8 * st) {
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = part[b + u * st];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) s += v[u];
   }
-  G[4 * t] = a;
-  G[4 * t + 1] = b;
-  G[4 * t + 2] = b;
-  G[4 * t + 3] = c;
+  for (; b < e; b += st) s += part[b];
+  return s;
+}
+
+// A node of up to FEW_CHUNKS chunks sums them in chunk order, a larger one by
+// the lanes of a wavefront.
+constexpr int FEW_CHUNKS = 16;
+
+// The Gram of node t (column-major) into G, by the first wavefront; ends with a
+// barrier.
+__device__ inline void node_gram(const GramParts &p, int t, double *G) {
+  if (threadIdx.x < 64) {
+    const long b = p.cb[t], e = p.cb[t + 1];
+    double s[3] = {0, 0, 0};
+    if (e - b <= FEW_CHUNKS) {
+      const int i = threadIdx.x < 3 ? threadIdx.x : 0;
+      const double v = ordered_sum(p.part, 3 * b + i, 3 * e, 3);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) s[q] = __shfl(v, q, 64);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 3; ++q) s[q] = ordered_sum(p.part, 3 * (b + threadIdx.x) + q, 3 * e, 3 * 64);
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+        for (int q = 0; q < 3; ++q) s[q] += __shfl_xor(s[q], off, 64);
+    }
+    if (threadIdx.x == 0) {
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+        if (p.extra) s[q] += p.extra[3 * t + q];
+      G[0] = s[0];
+      G[1] = s[1];
+      G[2] = s[1];
+      G[3] = s[2];
+    }
+  }
+  __syncthreads();
+}
+
+// sqrt of the sum of node t's chunk partials into *out, likewise.
+__device__ inline void node_norm(const double *part, const int *cb, int t, double *out) {
+  if (threadIdx.x < 64) {
+    const long b = cb[t], e = cb[t + 1];
+    double s;
+    if (e - b <= FEW_CHUNKS) {
+      s = ordered_sum(part, b, e, 1);
+    } else {
+      s = ordered_sum(part, b + threadIdx.x, e, 64);
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    }
+    if (threadIdx.x == 0) *out = sqrt(s);
+  }
+  __syncthreads();
 }
 
 // Gram over all m rows of the initial W of every node (iteration 0).
@@ -284,8 +341,6 @@ __global__ void init_factors(long nrows, const int *row_node, const int *row_ori
   }
 }
 
-// H update: WtA(:, lc) over the column's entries, then the R2 rule with the
-// node's W^T W.
 // Sums over the entries b, b+S, b+2S, ... < e1 of val * X[idx], taken in
 // that order; four entries' index/value loads are issued before their
 // gathers so each step waits on one memory round trip, not four.
@@ -330,50 +385,37 @@ __device__ inline double dot1_range(long b, long e1, long S, const int *__restri
   return s;
 }
 
-__global__ void h_update(long nlev, const long *col_ptr, const int *csc_row, const float *csc_val,
-                         const int *node_of_col, const double *W, const double *Gw, double *H) {
-  long lc = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (lc >= nlev) return;
+// Column chunks (at most 256 columns of one node per block): WtA(:, lc) over the
+// column's entries, the R2 rule with the node's W^T W, and the chunk's part of
+// H^T H.
+__global__ __launch_bounds__(256) void h_gram_kernel(const Chunk *ch, const long *col_ptr, const int *csc_row,
+                                                     const float *csc_val, const double *W, GramParts gw, double *H,
+                                                     double *part) {
+  __shared__ double G[4], red[3][4];
+  const Chunk c = ch[blockIdx.x];
+  const long lc = c.b + threadIdx.x;
   double s0 = 0, s1 = 0;
-  dot2_range(col_ptr[lc], col_ptr[lc + 1], 1, csc_row, csc_val, (const double2 *)W, s0, s1);
-  double x0, x1;
-  r2_solve(Gw + 4 * node_of_col[lc], s0, s1, x0, x1);
-  H[2 * lc] = x0;
-  H[2 * lc + 1] = x1;
+  if (lc < c.e) dot2_range(col_ptr[lc], col_ptr[lc + 1], 1, csc_row, csc_val, (const double2 *)W, s0, s1);
+  node_gram(gw, c.node, G);
+  double x0 = 0, x1 = 0;
+  if (lc < c.e) {
+    r2_solve(G, s0, s1, x0, x1);
+    ((double2 *)H)[lc] = double2{x0, x1};
+  }
+  double g0 = x0 * x0, g1 = x0 * x1, g2 = x1 * x1;
+  block_sum3(g0, g1, g2, red);
+  if (threadIdx.x == 0) {
+    part[3 * blockIdx.x] = g0;
+    part[3 * blockIdx.x + 1] = g1;
+    part[3 * blockIdx.x + 2] = g2;
+  }
 }
 
-// W update: (A H)(r, :) over the compacted row's entries, then the R2 rule
-// with the node's H^T H.  G lanes per row (a sub-wave group or a whole
-// wave, G in {4, 16, 64}, picked per level by timing); rows longer than `longlen` are
-// left to the segmented long-row kernels -- the power-law row
-// popularity of term-document matrices puts a few very long rows next to
-// millions of short ones.
 template <int G>
 __device__ inline double group_sum(double v) {
 #pragma unroll
   for (int off = G / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, G);
   return v;
-}
-
-template <int G>
-__global__ void w_update_short(long nrows, const long *row_ptr, const int *csr_col,
-                               const float *csr_val, const int *row_node, const double *H,
-                               const double *Gh, double *W, long longlen) {
-  long g = ((long)blockIdx.x * blockDim.x + threadIdx.x) / G;
-  int lane = threadIdx.x % G;
-  if (g >= nrows) return;
-  long b = row_ptr[g], e1 = row_ptr[g + 1];
-  if (e1 - b > longlen) return;
-  double s0 = 0, s1 = 0;
-  dot2_range(b + lane, e1, G, csr_col, csr_val, (const double2 *)H, s0, s1);
-  s0 = group_sum<G>(s0);
-  s1 = group_sum<G>(s1);
-  if (lane == 0) {
-    double x0, x1;
-    r2_solve(Gh + 4 * row_node[g], s0, s1, x0, x1);
-    W[2 * g] = x0;
-    W[2 * g + 1] = x1;
-  }
 }
 
 __device__ inline double block_sum256(double v, double *red) {
@@ -385,40 +427,183 @@ __device__ inline double block_sum256(double v, double *red) {
   return red[0] + red[1] + red[2] + red[3];
 }
 
-// Long rows are cut into segments of at most SEG_LEN entries (a block
-// each, partial sums to seg_part); the per-row finish adds a row's segment
-// partials in segment order, so the sums are taken in a fixed order.
+// Row classes.  A thread walks a short row (two steps of four gathers), 16
+// lanes a medium one (two steps of four gathers each); longer rows are cut into
+// segments of at most SEG_LEN entries (a block each, partial sums to
+// seg_part), and a row's segment partials are added in segment order.
+constexpr long SHORT_ROW = 8;
+constexpr long LONG_ROW = 128;
 constexpr long SEG_LEN = 4096;
 
-__global__ void w_update_seg(const int *seg_row, const long *seg_b, const int *list, const long *row_ptr,
-                             const int *csr_col, const float *csr_val, const double *H, double *seg_part) {
-  __shared__ double red[4];
-  long r = list[seg_row[blockIdx.x]];
-  long b = seg_b[blockIdx.x];
-  long e1 = min(b + SEG_LEN, row_ptr[r + 1]);
-  double s0 = 0, s1 = 0;
-  dot2_range(b + threadIdx.x, e1, blockDim.x, csr_col, csr_val, (const double2 *)H, s0, s1);
-  s0 = block_sum256(s0, red);
-  s1 = block_sum256(s1, red);
+struct LevelRows {
+  const long *row_ptr;
+  const int *col;
+  const float *val;
+  const Chunk *ch;  // at most 256 rows of one node
+  // long rows: segments and list
+  const int *seg_row;
+  const long *seg_b;
+  const int *list;
+  const long *seg_off;
+  const int *node_long0;  // long rows of node t: [node_long0[t], node_long0[t + 1])
+  int nseg;
+};
+
+// The sums of a short row by one thread, all its gathers in flight: the products
+// rounded and added as 16 lanes with one entry each would add them (group_sum),
+// so that a row's sum does not depend on which of the two took it and sums that
+// cancel in a degenerate node (a singular Gram) keep doing so exactly.
+template <class Load>
+__device__ inline double few_sum(long b, long e, const int *__restrict__ idx, const float *__restrict__ val, Load load,
+                                 double *second) {
+#pragma clang fp contract(off)
+  double p[SHORT_ROW], p2[SHORT_ROW];
+#pragma unroll
+  for (int u = 0; u < SHORT_ROW; ++u) {
+    p[u] = 0.0;
+    p2[u] = 0.0;
+    if (b + u < e) {
+      const double v = val[b + u];
+      double x1 = 0.0;
+      const double x0 = load(idx[b + u], x1);
+      p[u] = v * x0;
+      p2[u] = v * x1;
+    }
+  }
+  static_assert(SHORT_ROW == 8, "the tree below");
+  *second = ((p2[0] + p2[4]) + (p2[2] + p2[6])) + ((p2[1] + p2[5]) + (p2[3] + p2[7]));
+  return ((p[0] + p[4]) + (p[2] + p[6])) + ((p[1] + p[5]) + (p[3] + p[7]));
+}
+
+// Sums over one row of a row chunk for every thread's row: few(b, e) sums a
+// short one, one(b, e, S) entries b, b + S, ... < e, group_add the lanes of a
+// group.  sv: 256 values in LDS, list / cnt the medium rows.
+template <class V, class Few, class One, class Add>
+__device__ inline V chunk_row_sum(const LevelRows &L, const Chunk &c, Few few, One one, Add group_add, V *sv, int *list,
+                                  int *cnt, bool &is_long) {
+  const int tid = threadIdx.x;
+  const long r = c.b + tid;
+  long b = 0, e = 0;
+  if (r < c.e) {
+    b = L.row_ptr[r];
+    e = L.row_ptr[r + 1];
+  }
+  if (tid == 0) *cnt = 0;
+  __syncthreads();
+  is_long = e - b > LONG_ROW;
+  const bool medium = e - b > SHORT_ROW && !is_long;
+  if (medium) list[atomicAdd(cnt, 1)] = tid;
+  V v = V();
+  if (!medium && !is_long) v = few(b, e);
+  __syncthreads();
+  for (int i = tid / 16; i < *cnt; i += 16) {
+    const int t = list[i];
+    const long mb = L.row_ptr[c.b + t], me = L.row_ptr[c.b + t + 1];
+    V m = group_add(one(mb + tid % 16, me, 16L));
+    if (tid % 16 == 0) sv[t] = m;
+  }
+  __syncthreads();
+  return medium ? sv[tid] : v;
+}
+
+struct Pair {
+  double a, b;
+};
+
+// W update: (A H)(r, :) over the compacted row's entries, then the R2 rule with
+// the node's H^T H, and the chunk's part of W^T W (long rows: w_long_kernel).
+__global__ __launch_bounds__(256) void w_rows_kernel(LevelRows L, const double *H, GramParts gh, double *W,
+                                                     double *part, double *seg_part) {
+  __shared__ double G[4], red[3][4];
+  __shared__ Pair sv[256];
+  __shared__ int list[256], cnt;
+  const int *col = L.col;
+  const float *val = L.val;
+  auto one = [&](long b, long e, long S) {
+    Pair p{0.0, 0.0};
+    dot2_range(b, e, S, col, val, (const double2 *)H, p.a, p.b);
+    return p;
+  };
+  if ((int)blockIdx.x < L.nseg) {
+    const long r = L.list[L.seg_row[blockIdx.x]];
+    const long b = L.seg_b[blockIdx.x];
+    Pair p = one(b + threadIdx.x, min(b + SEG_LEN, L.row_ptr[r + 1]), 256L);
+    p.a = block_sum256(p.a, red[0]);
+    p.b = block_sum256(p.b, red[1]);
+    if (threadIdx.x == 0) {
+      seg_part[2 * blockIdx.x] = p.a;
+      seg_part[2 * blockIdx.x + 1] = p.b;
+    }
+    return;
+  }
+  const int ci = (int)blockIdx.x - L.nseg;
+  const Chunk c = L.ch[ci];
+  bool is_long;
+  auto few = [&](long b, long e) {
+    Pair p;
+    p.a = few_sum(
+        b, e, col, val,
+        [&](int i, double &x1) {
+          const double2 x = ((const double2 *)H)[i];
+          x1 = x.y;
+          return x.x;
+        },
+        &p.b);
+    return p;
+  };
+  const Pair p = chunk_row_sum<Pair>(
+      L, c, few, one,
+      [](Pair q) {
+        q.a = group_sum<16>(q.a);
+        q.b = group_sum<16>(q.b);
+        return q;
+      },
+      sv, list, &cnt, is_long);
+  node_gram(gh, c.node, G);
+  const long r = c.b + threadIdx.x;
+  double x0 = 0, x1 = 0;
+  if (r < c.e && !is_long) {
+    r2_solve(G, p.a, p.b, x0, x1);
+    ((double2 *)W)[r] = double2{x0, x1};
+  }
+  double g0 = x0 * x0, g1 = x0 * x1, g2 = x1 * x1;
+  block_sum3(g0, g1, g2, red);
   if (threadIdx.x == 0) {
-    seg_part[2 * blockIdx.x] = s0;
-    seg_part[2 * blockIdx.x + 1] = s1;
+    part[3 * ci] = g0;
+    part[3 * ci + 1] = g1;
+    part[3 * ci + 2] = g2;
   }
 }
-__global__ void w_update_long_fin(long nlong, const int *list, const long *seg_off, const double *seg_part,
-                                  const int *row_node, const double *Gh, double *W) {
-  long j = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= nlong) return;
-  long r = list[j];
-  double s0 = 0, s1 = 0;
-  for (long q = seg_off[j]; q < seg_off[j + 1]; ++q) {
-    s0 += seg_part[2 * q];
-    s1 += seg_part[2 * q + 1];
+
+// A block per node: its long rows, and their part of W^T W.
+__global__ __launch_bounds__(256) void w_long_kernel(LevelRows L, const double *seg_part, GramParts gh, double *W,
+                                                     double *extra) {
+  __shared__ double G[4], red[3][4];
+  const int t = blockIdx.x;
+  const int j0 = L.node_long0[t], j1 = L.node_long0[t + 1];
+  double g0 = 0, g1 = 0, g2 = 0;
+  if (j0 < j1) {  // uniform over the block
+    node_gram(gh, t, G);
+    for (int j = j0 + (int)threadIdx.x; j < j1; j += 256) {
+      double s0 = 0, s1 = 0;
+      for (long q = L.seg_off[j]; q < L.seg_off[j + 1]; ++q) {
+        s0 += seg_part[2 * q];
+        s1 += seg_part[2 * q + 1];
+      }
+      double x0, x1;
+      r2_solve(G, s0, s1, x0, x1);
+      ((double2 *)W)[L.list[j]] = double2{x0, x1};
+      g0 += x0 * x0;
+      g1 += x0 * x1;
+      g2 += x1 * x1;
+    }
+    block_sum3(g0, g1, g2, red);
   }
-  double x0, x1;
-  r2_solve(Gh + 4 * row_node[r], s0, s1, x0, x1);
-  W[2 * r] = x0;
-  W[2 * r + 1] = x1;
+  if (threadIdx.x == 0) {
+    extra[3 * t] = g0;
+    extra[3 * t + 1] = g1;
+    extra[3 * t + 2] = g2;
+  }
 }
 
 __global__ void flag_long(const long *row_ptr, long nrows, long longlen, int *flag) {
@@ -460,45 +645,63 @@ __global__ void pow_init(long nlev, const int *node_of_col, const long *node_col
   q[lc] = planc_rng::normal(seeds[t], 2, (uint64_t)(lc - node_col0[t]));
 }
 
-template <int G>
-__global__ void pow_rows_short(long nrows, const long *row_ptr, const int *csr_col,
-                               const float *csr_val, const int *row_node, const double *q,
-                               const double *sig, double *z, long longlen) {
-  long g = ((long)blockIdx.x * blockDim.x + threadIdx.x) / G;
-  int lane = threadIdx.x % G;
-  if (g >= nrows) return;
-  long b = row_ptr[g], e1 = row_ptr[g + 1];
-  if (e1 - b > longlen) return;
-  double s = dot1_range(b + lane, e1, G, csr_col, csr_val, q);
-  s = group_sum<G>(s);
-  if (lane == 0) z[g] = s / sig[row_node[g]];
+// z = A q / s by row chunks and segments; the node's s from the partials of
+// ||q||^2.
+__global__ __launch_bounds__(256) void pow_rows_kernel(LevelRows L, const double *q, const double *part,
+                                                       const int *cb, double *z, double *seg_part) {
+  __shared__ double red[4], sig;
+  __shared__ double sv[256];
+  __shared__ int list[256], cnt;
+  const int *col = L.col;
+  const float *val = L.val;
+  auto one = [&](long b, long e, long S) { return dot1_range(b, e, S, col, val, q); };
+  if ((int)blockIdx.x < L.nseg) {
+    const long r = L.list[L.seg_row[blockIdx.x]];
+    const long b = L.seg_b[blockIdx.x];
+    const double s = block_sum256(one(b + threadIdx.x, min(b + SEG_LEN, L.row_ptr[r + 1]), 256L), red);
+    if (threadIdx.x == 0) seg_part[blockIdx.x] = s;
+    return;
+  }
+  const Chunk c = L.ch[(int)blockIdx.x - L.nseg];
+  bool is_long;
+  auto few = [&](long b, long e) {
+    double unused;
+    return few_sum(b, e, col, val, [&](int i, double &) { return q[i]; }, &unused);
+  };
+  const double s = chunk_row_sum<double>(L, c, few, one, [](double v) { return group_sum<16>(v); }, sv, list, &cnt, is_long);
+  node_norm(part, cb, c.node, &sig);
+  const long r = c.b + threadIdx.x;
+  if (r < c.e && !is_long) z[r] = s / sig;
 }
 
-__global__ void pow_rows_seg(const int *seg_row, const long *seg_b, const int *list, const long *row_ptr,
-                             const int *csr_col, const float *csr_val, const double *q, double *seg_part) {
+__global__ __launch_bounds__(256) void pow_long_kernel(LevelRows L, const double *seg_part, const double *part,
+                                                       const int *cb, double *z) {
+  __shared__ double sig;
+  const int t = blockIdx.x;
+  const int j0 = L.node_long0[t], j1 = L.node_long0[t + 1];
+  if (j0 >= j1) return;
+  node_norm(part, cb, t, &sig);
+  for (int j = j0 + (int)threadIdx.x; j < j1; j += 256) {
+    double s = 0;
+    for (long q = L.seg_off[j]; q < L.seg_off[j + 1]; ++q) s += seg_part[q];
+    z[L.list[j]] = s / sig;
+  }
+}
+
+// q = A^T z and the column chunks' partials of ||q||^2.
+__global__ __launch_bounds__(256) void pow_cols_kernel(const Chunk *ch, const long *col_ptr, const int *csc_row,
+                                                       const float *csc_val, const double *z, double *q,
+                                                       double *part) {
   __shared__ double red[4];
-  long r = list[seg_row[blockIdx.x]];
-  long b = seg_b[blockIdx.x];
-  long e1 = min(b + SEG_LEN, row_ptr[r + 1]);
-  double s = dot1_range(b + threadIdx.x, e1, blockDim.x, csr_col, csr_val, q);
-  s = block_sum256(s, red);
-  if (threadIdx.x == 0) seg_part[blockIdx.x] = s;
-}
-__global__ void pow_rows_long_fin(long nlong, const int *list, const long *seg_off, const double *seg_part,
-                                  const int *row_node, const double *sig, double *z) {
-  long j = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= nlong) return;
-  long r = list[j];
-  double s = 0;
-  for (long q = seg_off[j]; q < seg_off[j + 1]; ++q) s += seg_part[q];
-  z[r] = s / sig[row_node[r]];
-}
-
-__global__ void pow_cols(long nlev, const long *col_ptr, const int *csc_row, const float *csc_val,
-                         const double *z, double *q) {
-  long lc = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (lc >= nlev) return;
-  q[lc] = dot1_range(col_ptr[lc], col_ptr[lc + 1], 1, csc_row, csc_val, z);
+  const Chunk c = ch[blockIdx.x];
+  const long lc = c.b + threadIdx.x;
+  double v = 0;
+  if (lc < c.e) {
+    v = dot1_range(col_ptr[lc], col_ptr[lc + 1], 1, csc_row, csc_val, z);
+    q[lc] = v;
+  }
+  const double s = block_sum256(v * v, red);
+  if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
 __global__ void sumsq_chunks(const Chunk *ch, const double *x, double *part) {
@@ -517,12 +720,8 @@ __global__ void sumsq_chunks(const Chunk *ch, const double *x, double *part) {
   }
 }
 
-__global__ void norm_finalize(const double *part, const int *cb, int nn, double *sig) {
-  int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nn) return;
-  double s = 0;
-  for (int q = cb[t]; q < cb[t + 1]; ++q) s += part[q];
-  sig[t] = sqrt(s);
+__global__ void norm_finalize(const double *part, const int *cb, double *sig) {
+  node_norm(part, cb, blockIdx.x, sig + blockIdx.x);
 }
 
 __global__ void fill_ones(double *x, int n) {
@@ -602,15 +801,14 @@ struct Engine {
   // level
   DBuf<long> perm, col_ptr, row_ptr, rstart, bsum, node_col0;
   DBuf<int> colmap, node_of_col, flag, row_node, row_orig, row_len, col_len, csr_col, csc_row,
-      cb_rows, cb_cols, cb_init, lflag, llist, row0, csc2csr, ent, ent_s, rid_of_entry, lcnt, seg_row;
+      cb_rows, cb_cols, cb_init, lflag, llist, node_long0, row0, csc2csr, ent, ent_s, rid_of_entry, lcnt, seg_row;
   DBuf<long> seg_off, seg_b;
   DBuf<double> seg_part;
   DBuf<unsigned> key, key_s;
   DBuf<unsigned char> temp;
   DBuf<long> lpos;
-  DBuf<double> Wscratch;
   DBuf<float> csr_val, csc_val;
-  DBuf<double> W, H, Gw, Gh, part, q, z, sig;
+  DBuf<double> W, H, part, part_h, extra, q, z, sig;
   DBuf<unsigned long long> seeds;
   DBuf<Chunk> ch_rows, ch_cols, ch_init;
   DBuf<unsigned char> mask;
@@ -624,65 +822,11 @@ struct Engine {
     cb_cols.release(); cb_init.release(); lflag.release(); llist.release(); row0.release();
     csc2csr.release(); ent.release(); ent_s.release(); rid_of_entry.release(); key.release();
     key_s.release(); temp.release(); csr_val.release(); csc_val.release(); W.release();
-    H.release(); Gw.release(); Gh.release(); part.release(); q.release(); z.release();
+    H.release(); part.release(); q.release(); z.release();
     sig.release(); seeds.release(); ch_rows.release(); ch_cols.release(); ch_init.release();
-    mask.release(); lpos.release(); Wscratch.release(); lcnt.release(); seg_row.release();
-    seg_off.release(); seg_b.release(); seg_part.release();
-  }
-
-  // Launches of the row kernels with G lanes per row.
-  void launch_w_short(int G, long nrows, double *Wout, long longlen) {
-    long thr = nrows * G;
-    unsigned nbk = (unsigned)((thr + 255) / 256);
-    if (nbk == 0) return;
-    if (G == 64)
-      w_update_short<64><<<nbk, 256, 0, ctx->stream>>>(nrows, row_ptr.p, csr_col.p, csr_val.p, row_node.p, H.p, Gh.p, Wout, longlen);
-    else if (G == 4)
-      w_update_short<4><<<nbk, 256, 0, ctx->stream>>>(nrows, row_ptr.p, csr_col.p, csr_val.p, row_node.p, H.p, Gh.p, Wout, longlen);
-    else
-      w_update_short<16><<<nbk, 256, 0, ctx->stream>>>(nrows, row_ptr.p, csr_col.p, csr_val.p, row_node.p, H.p, Gh.p, Wout, longlen);
-  }
-  void launch_pow_short(int G, long nrows, long longlen) {
-    long thr = nrows * G;
-    unsigned nbk = (unsigned)((thr + 255) / 256);
-    if (nbk == 0) return;
-    if (G == 64)
-      pow_rows_short<64><<<nbk, 256, 0, ctx->stream>>>(nrows, row_ptr.p, csr_col.p, csr_val.p, row_node.p, q.p, sig.p, z.p, longlen);
-    else if (G == 4)
-      pow_rows_short<4><<<nbk, 256, 0, ctx->stream>>>(nrows, row_ptr.p, csr_col.p, csr_val.p, row_node.p, q.p, sig.p, z.p, longlen);
-    else
-      pow_rows_short<16><<<nbk, 256, 0, ctx->stream>>>(nrows, row_ptr.p, csr_col.p, csr_val.p, row_node.p, q.p, sig.p, z.p, longlen);
-  }
-  // Lanes per row for this level: the fastest of {4, 16, 64} over a few
-  // timed launches of the W update into a scratch buffer.
-  int tune_group(long nrows, long longlen) {
-    if (nrows == 0) return 16;
-    if (Wscratch.get(ctx, 2 * nrows)) return 16;
-    const int cand[3] = {4, 16, 64};
-    float best = 1e30f;
-    int bestg = 16;
-    hipEvent_t e0, e1;
-    if (hipEventCreate(&e0) != hipSuccess) return 16;
-    if (hipEventCreate(&e1) != hipSuccess) {
-      (void)hipEventDestroy(e0);
-      return 16;
-    }
-    for (int c : cand) {
-      launch_w_short(c, nrows, Wscratch.p, longlen);
-      (void)hipEventRecord(e0, ctx->stream);
-      for (int rep = 0; rep < 3; ++rep) launch_w_short(c, nrows, Wscratch.p, longlen);
-      (void)hipEventRecord(e1, ctx->stream);
-      (void)hipEventSynchronize(e1);
-      float ms = 0;
-      (void)hipEventElapsedTime(&ms, e0, e1);
-      if (ms < best) {
-        best = ms;
-        bestg = c;
-      }
-    }
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    return bestg;
+    mask.release(); lpos.release(); lcnt.release(); seg_row.release();
+    seg_off.release(); seg_b.release(); seg_part.release(); node_long0.release(); part_h.release();
+    extra.release();
   }
 
   // out[i] = sum_{j < i} in[j] (64-bit sums); returns the total (synchronises).
@@ -719,13 +863,31 @@ struct Engine {
 };
 
 // Chunks of at most `chunk` consecutive items per node (node t owns
-// [off[t], off[t+1])); cb[t] is the first chunk of node t.
-void make_chunks(const std::vector<long> &off, long chunk, std::vector<Chunk> &ch, std::vector<int> &cb) {
+// [off[t], off[t+1])); cb[t] is the first chunk of node t.  With row pointers, a
+// chunk ends before its rows (those over LONG_ROW aside) pass CHUNK_ENTRIES
+// entries: the first rows of a node are its longest, and a block of 256 medium
+// rows alone took as long as the rest of the launch (51 us against 12).
+constexpr long CHUNK_ENTRIES = 1024;
+void make_chunks(const std::vector<long> &off, long chunk, std::vector<Chunk> &ch, std::vector<int> &cb,
+                 const std::vector<long> *ptr = nullptr) {
   ch.clear();
   cb.assign(off.size(), 0);
   for (size_t t = 0; t + 1 < off.size(); ++t) {
     cb[t] = (int)ch.size();
-    for (long b = off[t]; b < off[t + 1]; b += chunk) ch.push_back({(int)t, b, std::min(off[t + 1], b + chunk)});
+    for (long b = off[t]; b < off[t + 1];) {
+      long e = std::min(off[t + 1], b + chunk);
+      if (ptr) {
+        long used = 0, r = b;
+        for (; r < e; ++r) {
+          const long len = (*ptr)[r + 1] - (*ptr)[r];
+          if (len <= LONG_ROW) used += len;
+          if (used > CHUNK_ENTRIES && r > b) break;
+        }
+        e = r;
+      }
+      ch.push_back({(int)t, b, e});
+      b = e;
+    }
   }
   cb[off.size() - 1] = (int)ch.size();
 }
@@ -907,14 +1069,13 @@ int planc_hiernmf_run(planc_ctx *ctx, const planc_hier_desc *desc, const long *h
                                                      E.rid_of_entry.p, E.col_ptr.p, E.csc_row.p,
                                                      E.csc_val.p);
     PLANC_LAUNCH_CHECK(ctx);
-    // Rows longer than LONGLEN are cut into SEG_LEN segments, a block each
+    // Rows longer than LONG_ROW are cut into SEG_LEN segments, a block each
     // (lists built on the device).
-    const long LONGLEN = 2048;
     RC(E.lflag.get(ctx, nrows ? nrows : 1));
     RC(E.lpos.get(ctx, nrows ? nrows : 1));
     long nlong = 0;
     if (nrows) {
-      flag_long<<<nb(nrows), 256, 0, ctx->stream>>>(E.row_ptr.p, nrows, LONGLEN, E.lflag.p);
+      flag_long<<<nb(nrows), 256, 0, ctx->stream>>>(E.row_ptr.p, nrows, LONG_ROW, E.lflag.p);
       RC(E.scan(E.lflag.p, nrows, E.lpos.p, &nlong));
     }
     RC(E.llist.get(ctx, nlong ? nlong : 1));
@@ -937,17 +1098,30 @@ int planc_hiernmf_run(planc_ctx *ctx, const planc_hier_desc *desc, const long *h
     PLANC_LAUNCH_CHECK(ctx);
     // Node row ranges (rows of node t are contiguous: t-major flag scan).
     std::vector<int> rnode(nrows);
-    if (nrows)
+    std::vector<long> hptr(nrows + 1, 0);
+    if (nrows) {
       PLANC_HIP_CHECK(ctx, hipMemcpyAsync(rnode.data(), E.row_node.p, sizeof(int) * nrows,
                                           hipMemcpyDeviceToHost, ctx->stream));
+      PLANC_HIP_CHECK(ctx, hipMemcpyAsync(hptr.data(), E.row_ptr.p, sizeof(long) * (nrows + 1),
+                                          hipMemcpyDeviceToHost, ctx->stream));
+    }
+    std::vector<int> hlong(nlong);
+    if (nlong)
+      PLANC_HIP_CHECK(ctx, hipMemcpyAsync(hlong.data(), E.llist.p, sizeof(int) * nlong, hipMemcpyDeviceToHost,
+                                          ctx->stream));
     PLANC_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
+    std::vector<int> nlong0(nn + 1, 0);  // long rows ascend, so a node's are contiguous
+    for (int r : hlong) nlong0[rnode[r] + 1]++;
+    for (int t = 0; t < nn; ++t) nlong0[t + 1] += nlong0[t];
+    RC(E.node_long0.get(ctx, nn + 1));
+    PLANC_HIP_CHECK(ctx, up(E.node_long0.p, nlong0.data(), sizeof(int) * (nn + 1)));
     std::vector<long> roff(nn + 1, 0);
     for (long r = 0; r < nrows; ++r) roff[rnode[r] + 1]++;
     for (int t = 0; t < nn; ++t) roff[t + 1] += roff[t];
     std::vector<Chunk> chr, chc, chi;
     std::vector<int> cbr, cbc, cbi;
-    make_chunks(roff, 4096, chr, cbr);
-    make_chunks(noff, 4096, chc, cbc);
+    make_chunks(roff, 256, chr, cbr, &hptr);
+    make_chunks(noff, 256, chc, cbc);
     std::vector<long> ioff(nn + 1);
     for (int t = 0; t <= nn; ++t) ioff[t] = (long)t * m;
     make_chunks(ioff, 16384, chi, cbi);
@@ -969,45 +1143,35 @@ int planc_hiernmf_run(planc_ctx *ctx, const planc_hier_desc *desc, const long *h
     PLANC_HIP_CHECK(ctx, up(E.cb_rows.p, cbr.data(), sizeof(int) * (nn + 1)));
     PLANC_HIP_CHECK(ctx, up(E.cb_cols.p, cbc.data(), sizeof(int) * (nn + 1)));
     PLANC_HIP_CHECK(ctx, up(E.cb_init.p, cbi.data(), sizeof(int) * (nn + 1)));
-    size_t np = std::max(std::max(chr.size(), chc.size()), chi.size());
-    RC(E.part.get(ctx, 3 * np + 3));
+    RC(E.part.get(ctx, 3 * std::max(chr.size(), chi.size()) + 3));
+    RC(E.part_h.get(ctx, 3 * chc.size() + 3));
+    RC(E.extra.get(ctx, 3 * nn));
     RC(E.W.get(ctx, 2 * (nrows ? nrows : 1)));
     RC(E.H.get(ctx, 2 * nlev));
-    RC(E.Gw.get(ctx, 4 * nn));
-    RC(E.Gh.get(ctx, 4 * nn));
     RC(E.sig.get(ctx, nn));
     RC(E.q.get(ctx, nlev));
     RC(E.z.get(ctx, nrows ? nrows : 1));
     RC(E.mask.get(ctx, nlev));
 
-    // Lanes per CSR row of the row kernels (W update and the power
-    // iteration's row pass), timed once per batch (a choice from the mean
-    // row length was measured slower on the frontier's small batches).
-    int Gb = -1;
-    auto lanes = [&]() {
-      if (Gb < 0) Gb = E.tune_group(nrows, LONGLEN);
-      return Gb;
-    };
+    const LevelRows rows = {E.row_ptr.p, E.csr_col.p, E.csr_val.p, E.ch_rows.p, E.seg_row.p, E.seg_b.p,
+                            E.llist.p, E.seg_off.p, E.node_long0.p, (int)nseg};
+    const unsigned row_blocks = (unsigned)(nseg + (long)chr.size()), col_blocks = (unsigned)chc.size();
     // Sigma of this level's nodes (children created by the previous level):
     // 100-step power iteration of Node::compute_sigma (hiernmf/node.hpp:66-69).
     std::vector<double> sig(nn, 0.0);
     if (sigma_on) {
       pow_init<<<nb(nlev), 256, 0, ctx->stream>>>(nlev, E.node_of_col.p, E.node_col0.p, E.seeds.p, E.q.p);
-      sumsq_chunks<<<(unsigned)chc.size(), 256, 0, ctx->stream>>>(E.ch_cols.p, E.q.p, E.part.p);
-      norm_finalize<<<nb(nn), 256, 0, ctx->stream>>>(E.part.p, E.cb_cols.p, nn, E.sig.p);
-      const int Gp = lanes();
+      sumsq_chunks<<<col_blocks, 256, 0, ctx->stream>>>(E.ch_cols.p, E.q.p, E.part_h.p);
       for (int it = 0; it < iters; ++it) {
-        E.launch_pow_short(Gp, nrows, LONGLEN);
-        if (nlong) {
-          pow_rows_seg<<<(unsigned)nseg, 256, 0, ctx->stream>>>(E.seg_row.p, E.seg_b.p, E.llist.p, E.row_ptr.p,
-                                                                E.csr_col.p, E.csr_val.p, E.q.p, E.seg_part.p);
-          pow_rows_long_fin<<<nb(nlong, 64), 64, 0, ctx->stream>>>(nlong, E.llist.p, E.seg_off.p, E.seg_part.p,
-                                                                   E.row_node.p, E.sig.p, E.z.p);
-        }
-        pow_cols<<<nb(nlev), 256, 0, ctx->stream>>>(nlev, E.col_ptr.p, E.csc_row.p, E.csc_val.p, E.z.p, E.q.p);
-        sumsq_chunks<<<(unsigned)chc.size(), 256, 0, ctx->stream>>>(E.ch_cols.p, E.q.p, E.part.p);
-        norm_finalize<<<nb(nn), 256, 0, ctx->stream>>>(E.part.p, E.cb_cols.p, nn, E.sig.p);
+        if (row_blocks)
+          pow_rows_kernel<<<row_blocks, 256, 0, ctx->stream>>>(rows, E.q.p, E.part_h.p, E.cb_cols.p, E.z.p,
+                                                               E.seg_part.p);
+        if (nlong)
+          pow_long_kernel<<<(unsigned)nn, 256, 0, ctx->stream>>>(rows, E.seg_part.p, E.part_h.p, E.cb_cols.p, E.z.p);
+        pow_cols_kernel<<<col_blocks, 256, 0, ctx->stream>>>(E.ch_cols.p, E.col_ptr.p, E.csc_row.p, E.csc_val.p,
+                                                             E.z.p, E.q.p, E.part_h.p);
       }
+      norm_finalize<<<(unsigned)nn, 64, 0, ctx->stream>>>(E.part_h.p, E.cb_cols.p, E.sig.p);
       PLANC_LAUNCH_CHECK(ctx);
       if (iters > 0)
         PLANC_HIP_CHECK(ctx, hipMemcpyAsync(sig.data(), E.sig.p, sizeof(double) * nn,
@@ -1027,44 +1191,24 @@ int planc_hiernmf_run(planc_ctx *ctx, const planc_hier_desc *desc, const long *h
     }
     if (!split_on) return PLANC_OK;  // sigma only (leaves of this pass)
 
-    // Rank-2 NMF of every node of the level: the iteration loop is captured
-    // into one hipGraph and launched once.
+    // Rank-2 NMF of every node of the level.
     init_factors<<<nb(nrows + nlev), 256, 0, ctx->stream>>>(nrows, E.row_node.p, E.row_orig.p, nlev,
                                                             E.node_of_col.p, E.node_col0.p, E.seeds.p,
                                                             m, E.W.p, E.H.p);
     init_gram_chunks<<<(unsigned)chi.size(), 256, 0, ctx->stream>>>(E.ch_init.p, E.seeds.p, m, E.part.p);
-    gram2_finalize<<<nb(nn), 256, 0, ctx->stream>>>(E.part.p, E.cb_init.p, nn, E.Gw.p);
     PLANC_LAUNCH_CHECK(ctx);
-    const int Gw = lanes();
-    if (iters > 0) {
-      hipGraphExec_t exec = nullptr;
-      RC(capture_graph(ctx, [&]() -> int {
-        for (int it = 0; it < iters; ++it) {
-          if (it > 0) {
-            if (!chr.empty())
-              gram2_chunks<<<(unsigned)chr.size(), 256, 0, ctx->stream>>>(E.ch_rows.p, E.W.p, E.part.p);
-            gram2_finalize<<<nb(nn), 256, 0, ctx->stream>>>(E.part.p, E.cb_rows.p, nn, E.Gw.p);
-          }
-          h_update<<<nb(nlev), 256, 0, ctx->stream>>>(nlev, E.col_ptr.p, E.csc_row.p, E.csc_val.p,
-                                                     E.node_of_col.p, E.W.p, E.Gw.p, E.H.p);
-          gram2_chunks<<<(unsigned)chc.size(), 256, 0, ctx->stream>>>(E.ch_cols.p, E.H.p, E.part.p);
-          gram2_finalize<<<nb(nn), 256, 0, ctx->stream>>>(E.part.p, E.cb_cols.p, nn, E.Gh.p);
-          E.launch_w_short(Gw, nrows, E.W.p, LONGLEN);
-          if (nlong) {
-            w_update_seg<<<(unsigned)nseg, 256, 0, ctx->stream>>>(E.seg_row.p, E.seg_b.p, E.llist.p, E.row_ptr.p,
-                                                                  E.csr_col.p, E.csr_val.p, E.H.p, E.seg_part.p);
-            w_update_long_fin<<<nb(nlong, 64), 64, 0, ctx->stream>>>(nlong, E.llist.p, E.seg_off.p, E.seg_part.p,
-                                                                     E.row_node.p, E.Gh.p, E.W.p);
-          }
-        }
-        PLANC_LAUNCH_CHECK(ctx);
-        return PLANC_OK;
-      }, &exec));
-      hipError_t ce = hipGraphLaunch(exec, ctx->stream);
-      (void)hipStreamSynchronize(ctx->stream);
-      (void)hipGraphExecDestroy(exec);
-      if (ce != hipSuccess) return set_error(ctx, PLANC_EHIP, std::string("hiernmf launch: ") + hipGetErrorString(ce));
+    const GramParts gh = {E.part_h.p, E.cb_cols.p, nullptr};
+    for (int it = 0; it < iters; ++it) {
+      // W^T W: over all m rows of the initial W first, then over the rows kept.
+      const GramParts gw = {E.part.p, it == 0 ? E.cb_init.p : E.cb_rows.p, it > 0 && nlong ? E.extra.p : nullptr};
+      h_gram_kernel<<<col_blocks, 256, 0, ctx->stream>>>(E.ch_cols.p, E.col_ptr.p, E.csc_row.p, E.csc_val.p, E.W.p, gw,
+                                                         E.H.p, E.part_h.p);
+      if (row_blocks)
+        w_rows_kernel<<<row_blocks, 256, 0, ctx->stream>>>(rows, E.H.p, gh, E.W.p, E.part.p, E.seg_part.p);
+      if (nlong)
+        w_long_kernel<<<(unsigned)nn, 256, 0, ctx->stream>>>(rows, E.seg_part.p, gh, E.W.p, E.extra.p);
     }
+    PLANC_LAUNCH_CHECK(ctx);
     // Split rule H(:,0) >= H(:,1), larger side to the left child
     // (hiernmf/node.hpp:147-185).
     split_mask<<<nb(nlev), 256, 0, ctx->stream>>>(nlev, E.H.p, E.mask.p);
