@@ -9,17 +9,18 @@
 // column; a column that exceeds it reports -1 (the reference exits).
 //
 // One wavefront per right-hand side: lane i owns variable i, the passive set
-// is a 64-bit wave-uniform mask (ballots).  Two forms:
-//  * bpp_pair_kernel: with H = G^-1 formed once for all columns, a pivot step
-//    solves the smaller of the passive and the complementary system (at most
-//    k / 2 variables, compacted).  Bound by FP64 arithmetic and the lane
-//    broadcasts of the elimination (two v_readlane per FMA).  Taken where G's
-//    1-norm condition is at most BPP_COND.
-//  * bpp_kernel: a masked k x k elimination of the passive system per step,
-//    for any other G and for columns the first form gives up.
-// One ANLS-BPP iteration at 65536 x 16384, k = 64 (81920 columns, BF16
-// products): 70.8 ms with the masked elimination of all k columns alone, 2.57
-// ms with the pair (the products are 0.8 ms of it).
+// is a 64-bit wave-uniform mask (ballots), the variables of a step's system are
+// compacted to the first lanes.  Two forms of bpp_kernel:
+//  * the pair: with H = G^-1 formed once for all columns, a step solves the
+//    smaller of the passive and the complementary system (at most k / 2
+//    variables).  Taken where G's 1-norm condition is at most BPP_COND.
+//  * the passive system itself, for any other G and for columns the pair gives
+//    up.
+// Bound by FP64 arithmetic and the lane broadcasts of the elimination (two
+// v_readlane per FMA).  One ANLS-BPP iteration at 65536 x 16384, k = 64 (81920
+// columns, BF16 products): 70.8 ms with a masked elimination of all k columns
+// per step, 1.86 ms so (0.87 ms are the products; 65536 columns by the pair 0.13
+// ms, 16384 at a condition of 6e6 by the passive system 0.64 ms).
 #include <algorithm>
 
 #include "common.h"
@@ -65,159 +66,93 @@ struct Exchange {
   }
 };
 
-// General form: any G.  Takes every column when the shared inverse is not
-// usable (info->ok == 0), else only the columns that bpp_pair_kernel gave up
-// (iters < 0).  Columns of the tableau left of the pivot are already unit
-// vectors, so an elimination step only touches the columns right of it.
-template <int KM>
-__global__ __launch_bounds__(256) void bpp_kernel(const double *G, int k, const float *B, long b_cs,
-                                                  long b_rs, long nrhs, float *X, long x_cs, long x_rs,
-                                                  int maxit, const BppInfo *info, const int *iters, int *failed_out) {
-  __shared__ double Gs[KM][KM + 1];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  const bool all = info->ok == 0;
-  const long stride = (long)gridDim.x * nw;
-  const long col0 = (long)blockIdx.x * nw + wave;
-  if (!all) {
-    int any = 0;
-    for (long c = (long)blockIdx.x * nw + threadIdx.x % nw + (threadIdx.x / nw) * stride; c < nrhs;
-         c += (blockDim.x / nw) * stride)
-      any |= iters[c] < 0;  // the block's columns, spread over its threads
-    if (!__syncthreads_or(any)) return;
-  }
-  for (int e = threadIdx.x; e < KM * KM; e += blockDim.x) {
-    int r = e % KM, c = e / KM;
-    Gs[r][c] = (r < k && c < k) ? G[r + (size_t)k * c] : 0.0;
-  }
-  __syncthreads();
-  const bool live = lane < k;
-  for (long col = col0; col < nrhs; col += stride) {
-    if (!all && iters[col] >= 0) continue;
-    const double b = live ? (double)B[col * b_cs + lane * b_rs] : 0.0;
-    double x = 0.0, y = -b;
-    Exchange ex(k);
-    unsigned long long nonopt = ballot64(live && y < 0.0);
-    unsigned long long infea = 0ull;
-    int iter = 0;
-    bool failed = false;
-    while (nonopt | infea) {
-      if (++iter > maxit) {
-        failed = true;
-        break;
-      }
-      ex.step(nonopt, infea);
-      const unsigned long long P = ex.P;
-      // Masked system [G(P,P) 0; 0 I] x = [b_P; 0], lane = row.
-      const bool pi = (P >> lane) & 1ull;
-      double a[KM];
-#pragma unroll
-      for (int t = 0; t < KM; ++t) {
-        bool pt = (P >> t) & 1ull;
-        a[t] = (pi && pt) ? Gs[lane < KM ? lane : 0][t] : (lane == t ? 1.0 : 0.0);
-      }
-      double rhs = pi ? b : 0.0;
-      double diag = 1.0;
-#pragma unroll
-      for (int j = 0; j < KM; ++j) {
-        if ((P >> j) & 1ull) {
-          const double piv = bcast(a[j], j);
-          const double rj = bcast(rhs, j);
-          const double f = (lane != j) ? a[j] / piv : 0.0;
-          diag = lane == j ? piv : diag;
-#pragma unroll
-          for (int t = j + 1; t < KM; ++t) a[t] = fma(-f, bcast(a[t], j), a[t]);
-          rhs = fma(-f, rj, rhs);
-        }
-      }
-      x = pi ? rhs / diag : 0.0;
-      // Y = G x - b with the full Gram.
-      double gx = 0.0;
-#pragma unroll
-      for (int t = 0; t < KM; ++t) {
-        double xt = bcast(x, t);
-        if (live) gx = fma(Gs[lane][t], xt, gx);
-      }
-      y = live ? gx - b : 0.0;
-      if (fabs(x) < 1e-12) x = 0.0;
-      if (fabs(y) < 1e-12) y = 0.0;
-      nonopt = ballot64(live && y < 0.0 && !pi);
-      infea = ballot64(live && x < 0.0 && pi);
-    }
-    if (live) X[col * x_cs + lane * x_rs] = (float)x;
-    if (failed && lane == 0 && failed_out) *failed_out = 1;
-  }
-}
-
 // ---------------------------------------------------------------------------
-// H = G^-1 once for all columns (in-place Gauss-Jordan of the SPD Gram in
-// LDS, one block), its 1-norm, and whether bpp_pair_kernel may use it: G
-// positive definite with a 1-norm condition of at most BPP_COND, so that a
-// solution formed from H is good to about eps cond^2 <= 2e-6 before its
-// refinement (which squares that).
-constexpr double BPP_COND = 1e5;
-constexpr int BPP_INV_THR = 1024;
+// H = G^-1 once for all columns (in-place Gauss-Jordan of the SPD Gram, one
+// block), its 1-norm, and whether the pair form may use it: G positive
+// definite with a 1-norm condition of at most BPP_COND, so that a solution
+// formed from H is good to about eps cond^2 <= 2e-4, which each refinement
+// multiplies by as much again.  Thread (ty, tx) of 16 x 16 keeps the entries (T
+// ty + a, T tx + b), T = K / 16, in registers; a step passes the pivot's row and
+// column through LDS (two buffers, one barrier a step: a chain of k LDS round
+// trips and reciprocals; held in LDS with two barriers of 1024 threads a step it
+// took 72 us at k = 64).  Rows past k are those of the identity.
+constexpr double BPP_COND = 1e6;
 
-__global__ __launch_bounds__(BPP_INV_THR) void bpp_invert_kernel(const double *G, int k, double *H, BppInfo *info) {
-  __shared__ double S[64][65];
-  __shared__ double nrm[2][64];
-  const int tid = threadIdx.x;
-  const int kk = k * k;
-  constexpr int U = 4096 / BPP_INV_THR;
+template <int T>
+__global__ __launch_bounds__(256) void bpp_invert_kernel(const double *G, int k, double *H, BppInfo *info) {
+  constexpr int K = 16 * T;
+  __shared__ __attribute__((aligned(16))) double row[2][K], col[2][K];
+  __shared__ double out[K][K + 1];
+  __shared__ double nrm[2][K];
+  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
+  double s[T][T];
 #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const int e = tid + u * BPP_INV_THR;
-    if (e < kk) S[e % k][e / k] = G[e];
-  }
-  __syncthreads();
-  auto col_norm = [&](int which) {
-    if (tid < k) {
-      double t = 0.0;
-      for (int i = 0; i < k; ++i) t += fabs(S[i][tid]);
-      nrm[which][tid] = t;
+  for (int a = 0; a < T; ++a)
+#pragma unroll
+    for (int b = 0; b < T; ++b) {
+      const int i = T * ty + a, t = T * tx + b;
+      s[a][b] = i < k && t < k ? G[i + (size_t)k * t] : (i == t ? 1.0 : 0.0);
     }
+  auto col_norms = [&](int which) {
+#pragma unroll
+    for (int a = 0; a < T; ++a)
+#pragma unroll
+      for (int b = 0; b < T; ++b) out[T * ty + a][T * tx + b] = s[a][b];
+    __syncthreads();
+    if (tid < K) {
+      double v = 0.0;
+      for (int i = 0; i < k; ++i) v += fabs(out[i][tid]);
+      nrm[which][tid] = tid < k ? v : 0.0;
+    }
+    __syncthreads();
   };
-  col_norm(0);
-  __syncthreads();
+  col_norms(0);
   bool pos = true;
-  for (int j = 0; j < k; ++j) {
-    const double d = S[j][j];
-    pos = pos && d > 0.0;
-    const double p = 1.0 / d;
-    double v[U];
+  for (int jb = 0; jb * T < k; ++jb) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int e = tid + u * BPP_INV_THR, i = e % k, t = e / k;
-      if (e >= kk) continue;
-      const double aij = S[i][j], ajt = S[j][t];
-      if (i != j && t != j) v[u] = fma(-aij * p, ajt, S[i][t]);
-      else if (i == j && t == j) v[u] = p;
-      else v[u] = i == j ? ajt * p : -aij * p;
-    }
-    __syncthreads();
+    for (int jj = 0; jj < T; ++jj) {
+      const int j = jb * T + jj, buf = (T % 2 == 0 ? jj : j) & 1;
+      if (ty == jb)
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int e = tid + u * BPP_INV_THR;
-      if (e < kk) S[e % k][e / k] = v[u];
+        for (int b = 0; b < T; ++b) row[buf][T * tx + b] = s[jj][b];
+      if (tx == jb)
+#pragma unroll
+        for (int a = 0; a < T; ++a) col[buf][T * ty + a] = s[a][jj];
+      __syncthreads();
+      const double d = row[buf][j];
+      pos = pos && d > 0.0;
+      const double p = 1.0 / d;
+      double rv[T], cv[T];
+#pragma unroll
+      for (int b = 0; b < T; ++b) {
+        rv[b] = row[buf][T * tx + b] * p;
+        cv[b] = col[buf][T * ty + b];
+      }
+#pragma unroll
+      for (int a = 0; a < T; ++a)
+#pragma unroll
+        for (int b = 0; b < T; ++b) {
+          const bool ri = ty == jb && a == jj, ci = tx == jb && b == jj;
+          const double e = fma(-cv[a], rv[b], s[a][b]);
+          s[a][b] = ri ? (ci ? p : rv[b]) : (ci ? -cv[a] * p : e);
+        }
     }
-    __syncthreads();
   }
-  col_norm(1);
   __syncthreads();
+  col_norms(1);
+  for (int e = tid; e < k * k; e += 256) H[e] = 0.5 * (out[e % k][e / k] + out[e / k][e % k]);
+  if (tid < 64) {
+    double g = tid < K ? nrm[0][tid] : 0.0, h = tid < K ? nrm[1][tid] : 0.0;
+    const bool fin = __all(g < 1e300 && h < 1e300);  // NaN fails too
 #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const int e = tid + u * BPP_INV_THR;
-    if (e < kk) H[e] = 0.5 * (S[e % k][e / k] + S[e / k][e % k]);
-  }
-  if (tid == 0) {
-    double g = 0.0, h = 0.0;
-    bool fin = true;
-    for (int i = 0; i < k; ++i) {
-      fin = fin && nrm[0][i] < 1e300 && nrm[1][i] < 1e300;  // NaN fails too
-      g = fmax(g, nrm[0][i]);
-      h = fmax(h, nrm[1][i]);
+    for (int off = 32; off > 0; off >>= 1) {
+      g = fmax(g, __shfl_xor(g, off, 64));
+      h = fmax(h, __shfl_xor(h, off, 64));
     }
-    info->hnorm = h;
-    info->ok = pos && fin && g * h <= BPP_COND;
+    if (tid == 0) {
+      info->hnorm = h;
+      info->ok = pos && fin && g * h <= BPP_COND;
+    }
   }
 }
 
@@ -255,21 +190,29 @@ __device__ inline double gather_solve(const double *M, int sel, double rhs, int 
   return solve_compact<QM>(a, rhs, q, lane);
 }
 
-template <int KM, int LD>
+// QX: the largest q.  Steps of 4 up to 32, of 8 beyond (code size: a system of
+// 64 is 50 KB of unrolled elimination).
+template <int QX, int LD>
 __device__ inline double solve_selected(const double *M, int sel, double rhs, int q, int lane) {
   if (q == 0) return 0.0;
   if (q <= 4) return gather_solve<4, LD>(M, sel, rhs, q, lane);
-  if constexpr (KM > 8)
+  if constexpr (QX > 4)
     if (q <= 8) return gather_solve<8, LD>(M, sel, rhs, q, lane);
-  if constexpr (KM > 16) {
+  if constexpr (QX > 8) {
     if (q <= 12) return gather_solve<12, LD>(M, sel, rhs, q, lane);
     if (q <= 16) return gather_solve<16, LD>(M, sel, rhs, q, lane);
   }
-  if constexpr (KM > 32) {
+  if constexpr (QX > 16) {
     if (q <= 20) return gather_solve<20, LD>(M, sel, rhs, q, lane);
     if (q <= 24) return gather_solve<24, LD>(M, sel, rhs, q, lane);
     if (q <= 28) return gather_solve<28, LD>(M, sel, rhs, q, lane);
-    return gather_solve<32, LD>(M, sel, rhs, q, lane);
+    if (q <= 32) return gather_solve<32, LD>(M, sel, rhs, q, lane);
+  }
+  if constexpr (QX > 32) {
+    if (q <= 40) return gather_solve<40, LD>(M, sel, rhs, q, lane);
+    if (q <= 48) return gather_solve<48, LD>(M, sel, rhs, q, lane);
+    if (q <= 56) return gather_solve<56, LD>(M, sel, rhs, q, lane);
+    return gather_solve<64, LD>(M, sel, rhs, q, lane);
   }
   return 0.0;
 }
@@ -281,26 +224,40 @@ __device__ inline double solve_selected(const double *M, int sel, double rhs, in
 // -w); the smaller one is solved, so no system is larger than k / 2.  One
 // wavefront per column, lane = variable; the selected variables are
 // compacted to the first lanes.  When no variable is left to exchange, the
-// residual of the true normal equations is formed (y = G x - b); if it says
-// that x may be off by more than 1e-10 of its largest entry, one step of
-// refinement is solved on the same set, and the signs are tested again on the
-// final values.
-template <int KM>
-__global__ __launch_bounds__(512) void bpp_pair_kernel(const double *G, const double *H, const BppInfo *info, int k,
-                                                       const float *B, long b_cs, long b_rs, long nrhs, float *X,
-                                                       long x_cs, long x_rs, int maxit, int *iters_out) {
+// residual of the true normal equations is formed (y = G x - b); while it says
+// that x may be off by more than 1e-10 of its largest entry, a step of
+// refinement is solved on the same set (at most BPP_REFINE), and the signs are
+// tested again on the final values.
+// PAIR = false is the form for any other G: every step solves the passive system
+// itself, from G, and nothing is refined.  It takes all columns where the inverse
+// is not usable, else only those that the pair gave up (iters < 0), and sets
+// *failed_out for a column that needs more than maxit steps.
+constexpr int BPP_REFINE = 3;
+template <int KM, bool PAIR>
+__global__ __launch_bounds__(512) void bpp_kernel(const double *G, const double *H, const BppInfo *info, int k,
+                                                  const float *B, long b_cs, long b_rs, long nrhs, float *X,
+                                                  long x_cs, long x_rs, int maxit, int *iters, int *failed_out) {
   constexpr int LD = KM + 1;
-  __shared__ double Gs[KM * LD], Hs[KM * LD];
-  if (!info->ok) return;
+  __shared__ double Gs[KM * LD], Hs[PAIR ? KM * LD : 1];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const long stride = (long)gridDim.x * nw;
+  const bool usable = info->ok != 0;
+  if (PAIR && !usable) return;
+  if (!PAIR && usable) {
+    int any = 0;
+    for (long c = (long)blockIdx.x * nw + threadIdx.x % nw + (threadIdx.x / nw) * stride; c < nrhs;
+         c += (blockDim.x / nw) * stride)
+      any |= iters[c] < 0;  // the block's columns, spread over its threads
+    if (!__syncthreads_or(any)) return;
+  }
   const double hnorm = info->hnorm;
   for (int e = threadIdx.x; e < KM * KM; e += blockDim.x) {
     const int r = e % KM, c = e / KM;
     const bool in = r < k && c < k;
     Gs[r * LD + c] = in ? G[r + (size_t)k * c] : 0.0;
-    Hs[r * LD + c] = in ? H[r + (size_t)k * c] : 0.0;
+    if (PAIR) Hs[r * LD + c] = in ? H[r + (size_t)k * c] : 0.0;
   }
   __syncthreads();
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
   const bool live = lane < k;
   const int row = (lane < KM ? lane : KM - 1) * LD;
   const unsigned long long every = k < 64 ? (1ull << k) - 1ull : ~0ull;
@@ -314,10 +271,10 @@ __global__ __launch_bounds__(512) void bpp_pair_kernel(const double *G, const do
     }
     return s0 + s1;
   };
-  const long stride = (long)gridDim.x * nw;
   for (long col = (long)blockIdx.x * nw + wave; col < nrhs; col += stride) {
+    if (!PAIR && usable && iters[col] >= 0) continue;
     const double b = live ? (double)B[col * b_cs + lane * b_rs] : 0.0;
-    const double c = times(Hs, b);
+    const double c = PAIR ? times(Hs, b) : 0.0;
     double bb = b, cc = c;  // right-hand side of the current solve and H times it
     double x = 0.0, y = -b, xbase = 0.0;
     Exchange ex(k);
@@ -325,6 +282,7 @@ __global__ __launch_bounds__(512) void bpp_pair_kernel(const double *G, const do
     unsigned long long infea = 0ull;
     int iter = 0;
     bool failed = false, refine = false;
+    int refined = 0;
     while (refine || (nonopt | infea)) {
       if (!refine) {
         if (++iter > maxit) {
@@ -332,10 +290,11 @@ __global__ __launch_bounds__(512) void bpp_pair_kernel(const double *G, const do
           break;
         }
         ex.step(nonopt, infea);
+        refined = 0;
       }
       const unsigned long long P = ex.P & every;
       const int np = __popcll(P);
-      const bool primal = 2 * np <= k;
+      const bool primal = !PAIR || 2 * np <= k;
       const int q = primal ? np : k - np;
       const unsigned long long Q = primal ? P : (every & ~P);
       const bool pi = (P >> lane) & 1ull, qi = (Q >> lane) & 1ull;
@@ -345,7 +304,7 @@ __global__ __launch_bounds__(512) void bpp_pair_kernel(const double *G, const do
       const int sel = __builtin_amdgcn_ds_permute(4 * rank, lane);
       const double rhs = __shfl(primal ? bb : cc, sel, 64);
       const double *M = primal ? Gs : Hs;
-      const double w = solve_selected<KM, LD>(M, sel < KM ? sel : 0, lane < q ? rhs : 0.0, q, lane);
+      const double w = solve_selected<PAIR ? KM / 2 : KM, LD>(M, sel < KM ? sel : 0, lane < q ? rhs : 0.0, q, lane);
       const double wv = __shfl(w, rank, 64);  // back in variable order (Q only)
       double s0 = 0.0, s1 = 0.0;  // sum over Q of M(lane, j) w_j
       int j = 0;
@@ -370,19 +329,20 @@ __global__ __launch_bounds__(512) void bpp_pair_kernel(const double *G, const do
         if (fabs(y) < 1e-12) y = 0.0;
         nonopt = ballot64(live && y < 0.0 && !pi);
         infea = ballot64(live && x < 0.0 && pi);
-        if (nonopt | infea) continue;
+        if (!PAIR || (nonopt | infea)) continue;
       } else {
         x = pi ? xbase + xs : 0.0;
         if (fabs(x) < 1e-12) x = 0.0;
       }
       // Nothing left to exchange (or just refined): the true residual.
       y = live ? times(Gs, x) - b : 0.0;
-      if (!refine) {
+      if (refined < BPP_REFINE) {
         float xm = fabsf((float)x);
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) xm = fmaxf(xm, __shfl_xor(xm, off, 64));
         if (ballot64(pi && !(fabs(y) * hnorm <= 1e-10 * (double)xm))) {
           refine = true;
+          ++refined;
           xbase = x;
           bb = pi ? -y : 0.0;
           cc = times(Hs, bb);
@@ -396,8 +356,13 @@ __global__ __launch_bounds__(512) void bpp_pair_kernel(const double *G, const do
       nonopt = ballot64(live && y < 0.0 && !pi);
       infea = ballot64(live && x < 0.0 && pi);
     }
-    if (live && !failed) X[col * x_cs + lane * x_rs] = (float)x;
-    if (lane == 0) iters_out[col] = failed ? -1 : iter;
+    if (PAIR) {
+      if (live && !failed) X[col * x_cs + lane * x_rs] = (float)x;
+      if (lane == 0) iters[col] = failed ? -1 : iter;
+    } else {
+      if (live) X[col * x_cs + lane * x_rs] = (float)x;
+      if (failed && lane == 0 && failed_out) *failed_out = 1;
+    }
   }
 }
 
@@ -415,11 +380,11 @@ static void bpp_launch(planc_ctx *ctx, const double *G, const double *H, const B
   // 64); a few right-hand sides are spread over four-wave blocks instead.
   const int nw = nrhs <= 4L * ctx->num_cu ? 4 : 8;
   const long nb = std::min<long>((nrhs + nw - 1) / nw, 2L * ctx->num_cu);
-  bpp_pair_kernel<KM><<<(unsigned)nb, 64 * nw, 0, ctx->stream>>>(G, H, info, k, B, b_cs, b_rs, nrhs, X, x_cs, x_rs,
-                                                                5 * k, iters);
-  const long gb = std::min<long>((nrhs + 3) / 4, 4L * ctx->num_cu);
-  bpp_kernel<KM><<<(unsigned)gb, 256, 0, ctx->stream>>>(G, k, B, b_cs, b_rs, nrhs, X, x_cs, x_rs, 5 * k, info, iters,
-                                                       d_failed);
+  bpp_kernel<KM, true><<<(unsigned)nb, 64 * nw, 0, ctx->stream>>>(G, H, info, k, B, b_cs, b_rs, nrhs, X, x_cs, x_rs,
+                                                                 5 * k, iters, nullptr);
+  const long gb = std::min<long>((nrhs + 3) / 4, 3L * ctx->num_cu);
+  bpp_kernel<KM, false><<<(unsigned)gb, 256, 0, ctx->stream>>>(G, nullptr, info, k, B, b_cs, b_rs, nrhs, X, x_cs,
+                                                                  x_rs, 5 * k, iters, d_failed);
 }
 
 int bpp_solve(planc_ctx *ctx, const double *G, int k, const float *B, long b_cs, long b_rs, long nrhs,
@@ -431,7 +396,10 @@ int bpp_solve(planc_ctx *ctx, const double *G, int k, const float *B, long b_cs,
   if (!H) return set_error(ctx, PLANC_ENOMEM, "bpp: workspace");
   BppInfo *info = (BppInfo *)(H + 4096);
   int *iters = (int *)(info + 1);
-  bpp_invert_kernel<<<1, BPP_INV_THR, 0, ctx->stream>>>(G, k, H, info);
+  if (k <= 16) bpp_invert_kernel<1><<<1, 256, 0, ctx->stream>>>(G, k, H, info);
+  else if (k <= 32) bpp_invert_kernel<2><<<1, 256, 0, ctx->stream>>>(G, k, H, info);
+  else if (k <= 48) bpp_invert_kernel<3><<<1, 256, 0, ctx->stream>>>(G, k, H, info);
+  else bpp_invert_kernel<4><<<1, 256, 0, ctx->stream>>>(G, k, H, info);
   PLANC_LAUNCH_CHECK(ctx);
   if (k <= 16)
     bpp_launch<16>(ctx, G, H, info, k, B, b_cs, b_rs, nrhs, X, x_cs, x_rs, iters, d_failed);

@@ -1,10 +1,11 @@
 """Batched BPP from the Gram and its shared inverse, against the FP64 oracle,
 at the edges of its compact systems (k / 2 of 4, 8, ... 32 variables) and on
-both sides of the condition limit that selects it.
+both sides of the condition limit that selects it (past it the passive systems
+themselves are solved).
 
 Tolerance per column, relative to the column's largest entry: the results are
 FP32 (2^-24), and the solution is refined to 1e-10 of its largest entry, so
-2e-7 holds both; past the limit (the general kernel) eps * cond is added for
+2e-7 holds both; past the limit eps * cond is added for
 the two FP64 eliminations that are compared."""
 import numpy as np
 import pytest
