@@ -1303,28 +1303,26 @@ int planc_cp_loss_bwd(planc_ctx *ctx, const float *d_X, int nmodes, const long *
   const int N = nmodes;
   if (!d_X || !dims || !d_factors || !d_grads || N < 3 || N > 7 || k <= 0 || k > 64)
     return set_error(ctx, PLANC_EINVAL, "planc_cp_loss_bwd: bad arguments (3..7 modes, k 1..64)");
-  long Imax = 0;
-  for (int i = 0; i < N; ++i) {
+  for (int i = 0; i < N; ++i)
     if (dims[i] <= 0) return set_error(ctx, PLANC_EINVAL, "planc_cp_loss_bwd: empty mode");
-    Imax = std::max(Imax, dims[i]);
-  }
   const int s = cp_split(N, dims);
   long L = 1, R = 1;
   for (int i = 0; i <= s; ++i) L *= dims[i];
   for (int i = s + 1; i < N; ++i) R *= dims[i];
-  float *fb = (float *)ws_get(ctx, 13, sizeof(float) * ((size_t)(L + R) * k + (size_t)k * Imax));
+  long rows = 0;
+  for (int i = 0; i < N; ++i) rows += dims[i];
+  float *fb = (float *)ws_get(ctx, 13, sizeof(float) * (size_t)(L + R + rows) * k);
   const size_t kk = (size_t)k * k;
-  double *db = (double *)ws_get(ctx, 14, sizeof(double) * (N + 1) * kk);
+  double *db = (double *)ws_get(ctx, 14, sizeof(double) * N * kk);
   if (!fb || !db) return set_error(ctx, PLANC_ENOMEM, "planc_cp_loss_bwd: workspace");
-  float *P = fb, *Q = fb + (size_t)L * k, *M = fb + (size_t)(L + R) * k;
-  std::vector<const double *> G(N);
-  double *S = db + N * kk;
-  int rc;
-  for (int i = 0; i < N; ++i) {
-    G[i] = db + i * kk;
-    rc = gram(ctx, d_factors[i], dims[i], k, dims[i], db + i * kk);
-    if (rc) return rc;
-  }
+  float *P = fb, *Q = fb + (size_t)L * k;
+  std::vector<float *> M(N);  // every mode's MTTKRP (k x I)
+  M[0] = fb + (size_t)(L + R) * k;
+  for (int i = 1; i < N; ++i) M[i] = M[i - 1] + dims[i - 1] * k;
+  std::vector<double *> G(N);
+  for (int i = 0; i < N; ++i) G[i] = db + i * kk;
+  int rc = gram_set(ctx, d_factors, dims, N, k, G.data());
+  if (rc) return rc;
   KrpDesc kr{}, kl{};
   kr.nf = N - 1 - s;
   for (int q = s + 1; q < N; ++q) {
@@ -1346,16 +1344,14 @@ int planc_cp_loss_bwd(planc_ctx *ctx, const float *d_X, int nmodes, const long *
   for (int i = 0; i < N; ++i) ldf[i] = dims[i];
   for (int n = 0; n < N; ++n) {
     if (n <= s)
-      rc = contract_projection(ctx, P, L, s + 1, dims, d_factors, ldf, n, k, M, k);
+      rc = contract_projection(ctx, P, L, s + 1, dims, d_factors, ldf, n, k, M[n], k);
     else
       rc = contract_projection(ctx, Q, R, N - 1 - s, dims + s + 1, d_factors + s + 1, ldf + s + 1,
-                               n - s - 1, k, M, k);
-    if (rc) return rc;
-    rc = hadamard_grams(ctx, G.data(), N, n, k, S);
-    if (rc) return rc;
-    rc = cp_grad_from_mttkrp(ctx, d_factors[n], dims[n], k, S, M, d_grads[n]);
+                               n - s - 1, k, M[n], k);
     if (rc) return rc;
   }
+  rc = cp_grads(ctx, N, dims, d_factors, k, G.data(), M.data(), d_grads);
+  if (rc) return rc;
   PLANC_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
   return PLANC_OK;
 }

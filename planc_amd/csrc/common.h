@@ -207,6 +207,8 @@ int thin_gemm(planc_ctx *ctx, int dtype, int trans, const void *A, long lda, lon
 
 // nmf_kernels.hip
 int gram(planc_ctx *ctx, const float *X, long rows, int k, long ldx, double *G);
+// gram() of n <= 8 tight factors in two launches.
+int gram_set(planc_ctx *ctx, const float *const *F, const long *dims, int n, int k, double *const *G);
 int read_bandwidth(planc_ctx *ctx, const void *buf, size_t bytes, int reps, double *gbps);
 // kind 0: MU (eps), kind 1: HALS rows.  N(j, c) = N[j*nrs + c*ncs].
 int row_update(planc_ctx *ctx, int kind, float *H, long n, int k, long ldh, const float *N, long nrs,
@@ -321,8 +323,10 @@ int scale_cols_by(planc_ctx *ctx, const float *A, long I, int k, const double *s
 int cp_noalloc_setup(int device);
 int cp_loss_forward_noalloc(planc_ctx *ctx, const float *X, int N, const long *dims,
                             const float *const *F, int k, double *d_loss);
-int cp_grad_from_mttkrp(planc_ctx *ctx, const float *A, long I, int k, const double *S, const float *M,
-                        float *grad);
+// grads[n] = F[n] (Hadamard of the other G) - M[n]^T for all modes (F[n] dims[n]
+// x k, M[n] k x dims[n], tight).
+int cp_grads(planc_ctx *ctx, int N, const long *dims, const float *const *F, int k, const double *const *G,
+             const float *const *M, float *const *grads);
 int cp_split(int N, const long *dims);
 
 // ntf_kernels.hip

@@ -60,9 +60,23 @@ __global__ __launch_bounds__(NTHR) void read_probe_kernel(const floatx4 *p, long
 constexpr int GCR = 64;
 constexpr int GGROUPS = 4;
 
+// blockIdx.y picks one of a set of matrices, each with its own blocks (nb) and
+// partials.
+struct GramIn {
+  const float *x[8];
+  long rows[8], ldx[8];
+  int nb[8];
+  double *part[8];
+  double *g[8];
+};
+
 template <int KM>
-__global__ __launch_bounds__(NTHR * GGROUPS) void gram_mfma_kernel(const float *X, long rows, int k, long ldx,
-                                                                   double *part) {
+__global__ __launch_bounds__(NTHR * GGROUPS) void gram_mfma_kernel(GramIn in, int k) {
+  const int nblk = in.nb[blockIdx.y];
+  if ((int)blockIdx.x >= nblk) return;
+  const float *X = in.x[blockIdx.y];
+  const long rows = in.rows[blockIdx.y], ldx = in.ldx[blockIdx.y];
+  double *part = in.part[blockIdx.y];
   constexpr int NT = KM / 16, NUP = NT * (NT + 1) / 2, TPW = (NUP + 3) / 4;
   constexpr int PER = GCR * KM / NTHR;  // chunk values per thread
   constexpr int XS = KM * (GCR + 1);    // floats of one group's tile
@@ -107,10 +121,10 @@ __global__ __launch_bounds__(NTHR * GGROUPS) void gram_mfma_kernel(const float *
   }
   // Every group runs the same number of chunk steps (the barriers are
   // block-wide); a group past the last chunk loads zeros.
-  const long cstride = (long)gridDim.x * GGROUPS * GCR;
+  const long cstride = (long)nblk * GGROUPS * GCR;
   const long nsteps = (rows + cstride - 1) / cstride;
   float v[PER];
-  long r0 = ((long)grp * gridDim.x + blockIdx.x) * GCR;
+  long r0 = ((long)grp * nblk + blockIdx.x) * GCR;
   load(r0, v);
   for (long st = 0; st < nsteps; ++st, r0 += cstride) {
     __syncthreads();
@@ -180,8 +194,7 @@ __global__ __launch_bounds__(NTHR * GGROUPS) void gram_mfma_kernel(const float *
 // in j order.
 constexpr int GR_E = 16, GR_J = NTHR / GR_E, GR_U = 16;
 constexpr int gram_reduce_blocks(int kp) { return (kp * kp + GR_E - 1) / GR_E; }
-__global__ __launch_bounds__(NTHR) void gram_reduce_kernel(const double *part, long nparts, int k, int kp,
-                                                           double *G) {
+__device__ inline void gram_reduce(const double *part, long nparts, int k, int kp, double *G) {
   __shared__ double red[GR_J][GR_E];
   const int el = threadIdx.x % GR_E, j = threadIdx.x / GR_E;
   const long e = (long)blockIdx.x * GR_E + el;
@@ -207,6 +220,14 @@ __global__ __launch_bounds__(NTHR) void gram_reduce_kernel(const double *part, l
     const int a = (int)(e % kp), b = (int)(e / kp);
     if (a < k && b < k) G[a + (long)k * b] = t;
   }
+}
+
+__global__ __launch_bounds__(NTHR) void gram_reduce_kernel(const double *part, long nparts, int k, int kp,
+                                                           double *G) {
+  gram_reduce(part, nparts, k, kp, G);
+}
+__global__ __launch_bounds__(NTHR) void gram_reduce_set_kernel(GramIn in, int k, int kp) {
+  gram_reduce(in.part[blockIdx.y], in.nb[blockIdx.y], k, kp, in.g[blockIdx.y]);
 }
 
 // ---------------------------------------------------------------------------
@@ -1259,29 +1280,57 @@ int read_bandwidth(planc_ctx *ctx, const void *buf, size_t bytes, int reps, doub
   return PLANC_OK;
 }
 
-int gram(planc_ctx *ctx, const float *X, long rows, int k, long ldx, double *G) {
-  if (k <= 0 || k > 64 || rows < 0) return set_error(ctx, PLANC_EINVAL, "gram: k must be 1..64");
+// The Grams of n matrices, one partial per block (each block accumulates its
+// chunks; an empty matrix still writes zero partials).
+static int gram_launch(planc_ctx *ctx, GramIn &in, int n, int k) {
+  if (k <= 0 || k > 64) return set_error(ctx, PLANC_EINVAL, "gram: k must be 1..64");
   const int kp = ((k + 15) / 16) * 16;
-  long nchunks = (rows + GCR - 1) / GCR;
-  if (nchunks == 0) nchunks = 1;
-  long nb = nchunks < ctx->num_cu ? nchunks : ctx->num_cu;
-  // One partial per block (each block accumulates its chunks; rows == 0
-  // still writes zero partials).
-  double *part = (double *)ws_get(ctx, 1, sizeof(double) * (size_t)nb * kp * kp);
+  int nbmax = 1;
+  size_t tot = 0;
+  for (int i = 0; i < n; ++i) {
+    if (in.rows[i] < 0) return set_error(ctx, PLANC_EINVAL, "gram: k must be 1..64");
+    long nchunks = (in.rows[i] + GCR - 1) / GCR;
+    if (nchunks == 0) nchunks = 1;
+    in.nb[i] = (int)(nchunks < ctx->num_cu ? nchunks : ctx->num_cu);
+    if (in.nb[i] > nbmax) nbmax = in.nb[i];
+    tot += in.nb[i];
+  }
+  double *part = (double *)ws_get(ctx, 1, sizeof(double) * tot * kp * kp);
   if (!part) return set_error(ctx, PLANC_ENOMEM, "gram: workspace");
+  for (int i = 0; i < n; ++i) {
+    in.part[i] = part;
+    part += (size_t)in.nb[i] * kp * kp;
+  }
   const unsigned nt = NTHR * GGROUPS;
-  if (kp == 16)
-    gram_mfma_kernel<16><<<(unsigned)nb, nt, 0, ctx->stream>>>(X, rows, k, ldx, part);
-  else if (kp == 32)
-    gram_mfma_kernel<32><<<(unsigned)nb, nt, 0, ctx->stream>>>(X, rows, k, ldx, part);
-  else if (kp == 48)
-    gram_mfma_kernel<48><<<(unsigned)nb, nt, 0, ctx->stream>>>(X, rows, k, ldx, part);
-  else
-    gram_mfma_kernel<64><<<(unsigned)nb, nt, 0, ctx->stream>>>(X, rows, k, ldx, part);
+  const dim3 grid((unsigned)nbmax, (unsigned)n);
+  if (kp == 16) gram_mfma_kernel<16><<<grid, nt, 0, ctx->stream>>>(in, k);
+  else if (kp == 32) gram_mfma_kernel<32><<<grid, nt, 0, ctx->stream>>>(in, k);
+  else if (kp == 48) gram_mfma_kernel<48><<<grid, nt, 0, ctx->stream>>>(in, k);
+  else gram_mfma_kernel<64><<<grid, nt, 0, ctx->stream>>>(in, k);
   PLANC_LAUNCH_CHECK(ctx);
-  gram_reduce_kernel<<<(unsigned)gram_reduce_blocks(kp), NTHR, 0, ctx->stream>>>(part, nb, k, kp, G);
+  gram_reduce_set_kernel<<<dim3((unsigned)gram_reduce_blocks(kp), (unsigned)n), NTHR, 0, ctx->stream>>>(in, k, kp);
   PLANC_LAUNCH_CHECK(ctx);
   return PLANC_OK;
+}
+
+int gram(planc_ctx *ctx, const float *X, long rows, int k, long ldx, double *G) {
+  GramIn in{};
+  in.x[0] = X;
+  in.rows[0] = rows;
+  in.ldx[0] = ldx;
+  in.g[0] = G;
+  return gram_launch(ctx, in, 1, k);
+}
+
+int gram_set(planc_ctx *ctx, const float *const *F, const long *dims, int n, int k, double *const *G) {
+  if (n < 1 || n > 8) return set_error(ctx, PLANC_EINVAL, "gram_set: 1..8 matrices");
+  GramIn in{};
+  for (int i = 0; i < n; ++i) {
+    in.x[i] = F[i];
+    in.rows[i] = in.ldx[i] = dims[i];
+    in.g[i] = G[i];
+  }
+  return gram_launch(ctx, in, n, k);
 }
 
 int row_update(planc_ctx *ctx, int kind, float *H, long n, int k, long ldh, const float *N, long nrs,
