@@ -170,13 +170,16 @@ int nmf_loop(planc_ctx *ctx, const planc_nmf_desc *desc, NMFProducts &P, float *
   // Loop buffers.
   float *fbuf = (float *)ws_get(ctx, 4, sizeof(float) * ((size_t)k * n + (size_t)m * k));
   const size_t kk = (size_t)k * k;
-  double *dbuf = (double *)ws_get(ctx, 5, sizeof(double) * (4 * kk + 8 + (size_t)iters));
+  // Four Grams, ||A||^2 and a trace, the errors, then NMF_ERR_RING pairs (W^T W,
+  // H^T H) of the MU / HALS iterations whose errors are still to be formed.
+  double *dbuf = (double *)ws_get(ctx, 5, sizeof(double) * ((4 + 2 * NMF_ERR_RING) * kk + 8 + (size_t)iters));
   if (!fbuf || !dbuf) return set_error(ctx, PLANC_ENOMEM, "planc_nmf_run: workspace");
   float *WtA = fbuf;                // k x n
   float *AH = fbuf + (size_t)k * n;  // m x k
   double *WtW = dbuf, *HtH = dbuf + kk, *Greg = dbuf + 2 * kk, *WtW2 = dbuf + 3 * kk;
   double *normA2 = dbuf + 4 * kk, *dotv = normA2 + 1, *nrm = normA2 + 2;  // nrm unused slot
   double *rel = normA2 + 8;
+  double *ring = rel + iters;  // W^T W of place p at ring + 2 p kk, H^T H behind it
   (void)nrm;
   int rc;
 #define RC(x)          \
@@ -319,6 +322,8 @@ int nmf_loop(planc_ctx *ctx, const planc_nmf_desc *desc, NMFProducts &P, float *
   const bool fuseH = rows_gram_ok(d_H, n, WtA, k, 1, k);
   const bool fuseW = algo == PLANC_MU && rows_gram_ok(d_W, m, AH, 1, m, k);
   for (int it = 0; it < iters; ++it) {
+    const int place = it % NMF_ERR_RING;
+    double *HtH = ring + 2 * place * kk + kk, *WtW2 = ring + 2 * place * kk;
     // H half-step: W^T A, W^T W (+ regH).
     RC(P.wta(d_W, WtA));
     if (!wtw_valid) RC(gram(ctx, d_W, m, k, m, WtW));
@@ -330,7 +335,7 @@ int nmf_loop(planc_ctx *ctx, const planc_nmf_desc *desc, NMFProducts &P, float *
     }
     if (fuseH)
       RC(row_update_gram(ctx, algo == PLANC_MU ? 0 : 1, d_H, n, k, n, WtA, k, 1, Gh, 1e-17f, HtH, nullptr,
-                         nullptr));
+                         nullptr, 0));
     else
       RC(row_update(ctx, algo == PLANC_MU ? 0 : 1, d_H, n, k, n, WtA, k, 1, Gh, 1e-17f));
     // W half-step: A H, H^T H (+ regW).
@@ -349,16 +354,18 @@ int nmf_loop(planc_ctx *ctx, const planc_nmf_desc *desc, NMFProducts &P, float *
     long ndp = 0;
     if (fuseW) {
       RC(row_update_gram(ctx, 0, d_W, m, k, m, AH, 1, m, Gw, 1e-17f, WtW2,
-                         desc->compute_error ? &dparts : nullptr, &ndp));
+                         desc->compute_error ? &dparts : nullptr, &ndp, place));
     } else {
       if (algo == PLANC_MU)
         RC(row_update(ctx, 0, d_W, m, k, m, AH, 1, m, Gw, 1e-17f));
       else
         RC(hals_cols(ctx, d_W, m, k, m, AH, m, Gw));
       RC(gram(ctx, d_W, m, k, m, WtW2));
-      if (desc->compute_error) RC(dot_parts(ctx, d_W, 1, m, AH, 1, m, m, k, &dparts, &ndp));
+      if (desc->compute_error) RC(dot_parts(ctx, d_W, 1, m, AH, 1, m, m, k, &dparts, &ndp, place));
     }
-    if (desc->compute_error) RC(nmf_relerr_parts(ctx, normA2, dparts, ndp, WtW2, HtH, k, rel + it));
+    if (desc->compute_error && (place == NMF_ERR_RING - 1 || it == iters - 1))
+      RC(nmf_relerr_parts(ctx, normA2, dparts - place * ndp, ndp, ndp, ring, ring + kk, 2 * (long)kk, k,
+                          rel + it - place, place + 1));
     if (algo == PLANC_HALS) {
       // normalize_by_W: the column norms are the square roots of diag(W^T W);
       // the next W^T W is D^-1 (W^T W) D^-1.
@@ -366,7 +373,7 @@ int nmf_loop(planc_ctx *ctx, const planc_nmf_desc *desc, NMFProducts &P, float *
       RC(scale_cols(ctx, d_W, m, m, d_H, n, n, k, wnorms));
       RC(gram_rescale(ctx, WtW2, k, wnorms, WtW));
     } else {
-      std::swap(WtW, WtW2);  // this W^T W serves the next H half-step
+      WtW = WtW2;  // this W^T W serves the next H half-step
     }
     wtw_valid = true;
   }

@@ -216,13 +216,14 @@ int row_update(planc_ctx *ctx, int kind, float *H, long n, int k, long ldh, cons
 int hals_cols(planc_ctx *ctx, float *W, long m, int k, long ldw, const float *AH, long ldah,
               const double *G);
 // row_update fused with the FP64 Gram of the updated rows (into Gout, k x k)
-// and, with dparts, FP64 block partials of <updated rows, N> (*ndp of them,
-// workspace slot 3, for nmf_relerr_parts).  rows_gram_ok: the layouts it
+// and, with dparts, FP64 block partials of <updated rows, N> (*ndp of them, at
+// place `slot` of NMF_ERR_RING in workspace slot 3, for nmf_relerr_parts).  rows_gram_ok: the layouts it
 // takes (N column-major, nrs == 1, or row-major, ncs == 1; leading
 // dimensions multiples of 4; 16-byte aligned H and N; k <= 64).
 bool rows_gram_ok(const float *H, long ldh, const float *N, long nrs, long ncs, int k);
+constexpr int NMF_ERR_RING = 16;
 int row_update_gram(planc_ctx *ctx, int kind, float *H, long n, int k, long ldh, const float *N, long nrs,
-                    long ncs, const double *G, float eps, double *Gout, double **dparts, long *ndp);
+                    long ncs, const double *G, float eps, double *Gout, double **dparts, long *ndp, int slot);
 int col_norms(planc_ctx *ctx, const float *X, long rows, int k, long ldx, double *norms);
 // NCPFactors::normalize() of n tight factors (dims[i] x k, ld dims[i]) with
 // lambda = the product of their column norms and G[i] = the FP64 Gram of
@@ -237,12 +238,13 @@ int dot(planc_ctx *ctx, const float *X, long xrs, long xcs, const float *Y, long
         long rows, long cols, double *out, int accumulate);
 int nmf_relerr(planc_ctx *ctx, const double *normA2, const double *dotv, const double *WtW,
                const double *HtH, int k, double *relerr_out, double *fit_out);
-// dot() without its final sum: the block partials (workspace slot 3) and
-// their count; nmf_relerr_parts sums them inside the error kernel.
+// dot() without its final sum: the block partials (place `slot` of workspace
+// slot 3) and their count; nmf_relerr_parts sums them inside the error kernel,
+// for n consecutive places at a time.
 int dot_parts(planc_ctx *ctx, const float *X, long xrs, long xcs, const float *Y, long yrs, long ycs,
-              long rows, long cols, double **part, long *nparts);
-int nmf_relerr_parts(planc_ctx *ctx, const double *normA2, const double *part, long nparts, const double *WtW,
-                     const double *HtH, int k, double *relerr_out);
+              long rows, long cols, double **part, long *nparts, int slot);
+int nmf_relerr_parts(planc_ctx *ctx, const double *normA2, const double *part, long nparts, long pstride,
+                     const double *WtW, const double *HtH, long gstride, int k, double *relerr_out, int n);
 int apply_reg(planc_ctx *ctx, double *G, int k, const double *reg);
 // hi = X rounded to dtype's 16-bit format (as float), lo = X - hi; Y += X.
 // G += sr I, R(j, c) += sr F(j, c) (R element (j, c) at R[j*rs + c*cs]); no-op for sr <= 0.

@@ -987,10 +987,19 @@ __global__ __launch_bounds__(NTHR) void sum_partials_kernel(const double *part, 
 // sqrt(fit^2)/||A||, or 1 when fit^2 <= 0 (common/nmf.hpp:462).  <W, A H>
 // is *dotv, or (dotv null) the sum of the nparts block partials of a dot
 // kernel, taken here as sum_partials_kernel takes it.
+// Block b takes the b-th of a run of iterations whose Grams lie gstride apart
+// and whose partials lie pstride apart: the loops leave up to NMF_ERR_RING of
+// them to one launch (a launch of its own per iteration, 4.4 us of a chain of
+// dependent ones, was 9% of a 2000 x 1000, k = 20 MU iteration).
 __global__ __launch_bounds__(NTHR) void nmf_relerr_kernel(const double *normA2, const double *dotv,
                                                           const double *WtW, const double *HtH, int k,
                                                           double *relerr_out, double *fit_out,
-                                                          const double *part, long nparts) {
+                                                          const double *part, long nparts, long gstride,
+                                                          long pstride) {
+  WtW += blockIdx.x * gstride;
+  HtH += blockIdx.x * gstride;
+  part += blockIdx.x * pstride;
+  relerr_out += blockIdx.x;
   __shared__ double red[NTHR / 64];
   // tr(WtW HtH): the loads of the first 16 NTHR products are issued before
   // the partial sum (one round trip for both at k <= 64).
@@ -1375,7 +1384,7 @@ bool rows_gram_ok(const float *H, long ldh, const float *N, long nrs, long ncs, 
 }
 
 int row_update_gram(planc_ctx *ctx, int kind, float *H, long n, int k, long ldh, const float *N, long nrs,
-                    long ncs, const double *G, float eps, double *Gout, double **dparts, long *ndp) {
+                    long ncs, const double *G, float eps, double *Gout, double **dparts, long *ndp, int slot) {
   if (!rows_gram_ok(H, ldh, N, nrs, ncs, k))
     return set_error(ctx, PLANC_EINVAL, "row_update_gram: layout not supported");
   const bool nrow = ncs == 1;
@@ -1386,8 +1395,9 @@ int row_update_gram(planc_ctx *ctx, int kind, float *H, long n, int k, long ldh,
   if (nb > ctx->num_cu) nb = ctx->num_cu;
   if (nb < 1) nb = 1;
   double *gpart = (double *)ws_get(ctx, 1, sizeof(double) * (size_t)nb * kp * kp);
-  double *dpart = dparts ? (double *)ws_get(ctx, 3, sizeof(double) * (size_t)nb) : nullptr;
+  double *dpart = dparts ? (double *)ws_get(ctx, 3, sizeof(double) * (size_t)nb * NMF_ERR_RING) : nullptr;
   if (!gpart || (dparts && !dpart)) return set_error(ctx, PLANC_ENOMEM, "row_update_gram: workspace");
+  if (dpart) dpart += (long)slot * nb;
   int rc;
   if (kp == 16) rc = launch_rows_gram<16>(ctx, kind, H, n, k, ldh, N, ldn, nrow, G, eps, gpart, nb, dpart);
   else if (kp == 32) rc = launch_rows_gram<32>(ctx, kind, H, n, k, ldh, N, ldn, nrow, G, eps, gpart, nb, dpart);
@@ -1456,13 +1466,14 @@ int scale_cols(planc_ctx *ctx, float *X, long rows, long ldx, float *Y, long yro
 // The partial kernel of dot(): one FP64 partial per block into workspace
 // slot 3 (*part, *nparts).
 int dot_parts(planc_ctx *ctx, const float *X, long xrs, long xcs, const float *Y, long yrs, long ycs,
-              long rows, long cols, double **part_out, long *nparts) {
+              long rows, long cols, double **part_out, long *nparts, int slot) {
   long tot = rows * cols;
   long nb = (tot + NTHR * 8 - 1) / (NTHR * 8);
   if (nb > 2048) nb = 2048;
   if (nb < 1) nb = 1;
-  double *part = (double *)ws_get(ctx, 3, sizeof(double) * (size_t)nb);
+  double *part = (double *)ws_get(ctx, 3, sizeof(double) * (size_t)nb * NMF_ERR_RING);
   if (!part) return set_error(ctx, PLANC_ENOMEM, "dot: workspace");
+  part += (long)slot * nb;
   const bool flat = xrs == 1 && yrs == 1 && (cols == 1 || (xcs == rows && ycs == rows)) &&
                     (uintptr_t)X % 16 == 0 && (uintptr_t)Y % 16 == 0;
   if (flat)
@@ -1499,16 +1510,18 @@ int dot(planc_ctx *ctx, const float *X, long xrs, long xcs, const float *Y, long
 
 int nmf_relerr(planc_ctx *ctx, const double *normA2, const double *dotv, const double *WtW,
                const double *HtH, int k, double *relerr_out, double *fit_out) {
-  nmf_relerr_kernel<<<1, NTHR, 0, ctx->stream>>>(normA2, dotv, WtW, HtH, k, relerr_out, fit_out, nullptr, 0);
+  nmf_relerr_kernel<<<1, NTHR, 0, ctx->stream>>>(normA2, dotv, WtW, HtH, k, relerr_out, fit_out, nullptr, 0, 0, 0);
   PLANC_LAUNCH_CHECK(ctx);
   return PLANC_OK;
 }
 
-// The NMF error of <W, A H> = sum of the dot partials of dot_parts(): the
-// partial sum and the error in one launch.
-int nmf_relerr_parts(planc_ctx *ctx, const double *normA2, const double *part, long nparts, const double *WtW,
-                     const double *HtH, int k, double *relerr_out) {
-  nmf_relerr_kernel<<<1, NTHR, 0, ctx->stream>>>(normA2, nullptr, WtW, HtH, k, relerr_out, nullptr, part, nparts);
+// The errors of n consecutive iterations, <W, A H> of each the sum of its dot
+// partials (nparts of them every pstride), its Grams every gstride.
+int nmf_relerr_parts(planc_ctx *ctx, const double *normA2, const double *part, long nparts, long pstride,
+                     const double *WtW, const double *HtH, long gstride, int k, double *relerr_out, int n) {
+  if (n <= 0) return PLANC_OK;
+  nmf_relerr_kernel<<<n, NTHR, 0, ctx->stream>>>(normA2, nullptr, WtW, HtH, k, relerr_out, nullptr, part, nparts,
+                                                gstride, pstride);
   PLANC_LAUNCH_CHECK(ctx);
   return PLANC_OK;
 }

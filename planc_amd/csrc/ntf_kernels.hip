@@ -416,7 +416,7 @@ __global__ __launch_bounds__(4 * MRT *(NVB > 0 ? NVB : 1)) void mode_rows_kernel
     for (int u = 0; u < Q; ++u) {
       const int t = q * Q + u;
       Us[t][rr] = valid ? h[u] : 0.0f;
-      Ms[t][rr] = valid ? mv[u] : 0.0f;
+      if (p.rel_out) Ms[t][rr] = valid ? mv[u] : 0.0f;
       if (NVB == 0 && valid && t < k) p.F[i + p.ldf * t] = h[u];
     }
     const bool more = NVB == 0 && r0 + stride < p.I;
@@ -456,8 +456,10 @@ __global__ __launch_bounds__(4 * MRT *(NVB > 0 ? NVB : 1)) void mode_rows_kernel
 #pragma unroll
       for (int j = 0; j < TPW; ++j) gacc[j] += g2[j];
     }
-    // Column dots sum_r U(r, c) M(c, r): pair (c, quarter) = gt + NTH j,
-    // the four quarters of a column in consecutive lanes (quad sum below).
+    // Column dots sum_r U(r, c) M(c, r), which only the error needs: pair (c,
+    // quarter) = gt + NTH j, the four quarters of a column in consecutive lanes
+    // (quad sum below).
+    if (p.rel_out)
 #pragma unroll
     for (int j = 0; j < NDP; ++j) {
       const int pi = gt + NTH * j;
