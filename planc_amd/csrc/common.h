@@ -286,8 +286,10 @@ struct SparseOps {
   const int *t_indices = nullptr;
   const float *t_values = nullptr;
 };
+// (out_entries, optional: the entry of the CSR behind each of the transpose.)
 int csr_transpose(planc_ctx *ctx, long m, long n, long nnz, const long *indptr, const int *indices,
-                  const float *values, long *out_indptr, int *out_indices, float *out_values);
+                  const float *values, long *out_indptr, int *out_indices, float *out_values,
+                  int *out_entries = nullptr);
 int spmm_plan(planc_ctx *ctx, int slot, long rows, const long *indptr, long nnz, SpmmPlan *plan);
 int spmm_csr(planc_ctx *ctx, const SpmmPlan &plan, long rows, const long *indptr, const int *indices,
              const float *values, const float *F, long ldf, int k, float *out, long ors, long ocs);

@@ -180,6 +180,7 @@ __global__ void r2_update_kernel(const double *G, const float *R, long r_js, lon
 
 struct Chunk {
   int node;
+  int q0, q1;  // the node's chunks on the other side (rows / columns): the Gram partials it needs
   long b, e;
 };
 
@@ -205,55 +206,51 @@ __device__ inline void block_sum3(double &s0, double &s1, double &s2, double (*r
   }
 }
 
-// Partials of a node's 2 x 2 Gram (x0^2, x0 x1, x1^2): chunks [cb[t], cb[t+1])
-// of `part` and, with `extra`, entry t of it (the long rows' share).
-struct GramParts {
-  const double *part;
-  const int *cb;
-  const double *extra;
+// Sums over a node's chunk partials, Q values each, by the first wavefront: lane
+// j takes chunks j, j + 64, ...  The first of them is loaded ahead (load()), so
+// that it is in flight while the block works on its rows or columns.  A node of
+// up to FEW_CHUNKS chunks adds them in chunk order.
+constexpr int FEW_CHUNKS = 16;
+template <int Q>
+struct PartSum {
+  double v[Q];
+  __device__ void load(const double *part, int q0, int q1) {
+    const int j = q0 + (int)threadIdx.x;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) v[q] = threadIdx.x < 64 && j < q1 ? part[(long)Q * j + q] : 0.0;
+  }
+  __device__ void sum(const double *part, int q0, int q1, double (&s)[Q]) {  // the first wavefront
+#pragma unroll
+    for (int q = 0; q < Q; ++q) s[q] = 0.0;
+    if (q1 - q0 <= FEW_CHUNKS) {
+      for (int j = 0; j < q1 - q0; ++j)
+#pragma unroll
+        for (int q = 0; q < Q; ++q) s[q] += __shfl(v[q], j, 64);
+      return;
+    }
+    for (int j = q0 + 64 + (int)threadIdx.x; j < q1; j += 64)
+#pragma unroll
+      for (int q = 0; q < Q; ++q) v[q] += part[(long)Q * j + q];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+      for (int q = 0; q < Q; ++q) v[q] += __shfl_xor(v[q], off, 64);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) s[q] = v[q];
+  }
 };
 
-// Sum of entries b, b + st, ... < e in order, eight loads in flight.
-__device__ inline double ordered_sum(const double *part, long b, long e, long st) {
-  double s = 0;
-  for (; b + 7 * st < e; b += 8 * st) {
-    double v[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = part[b + u * st];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) s += v[u];
-  }
-  for (; b < e; b += st) s += part[b];
-  return s;
-}
-
-// A node of up to FEW_CHUNKS chunks sums them in chunk order, a larger one by
-// the lanes of a wavefront.
-constexpr int FEW_CHUNKS = 16;
-
-// The Gram of node t (column-major) into G, by the first wavefront; ends with a
-// barrier.
-__device__ inline void node_gram(const GramParts &p, int t, double *G) {
+// A node's 2 x 2 Gram (column-major) into G from partials (x0^2, x0 x1, x1^2) and,
+// with `extra`, entry t of it (the long rows' share); ends with a barrier.
+__device__ inline void node_gram(PartSum<3> &ps, const double *part, int q0, int q1, const double *extra, int t,
+                                 double *G) {
   if (threadIdx.x < 64) {
-    const long b = p.cb[t], e = p.cb[t + 1];
-    double s[3] = {0, 0, 0};
-    if (e - b <= FEW_CHUNKS) {
-      const int i = threadIdx.x < 3 ? threadIdx.x : 0;
-      const double v = ordered_sum(p.part, 3 * b + i, 3 * e, 3);
-#pragma unroll
-      for (int q = 0; q < 3; ++q) s[q] = __shfl(v, q, 64);
-    } else {
-#pragma unroll
-      for (int q = 0; q < 3; ++q) s[q] = ordered_sum(p.part, 3 * (b + threadIdx.x) + q, 3 * e, 3 * 64);
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1)
-#pragma unroll
-        for (int q = 0; q < 3; ++q) s[q] += __shfl_xor(s[q], off, 64);
-    }
+    double s[3];
+    ps.sum(part, q0, q1, s);
     if (threadIdx.x == 0) {
 #pragma unroll
       for (int q = 0; q < 3; ++q)
-        if (p.extra) s[q] += p.extra[3 * t + q];
+        if (extra) s[q] += extra[3 * t + q];
       G[0] = s[0];
       G[1] = s[1];
       G[2] = s[1];
@@ -263,19 +260,12 @@ __device__ inline void node_gram(const GramParts &p, int t, double *G) {
   __syncthreads();
 }
 
-// sqrt of the sum of node t's chunk partials into *out, likewise.
-__device__ inline void node_norm(const double *part, const int *cb, int t, double *out) {
+// sqrt of the sum of a node's chunk partials into *out, likewise.
+__device__ inline void node_norm(PartSum<1> &ps, const double *part, int q0, int q1, double *out) {
   if (threadIdx.x < 64) {
-    const long b = cb[t], e = cb[t + 1];
-    double s;
-    if (e - b <= FEW_CHUNKS) {
-      s = ordered_sum(part, b, e, 1);
-    } else {
-      s = ordered_sum(part, b + threadIdx.x, e, 64);
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-    }
-    if (threadIdx.x == 0) *out = sqrt(s);
+    double s[1];
+    ps.sum(part, q0, q1, s);
+    if (threadIdx.x == 0) *out = sqrt(s[0]);
   }
   __syncthreads();
 }
@@ -389,14 +379,18 @@ __device__ inline double dot1_range(long b, long e1, long S, const int *__restri
 // column's entries, the R2 rule with the node's W^T W, and the chunk's part of
 // H^T H.
 __global__ __launch_bounds__(256) void h_gram_kernel(const Chunk *ch, const long *col_ptr, const int *csc_row,
-                                                     const float *csc_val, const double *W, GramParts gw, double *H,
-                                                     double *part) {
+                                                     const float *csc_val, const double *W, const double *gw,
+                                                     const double *extra, int init_chunks, double *H, double *part) {
   __shared__ double G[4], red[3][4];
   const Chunk c = ch[blockIdx.x];
+  // (W^T W of the initial W: init_chunks partials per node.)
+  const int q0 = init_chunks ? c.node * init_chunks : c.q0, q1 = init_chunks ? q0 + init_chunks : c.q1;
+  PartSum<3> ps;
+  ps.load(gw, q0, q1);
   const long lc = c.b + threadIdx.x;
   double s0 = 0, s1 = 0;
   if (lc < c.e) dot2_range(col_ptr[lc], col_ptr[lc + 1], 1, csc_row, csc_val, (const double2 *)W, s0, s1);
-  node_gram(gw, c.node, G);
+  node_gram(ps, gw, q0, q1, extra, c.node, G);
   double x0 = 0, x1 = 0;
   if (lc < c.e) {
     r2_solve(G, s0, s1, x0, x1);
@@ -477,10 +471,11 @@ __device__ inline double few_sum(long b, long e, const int *__restrict__ idx, co
 
 // Sums over one row of a row chunk for every thread's row: few(b, e) sums a
 // short one, one(b, e, S) entries b, b + S, ... < e, group_add the lanes of a
-// group.  sv: 256 values in LDS, list / cnt the medium rows.
+// group.  sv: 256 values in LDS, list / cnt the medium rows, sb / sn where they
+// begin and their lengths.
 template <class V, class Few, class One, class Add>
 __device__ inline V chunk_row_sum(const LevelRows &L, const Chunk &c, Few few, One one, Add group_add, V *sv, int *list,
-                                  int *cnt, bool &is_long) {
+                                  int *cnt, long *sb, int *sn, bool &is_long) {
   const int tid = threadIdx.x;
   const long r = c.b + tid;
   long b = 0, e = 0;
@@ -492,14 +487,18 @@ __device__ inline V chunk_row_sum(const LevelRows &L, const Chunk &c, Few few, O
   __syncthreads();
   is_long = e - b > LONG_ROW;
   const bool medium = e - b > SHORT_ROW && !is_long;
-  if (medium) list[atomicAdd(cnt, 1)] = tid;
+  if (medium) {
+    list[atomicAdd(cnt, 1)] = tid;
+    sb[tid] = b;
+    sn[tid] = (int)(e - b);
+  }
   V v = V();
   if (!medium && !is_long) v = few(b, e);
   __syncthreads();
   for (int i = tid / 16; i < *cnt; i += 16) {
     const int t = list[i];
-    const long mb = L.row_ptr[c.b + t], me = L.row_ptr[c.b + t + 1];
-    V m = group_add(one(mb + tid % 16, me, 16L));
+    const long mb = sb[t];
+    V m = group_add(one(mb + tid % 16, mb + sn[t], 16L));
     if (tid % 16 == 0) sv[t] = m;
   }
   __syncthreads();
@@ -512,11 +511,12 @@ struct Pair {
 
 // W update: (A H)(r, :) over the compacted row's entries, then the R2 rule with
 // the node's H^T H, and the chunk's part of W^T W (long rows: w_long_kernel).
-__global__ __launch_bounds__(256) void w_rows_kernel(LevelRows L, const double *H, GramParts gh, double *W,
+__global__ __launch_bounds__(256) void w_rows_kernel(LevelRows L, const double *H, const double *gh, double *W,
                                                      double *part, double *seg_part) {
   __shared__ double G[4], red[3][4];
   __shared__ Pair sv[256];
-  __shared__ int list[256], cnt;
+  __shared__ long sb[256];
+  __shared__ int list[256], sn[256], cnt;
   const int *col = L.col;
   const float *val = L.val;
   auto one = [&](long b, long e, long S) {
@@ -538,6 +538,8 @@ __global__ __launch_bounds__(256) void w_rows_kernel(LevelRows L, const double *
   }
   const int ci = (int)blockIdx.x - L.nseg;
   const Chunk c = L.ch[ci];
+  PartSum<3> ps;
+  ps.load(gh, c.q0, c.q1);
   bool is_long;
   auto few = [&](long b, long e) {
     Pair p;
@@ -558,8 +560,8 @@ __global__ __launch_bounds__(256) void w_rows_kernel(LevelRows L, const double *
         q.b = group_sum<16>(q.b);
         return q;
       },
-      sv, list, &cnt, is_long);
-  node_gram(gh, c.node, G);
+      sv, list, &cnt, sb, sn, is_long);
+  node_gram(ps, gh, c.q0, c.q1, nullptr, c.node, G);
   const long r = c.b + threadIdx.x;
   double x0 = 0, x1 = 0;
   if (r < c.e && !is_long) {
@@ -576,14 +578,17 @@ __global__ __launch_bounds__(256) void w_rows_kernel(LevelRows L, const double *
 }
 
 // A block per node: its long rows, and their part of W^T W.
-__global__ __launch_bounds__(256) void w_long_kernel(LevelRows L, const double *seg_part, GramParts gh, double *W,
-                                                     double *extra) {
+__global__ __launch_bounds__(256) void w_long_kernel(LevelRows L, const double *seg_part, const double *gh,
+                                                     const int *cb, double *W, double *extra) {
   __shared__ double G[4], red[3][4];
   const int t = blockIdx.x;
   const int j0 = L.node_long0[t], j1 = L.node_long0[t + 1];
   double g0 = 0, g1 = 0, g2 = 0;
   if (j0 < j1) {  // uniform over the block
-    node_gram(gh, t, G);
+    PartSum<3> ps;
+    const int q0 = cb[t], q1 = cb[t + 1];
+    ps.load(gh, q0, q1);
+    node_gram(ps, gh, q0, q1, nullptr, t, G);
     for (int j = j0 + (int)threadIdx.x; j < j1; j += 256) {
       double s0 = 0, s1 = 0;
       for (long q = L.seg_off[j]; q < L.seg_off[j + 1]; ++q) {
@@ -647,11 +652,12 @@ __global__ void pow_init(long nlev, const int *node_of_col, const long *node_col
 
 // z = A q / s by row chunks and segments; the node's s from the partials of
 // ||q||^2.
-__global__ __launch_bounds__(256) void pow_rows_kernel(LevelRows L, const double *q, const double *part,
-                                                       const int *cb, double *z, double *seg_part) {
+__global__ __launch_bounds__(256) void pow_rows_kernel(LevelRows L, const double *q, const double *part, double *z,
+                                                       double *seg_part) {
   __shared__ double red[4], sig;
   __shared__ double sv[256];
-  __shared__ int list[256], cnt;
+  __shared__ long sb[256];
+  __shared__ int list[256], sn[256], cnt;
   const int *col = L.col;
   const float *val = L.val;
   auto one = [&](long b, long e, long S) { return dot1_range(b, e, S, col, val, q); };
@@ -663,13 +669,16 @@ __global__ __launch_bounds__(256) void pow_rows_kernel(LevelRows L, const double
     return;
   }
   const Chunk c = L.ch[(int)blockIdx.x - L.nseg];
+  PartSum<1> ps;
+  ps.load(part, c.q0, c.q1);
   bool is_long;
   auto few = [&](long b, long e) {
     double unused;
     return few_sum(b, e, col, val, [&](int i, double &) { return q[i]; }, &unused);
   };
-  const double s = chunk_row_sum<double>(L, c, few, one, [](double v) { return group_sum<16>(v); }, sv, list, &cnt, is_long);
-  node_norm(part, cb, c.node, &sig);
+  const double s = chunk_row_sum<double>(L, c, few, one, [](double v) { return group_sum<16>(v); }, sv, list, &cnt,
+                                          sb, sn, is_long);
+  node_norm(ps, part, c.q0, c.q1, &sig);
   const long r = c.b + threadIdx.x;
   if (r < c.e && !is_long) z[r] = s / sig;
 }
@@ -680,7 +689,10 @@ __global__ __launch_bounds__(256) void pow_long_kernel(LevelRows L, const double
   const int t = blockIdx.x;
   const int j0 = L.node_long0[t], j1 = L.node_long0[t + 1];
   if (j0 >= j1) return;
-  node_norm(part, cb, t, &sig);
+  PartSum<1> ps;
+  const int q0 = cb[t], q1 = cb[t + 1];
+  ps.load(part, q0, q1);
+  node_norm(ps, part, q0, q1, &sig);
   for (int j = j0 + (int)threadIdx.x; j < j1; j += 256) {
     double s = 0;
     for (long q = L.seg_off[j]; q < L.seg_off[j + 1]; ++q) s += seg_part[q];
@@ -721,7 +733,10 @@ __global__ void sumsq_chunks(const Chunk *ch, const double *x, double *part) {
 }
 
 __global__ void norm_finalize(const double *part, const int *cb, double *sig) {
-  node_norm(part, cb, blockIdx.x, sig + blockIdx.x);
+  PartSum<1> ps;
+  const int q0 = cb[blockIdx.x], q1 = cb[blockIdx.x + 1];
+  ps.load(part, q0, q1);
+  node_norm(ps, part, q0, q1, sig + blockIdx.x);
 }
 
 __global__ void fill_ones(double *x, int n) {
@@ -801,7 +816,7 @@ struct Engine {
   // level
   DBuf<long> perm, col_ptr, row_ptr, rstart, bsum, node_col0;
   DBuf<int> colmap, node_of_col, flag, row_node, row_orig, row_len, col_len, csr_col, csc_row,
-      cb_rows, cb_cols, cb_init, lflag, llist, node_long0, row0, csc2csr, ent, ent_s, rid_of_entry, lcnt, seg_row;
+      cb_rows, cb_cols, lflag, llist, node_long0, row0, csc2csr, ent, ent_s, rid_of_entry, lcnt, seg_row;
   DBuf<long> seg_off, seg_b;
   DBuf<double> seg_part;
   DBuf<unsigned> key, key_s;
@@ -819,7 +834,7 @@ struct Engine {
     bsum.release(); node_col0.release(); colmap.release(); node_of_col.release();
     flag.release(); row_node.release(); row_orig.release(); row_len.release();
     col_len.release(); csr_col.release(); csc_row.release(); cb_rows.release();
-    cb_cols.release(); cb_init.release(); lflag.release(); llist.release(); row0.release();
+    cb_cols.release(); lflag.release(); llist.release(); row0.release();
     csc2csr.release(); ent.release(); ent_s.release(); rid_of_entry.release(); key.release();
     key_s.release(); temp.release(); csr_val.release(); csc_val.release(); W.release();
     H.release(); part.release(); q.release(); z.release();
@@ -885,7 +900,7 @@ void make_chunks(const std::vector<long> &off, long chunk, std::vector<Chunk> &c
         }
         e = r;
       }
-      ch.push_back({(int)t, b, e});
+      ch.push_back({(int)t, 0, 0, b, e});
       b = e;
     }
   }
@@ -930,22 +945,6 @@ int planc_hiernmf_run(planc_ctx *ctx, const planc_hier_desc *desc, const long *h
     rc = (x);          \
     if (rc) return rc; \
   } while (0)
-  // CSC of A on the host (counting sort, rows ascending within a column).
-  std::vector<long> cptr(n + 1, 0);
-  for (long e = 0; e < nnz; ++e) cptr[h_indices[e] + 1]++;
-  for (long j = 0; j < n; ++j) cptr[j + 1] += cptr[j];
-  std::vector<int> ridx(nnz), c2r(nnz);
-  std::vector<float> cval(nnz);
-  {
-    std::vector<long> cur(cptr.begin(), cptr.end() - 1);
-    for (long i = 0; i < m; ++i)
-      for (long e = h_indptr[i]; e < h_indptr[i + 1]; ++e) {
-        long p = cur[h_indices[e]]++;
-        ridx[p] = (int)i;
-        cval[p] = h_data[e];
-        c2r[p] = (int)e;
-      }
-  }
   RC(E.rptr0.get(ctx, m + 1));
   RC(E.cptr0.get(ctx, n + 1));
   RC(E.cidx0.get(ctx, nnz));
@@ -965,16 +964,14 @@ int planc_hiernmf_run(planc_ctx *ctx, const planc_hier_desc *desc, const long *h
     return hipMemcpyAsync(d, h, b, hipMemcpyHostToDevice, ctx->stream);
   };
   PLANC_HIP_CHECK(ctx, up(E.rptr0.p, h_indptr, sizeof(long) * (m + 1)));
-  PLANC_HIP_CHECK(ctx, up(E.cptr0.p, cptr.data(), sizeof(long) * (n + 1)));
   if (nnz) {
     PLANC_HIP_CHECK(ctx, up(E.cidx0.p, h_indices, sizeof(int) * nnz));
-    PLANC_HIP_CHECK(ctx, up(E.ridx0.p, ridx.data(), sizeof(int) * nnz));
     PLANC_HIP_CHECK(ctx, up(E.val0.p, h_data, sizeof(float) * nnz));
-    PLANC_HIP_CHECK(ctx, up(E.cval0.p, cval.data(), sizeof(float) * nnz));
-    PLANC_HIP_CHECK(ctx, up(E.csc2csr.p, c2r.data(), sizeof(int) * nnz));
     entry_rows<<<nb(nnz), 256, 0, ctx->stream>>>(m, nnz, E.rptr0.p, E.row0.p);
     PLANC_LAUNCH_CHECK(ctx);
   }
+  // CSC of A (rows ascending within a column).
+  RC(csr_transpose(ctx, m, n, nnz, E.rptr0.p, E.cidx0.p, E.val0.p, E.cptr0.p, E.ridx0.p, E.cval0.p, E.csc2csr.p));
 
   // Tree state.
   struct HNode {
@@ -1122,6 +1119,14 @@ int planc_hiernmf_run(planc_ctx *ctx, const planc_hier_desc *desc, const long *h
     std::vector<int> cbr, cbc, cbi;
     make_chunks(roff, 256, chr, cbr, &hptr);
     make_chunks(noff, 256, chc, cbc);
+    for (Chunk &c : chr) {
+      c.q0 = cbc[c.node];
+      c.q1 = cbc[c.node + 1];
+    }
+    for (Chunk &c : chc) {
+      c.q0 = cbr[c.node];
+      c.q1 = cbr[c.node + 1];
+    }
     std::vector<long> ioff(nn + 1);
     for (int t = 0; t <= nn; ++t) ioff[t] = (long)t * m;
     make_chunks(ioff, 16384, chi, cbi);
@@ -1136,13 +1141,11 @@ int planc_hiernmf_run(planc_ctx *ctx, const planc_hier_desc *desc, const long *h
     RC(E.ch_init.get(ctx, chi.size()));
     RC(E.cb_rows.get(ctx, nn + 1));
     RC(E.cb_cols.get(ctx, nn + 1));
-    RC(E.cb_init.get(ctx, nn + 1));
     if (!chr.empty()) PLANC_HIP_CHECK(ctx, up(E.ch_rows.p, chr.data(), sizeof(Chunk) * chr.size()));
     if (!chc.empty()) PLANC_HIP_CHECK(ctx, up(E.ch_cols.p, chc.data(), sizeof(Chunk) * chc.size()));
     PLANC_HIP_CHECK(ctx, up(E.ch_init.p, chi.data(), sizeof(Chunk) * chi.size()));
     PLANC_HIP_CHECK(ctx, up(E.cb_rows.p, cbr.data(), sizeof(int) * (nn + 1)));
     PLANC_HIP_CHECK(ctx, up(E.cb_cols.p, cbc.data(), sizeof(int) * (nn + 1)));
-    PLANC_HIP_CHECK(ctx, up(E.cb_init.p, cbi.data(), sizeof(int) * (nn + 1)));
     RC(E.part.get(ctx, 3 * std::max(chr.size(), chi.size()) + 3));
     RC(E.part_h.get(ctx, 3 * chc.size() + 3));
     RC(E.extra.get(ctx, 3 * nn));
@@ -1164,8 +1167,7 @@ int planc_hiernmf_run(planc_ctx *ctx, const planc_hier_desc *desc, const long *h
       sumsq_chunks<<<col_blocks, 256, 0, ctx->stream>>>(E.ch_cols.p, E.q.p, E.part_h.p);
       for (int it = 0; it < iters; ++it) {
         if (row_blocks)
-          pow_rows_kernel<<<row_blocks, 256, 0, ctx->stream>>>(rows, E.q.p, E.part_h.p, E.cb_cols.p, E.z.p,
-                                                               E.seg_part.p);
+          pow_rows_kernel<<<row_blocks, 256, 0, ctx->stream>>>(rows, E.q.p, E.part_h.p, E.z.p, E.seg_part.p);
         if (nlong)
           pow_long_kernel<<<(unsigned)nn, 256, 0, ctx->stream>>>(rows, E.seg_part.p, E.part_h.p, E.cb_cols.p, E.z.p);
         pow_cols_kernel<<<col_blocks, 256, 0, ctx->stream>>>(E.ch_cols.p, E.col_ptr.p, E.csc_row.p, E.csc_val.p,
@@ -1197,16 +1199,17 @@ int planc_hiernmf_run(planc_ctx *ctx, const planc_hier_desc *desc, const long *h
                                                             m, E.W.p, E.H.p);
     init_gram_chunks<<<(unsigned)chi.size(), 256, 0, ctx->stream>>>(E.ch_init.p, E.seeds.p, m, E.part.p);
     PLANC_LAUNCH_CHECK(ctx);
-    const GramParts gh = {E.part_h.p, E.cb_cols.p, nullptr};
+    const int init_chunks = cbi[1] - cbi[0];
     for (int it = 0; it < iters; ++it) {
       // W^T W: over all m rows of the initial W first, then over the rows kept.
-      const GramParts gw = {E.part.p, it == 0 ? E.cb_init.p : E.cb_rows.p, it > 0 && nlong ? E.extra.p : nullptr};
-      h_gram_kernel<<<col_blocks, 256, 0, ctx->stream>>>(E.ch_cols.p, E.col_ptr.p, E.csc_row.p, E.csc_val.p, E.W.p, gw,
-                                                         E.H.p, E.part_h.p);
+      h_gram_kernel<<<col_blocks, 256, 0, ctx->stream>>>(E.ch_cols.p, E.col_ptr.p, E.csc_row.p, E.csc_val.p, E.W.p,
+                                                         E.part.p, it > 0 && nlong ? E.extra.p : nullptr,
+                                                         it == 0 ? init_chunks : 0, E.H.p, E.part_h.p);
       if (row_blocks)
-        w_rows_kernel<<<row_blocks, 256, 0, ctx->stream>>>(rows, E.H.p, gh, E.W.p, E.part.p, E.seg_part.p);
+        w_rows_kernel<<<row_blocks, 256, 0, ctx->stream>>>(rows, E.H.p, E.part_h.p, E.W.p, E.part.p, E.seg_part.p);
       if (nlong)
-        w_long_kernel<<<(unsigned)nn, 256, 0, ctx->stream>>>(rows, E.seg_part.p, gh, E.W.p, E.extra.p);
+        w_long_kernel<<<(unsigned)nn, 256, 0, ctx->stream>>>(rows, E.seg_part.p, E.part_h.p, E.cb_cols.p, E.W.p,
+                                                             E.extra.p);
     }
     PLANC_LAUNCH_CHECK(ctx);
     // Split rule H(:,0) >= H(:,1), larger side to the left child

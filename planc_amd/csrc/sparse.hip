@@ -50,12 +50,14 @@ __global__ void iota_kernel(long n, int *v) {
 // column changes (each thread writes those of the columns that begin at its
 // entry, empty ones among them; the last entry's thread the ones behind it).
 __global__ void csr_t_gather_kernel(long nnz, long n, const int *ent, const unsigned *key, const int *rowid,
-                                    const float *values, int *out_indices, float *out_values, long *out_indptr) {
+                                    const float *values, int *out_indices, float *out_values, long *out_indptr,
+                                    int *out_entries) {
   long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= nnz) return;
   const int e = ent[p];
   out_indices[p] = rowid[e];
   out_values[p] = values[e];
+  if (out_entries) out_entries[p] = e;
   const long c = key[p];
   for (long q = p > 0 ? (long)key[p - 1] + 1 : 0; q <= c; ++q) out_indptr[q] = p;
   if (p == nnz - 1)
@@ -281,7 +283,7 @@ __global__ void sparse_fit_finalize_kernel(const double *part, int nb, const dou
 // Stable transpose of a CSR matrix (m x n) into the CSR of its transpose
 // (n x m): entries grouped by column, rows increasing within a column.
 int csr_transpose(planc_ctx *ctx, long m, long n, long nnz, const long *indptr, const int *indices,
-                  const float *values, long *out_indptr, int *out_indices, float *out_values) {
+                  const float *values, long *out_indptr, int *out_indices, float *out_values, int *out_entries) {
   if (nnz >= (1L << 31) || n >= (1L << 31) || m >= (1L << 31))
     return set_error(ctx, PLANC_EUNSUPPORTED, "csr_transpose: at most 2^31-1 rows, columns and entries");
   if (nnz == 0) {
@@ -310,7 +312,8 @@ int csr_transpose(planc_ctx *ctx, long m, long n, long nnz, const long *indptr, 
   PLANC_HIP_CHECK(ctx, hipcub::DeviceRadixSort::SortPairs(temp, bytes, keys, keys_s, ent, ent_s, (int)nnz, 0,
                                                           bits, ctx->stream));
   csr_t_gather_kernel<<<(unsigned)((nnz + 255) / 256), 256, 0, ctx->stream>>>(nnz, n, ent_s, keys_s, rowid, values,
-                                                                              out_indices, out_values, out_indptr);
+                                                                              out_indices, out_values, out_indptr,
+                                                                              out_entries);
   PLANC_LAUNCH_CHECK(ctx);
   return PLANC_OK;
 }
