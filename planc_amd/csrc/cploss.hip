@@ -17,6 +17,7 @@
 #include <string>
 
 #include "common.h"
+#include "wave.h"
 
 namespace planc {
 
@@ -185,8 +186,7 @@ __global__ __launch_bounds__(FWD_THR) void cp_loss_fwd_kernel(CPParams p) {
     }
   }
   // Block reduction (fixed order).
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) acc2 += __shfl_xor(acc2, off, 64);
+  acc2 = wave_sum(acc2);
   if (lane == 0) red[wave] = acc2;
   __syncthreads();
   if (tid == 0) {
@@ -210,8 +210,7 @@ __global__ __launch_bounds__(256) void sum_half_kernel(const double *part, long 
     for (int u = 0; u < 8; ++u) t += v[u];
   }
   for (; b < n; b += 256) t += part[b];
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+  t = wave_sum(t);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = t;
   __syncthreads();
   if (threadIdx.x == 0) *out = 0.5 * (red[0] + red[1] + red[2] + red[3]);

@@ -40,6 +40,7 @@
 
 #include "common.h"
 #include "philox.h"
+#include "wave.h"
 
 // After common.h: hipCUB picks its backend from the platform macro that
 // hip_runtime.h defines.
@@ -186,12 +187,9 @@ struct Chunk {
 
 // Sums over a block of 256 threads (valid in thread 0), fixed order.
 __device__ inline void block_sum3(double &s0, double &s1, double &s2, double (*red)[4]) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    s0 += __shfl_xor(s0, off, 64);
-    s1 += __shfl_xor(s1, off, 64);
-    s2 += __shfl_xor(s2, off, 64);
-  }
+  s0 = wave_sum(s0);
+  s1 = wave_sum(s1);
+  s2 = wave_sum(s2);
   const int w = threadIdx.x >> 6;
   if ((threadIdx.x & 63) == 0) {
     red[0][w] = s0;
@@ -225,18 +223,14 @@ struct PartSum {
     if (q1 - q0 <= FEW_CHUNKS) {
       for (int j = 0; j < q1 - q0; ++j)
 #pragma unroll
-        for (int q = 0; q < Q; ++q) s[q] += __shfl(v[q], j, 64);
+        for (int q = 0; q < Q; ++q) s[q] += lane_value(v[q], j);
       return;
     }
     for (int j = q0 + 64 + (int)threadIdx.x; j < q1; j += 64)
 #pragma unroll
       for (int q = 0; q < Q; ++q) v[q] += part[(long)Q * j + q];
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1)
-#pragma unroll
-      for (int q = 0; q < Q; ++q) v[q] += __shfl_xor(v[q], off, 64);
-#pragma unroll
-    for (int q = 0; q < Q; ++q) s[q] = v[q];
+    for (int q = 0; q < Q; ++q) s[q] = wave_sum(v[q]);
   }
 };
 
@@ -284,12 +278,9 @@ __global__ void init_gram_chunks(const Chunk *ch, const unsigned long long *seed
     s01 += x0 * x1;
     s11 += x1 * x1;
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    s00 += __shfl_xor(s00, off, 64);
-    s01 += __shfl_xor(s01, off, 64);
-    s11 += __shfl_xor(s11, off, 64);
-  }
+  s00 = wave_sum(s00);
+  s01 = wave_sum(s01);
+  s11 = wave_sum(s11);
   int w = threadIdx.x >> 6;
   if ((threadIdx.x & 63) == 0) {
     red[0][w] = s00;
@@ -405,16 +396,8 @@ __global__ __launch_bounds__(256) void h_gram_kernel(const Chunk *ch, const long
   }
 }
 
-template <int G>
-__device__ inline double group_sum(double v) {
-#pragma unroll
-  for (int off = G / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, G);
-  return v;
-}
-
 __device__ inline double block_sum256(double v, double *red) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  v = wave_sum(v);
   __syncthreads();
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
@@ -444,7 +427,7 @@ struct LevelRows {
 };
 
 // The sums of a short row by one thread, all its gathers in flight: the products
-// rounded and added as 16 lanes with one entry each would add them (group_sum),
+// rounded and added as 16 lanes with one entry each would add them (row_sum),
 // so that a row's sum does not depend on which of the two took it and sums that
 // cancel in a degenerate node (a singular Gram) keep doing so exactly.
 template <class Load>
@@ -556,8 +539,8 @@ __global__ __launch_bounds__(256) void w_rows_kernel(LevelRows L, const double *
   const Pair p = chunk_row_sum<Pair>(
       L, c, few, one,
       [](Pair q) {
-        q.a = group_sum<16>(q.a);
-        q.b = group_sum<16>(q.b);
+        q.a = row_sum(q.a);
+        q.b = row_sum(q.b);
         return q;
       },
       sv, list, &cnt, sb, sn, is_long);
@@ -676,7 +659,7 @@ __global__ __launch_bounds__(256) void pow_rows_kernel(LevelRows L, const double
     double unused;
     return few_sum(b, e, col, val, [&](int i, double &) { return q[i]; }, &unused);
   };
-  const double s = chunk_row_sum<double>(L, c, few, one, [](double v) { return group_sum<16>(v); }, sv, list, &cnt,
+  const double s = chunk_row_sum<double>(L, c, few, one, [](double v) { return row_sum(v); }, sv, list, &cnt,
                                           sb, sn, is_long);
   node_norm(ps, part, c.q0, c.q1, &sig);
   const long r = c.b + threadIdx.x;
@@ -721,8 +704,7 @@ __global__ void sumsq_chunks(const Chunk *ch, const double *x, double *part) {
   Chunk c = ch[blockIdx.x];
   double s = 0;
   for (long r = c.b + threadIdx.x; r < c.e; r += blockDim.x) s += x[r] * x[r];
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+  s = wave_sum(s);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
   __syncthreads();
   if (threadIdx.x == 0) {

@@ -7,6 +7,7 @@
 // write of the factor plus one read of the numerator.
 #include "common.h"
 #include "rowupd.h"
+#include "wave.h"
 
 namespace planc {
 
@@ -14,13 +15,7 @@ namespace {
 
 constexpr int NTHR = 256;
 
-__device__ inline double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
-
-// Deterministic block sum (fixed shuffle pattern, waves summed in order).
+// Deterministic block sum (fixed lane pattern, waves summed in order).
 __device__ inline double block_sum(double v, double *red) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   v = wave_sum(v);

@@ -3,18 +3,13 @@
 // of the CP relative error.
 #include "common.h"
 #include "rowupd.h"
+#include "wave.h"
 
 namespace planc {
 
 namespace {
 
 constexpr int NTHR = 256;
-
-__device__ inline double wave_sum_d(double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
 
 struct ContractParams {
   const float *P;  // E x k, column-major (ld ldp); E = prod d[0..nb)
@@ -147,7 +142,7 @@ __global__ __launch_bounds__(256) void contract_wave_kernel(ContractParams p) {
 #pragma unroll
   for (int r = 0; r < CW_OUT; ++r) {
     const long i = i0 + 4 * r;
-    const double t = wave_sum_d((double)acc[r]);
+    const double t = wave_sum((double)acc[r]);
     if (lane == 0 && i < p.In) p.M[c + p.ldo * i] = (float)t;
   }
 }
@@ -186,7 +181,7 @@ __global__ __launch_bounds__(256) void contract_inner_kernel(ContractParams p) {
   }
 #pragma unroll
   for (int t = 0; t < TI; ++t) {
-    double v = wave_sum_d((double)acc[t]);
+    double v = wave_sum((double)acc[t]);
     if (lane == 0) red[t][wave] = v;
   }
   __syncthreads();
@@ -226,7 +221,7 @@ __global__ __launch_bounds__(NTHR) void lambda_dot_partial_kernel(const float *F
     int c = (int)(e / I);
     s += lambda[c] * (double)F[i + ldf * c] * (double)M[c + ldm * i];
   }
-  s = wave_sum_d(s);
+  s = wave_sum(s);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (lane == 0) red[wave] = s;
   __syncthreads();
@@ -244,7 +239,7 @@ __global__ void ntf_relerr_kernel(const double *normX2, const double *part, long
   if (threadIdx.x >= 64) return;
   double t = 0.0;
   for (long b = threadIdx.x; b < nparts; b += 64) t += part[b];
-  t = wave_sum_d(t);
+  t = wave_sum(t);
   double xh = 0.0;
   for (int e = threadIdx.x; e < k * k; e += 64) {
     int a = e % k, b = e / k;
@@ -252,7 +247,7 @@ __global__ void ntf_relerr_kernel(const double *normX2, const double *part, long
     for (int i = 0; i < gs.n; ++i) v *= gs.g[i][e];
     xh += v;
   }
-  xh = wave_sum_d(xh);
+  xh = wave_sum(xh);
   if (threadIdx.x == 0) {
     double e2 = *normX2 - 2.0 * t + xh;
     if (e2 < 0) e2 = 0;
@@ -572,8 +567,8 @@ __global__ __launch_bounds__(4 * MRT *(NVB > 0 ? NVB : 1)) void mode_rows_kernel
         const int a = e % KM, b = e / KM;
         if (e < KM * KM && a < k && b < k) xh += Gu[a + k * b] * dS[it];
       }
-      t1 = wave_sum_d(t1);
-      xh = wave_sum_d(xh);
+      t1 = wave_sum(t1);
+      xh = wave_sum(xh);
       if (lane == 0) {
         red[0][tid >> 6] = t1;
         red[1][tid >> 6] = xh;
@@ -654,8 +649,8 @@ __global__ __launch_bounds__(256) void mode_finalize_kernel(ModeParams p, int nb
       if (g < p.ng && g != p.skip) v *= p.g[g][e];
     xh += v;
   }
-  t1 = wave_sum_d(t1);
-  xh = wave_sum_d(xh);
+  t1 = wave_sum(t1);
+  xh = wave_sum(xh);
   __syncthreads();
   if (lane == 0) red[wave] = t1;
   __syncthreads();

@@ -23,6 +23,7 @@
 #include <algorithm>
 
 #include "common.h"
+#include "wave.h"
 
 // After common.h: hipCUB picks its backend from the platform macro that
 // hip_runtime.h defines.
@@ -243,8 +244,7 @@ __global__ __launch_bounds__(256) void sparse_fit_kernel(long m, const long *ind
     for (long e = indptr[r]; e < indptr[r + 1]; ++e) {
       const int j = indices[e];
       double t = lane < k ? w * (double)Hk[(long)j * k + lane] : 0.0;
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+      t = wave_sum(t);
       const double d = (double)values[e] - t;
       sse += d * d;  // identical in every lane
       wh2 += t * t;
