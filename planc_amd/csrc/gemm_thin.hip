@@ -1868,15 +1868,39 @@ std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K,
   const long ksteps = (K + step - 1) / step;
   const int esz = dtype == PLANC_F32 ? 4 : 2;
   const double abytes = (double)L * (double)K * esz;
-  // K splits: the partial tiles' round trip may be 10% of A's bytes, or 8 MB
-  // (they stay in L2) where A is small and one pass of its few groups leaves
+  // K splits: the partial tiles' round trip may be 10% of A's bytes (20% for
+  // FP32, whose products are bound by MFMA as much as by reading and gain more
+  // from an even grid), or 8 MB (they stay in L2) where A is small and one pass of its few groups leaves
   // most CUs idle; each wave keeps 8 k steps, 2 there (2000 x 1000, k = 20:
   // 37 and 21 us products with one split of 32 waves).
   const bool small = abytes <= (double)(64L << 20);
   const long min_steps = small ? 2 : 8;
+  const double share = dtype == PLANC_F32 ? 0.20 : 0.10;
   auto partials_fit = [&](const Geometry &g, double share) {
     const double b = 2.0 * g.nsplit * g.groups * g.tile_bytes;
     return b <= share * abytes || (small && b <= (double)(8L << 20));
+  };
+  // Split counts tried for a grid of bx blocks: powers of two, and those that
+  // make it 1, 2, 3 or 4 blocks per CU where no power of two comes within 8%
+  // below such a whole number (96^4: 36 and 72 blocks a split; 16 splits of 36
+  // leave a quarter of the SIMDs idle in the last round).
+  auto split_counts = [&](long bx) {
+    std::vector<long> out;
+    for (long ns = 1; ns <= 4096; ns *= 2) out.push_back(ns);
+    const long cu = ctx->num_cu;
+    bool even = false;
+    for (long ns = 1; ns <= 4096 && bx * ns <= 4 * cu; ns *= 2) {
+      const long b = bx * ns, up = (b + cu - 1) / cu * cu;
+      even = even || (b >= cu / 2 && b * 100 >= up * 92);
+    }
+    if (!even)
+      for (long t = 1; t <= 4; ++t) {
+        const long ns = t * cu / bx;
+        if (ns > 1 && (ns & (ns - 1)) != 0) out.push_back(ns);
+      }
+    std::sort(out.begin(), out.end());
+    out.erase(std::unique(out.begin(), out.end()), out.end());
+    return out;
   };
   if (!trans && dtype != PLANC_F32) {
     // Streaming 16-bit NN: one k phase, K splits only; per-wave or
@@ -1890,7 +1914,7 @@ std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K,
       for (long ns = 1; ns <= 4096; ns *= 2) {
         Geometry g = make_geometry(L, K, trans, dtype, NT, 1, 1, ns, 0, sh);
         if (ns > 1 && (g.nsplit < ns || ksteps / g.nsplit < min_steps)) break;
-        if (ns > 1 && !partials_fit(g, 0.10)) break;
+        if (ns > 1 && !partials_fit(g, share)) break;
         const long waves = g.blocks_x * 4 * g.nsplit;
         if (ns > 1 && waves > 16L * 1024) break;
         if (!out.empty() && waves < 2L * ctx->num_cu && ns < 4096) {
@@ -1936,10 +1960,12 @@ std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K,
   for (int cw : cws)
     for (int wk = 1; wk <= 4; wk *= 2) {
       if (wk > 1 && ksteps < 8L * wk * (dual ? 2 : 1)) break;
-      for (long ns = 1; ns <= 4096; ns *= 2) {
+      for (long ns : split_counts(make_geometry(L, K, trans, dtype, NT, cw, wk, 1, dual).blocks_x)) {
         Geometry g = make_geometry(L, K, trans, dtype, NT, cw, wk, ns, dual);
-        if (ns > 1 && (g.nsplit < ns || ksteps / ((long)g.nsplit * wk * (dual ? 2 : 1)) < min_steps)) break;
-        if (ns > 1 && !partials_fit(g, 0.10)) break;
+        const bool p2 = (ns & (ns - 1)) == 0;
+        if (ns > 1 && ((p2 && g.nsplit < ns) || ksteps / ((long)g.nsplit * wk * (dual ? 2 : 1)) < min_steps)) break;
+        if (!p2 && g.nsplit < ns - ns / 8) continue;
+        if (ns > 1 && !partials_fit(g, share)) break;
         const long waves = g.blocks_x * 4 * g.nsplit;
         if (ns > 1 && waves > 16L * 1024) break;
         if (waves < 2L * ctx->num_cu && ns < 4096) continue;  // too few waves: try more splits
@@ -1952,10 +1978,12 @@ std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K,
     for (int cw : scws) {
       const int sstep = dtype == PLANC_F32 ? 16 : 64;
       const long sk = (K + sstep - 1) / sstep;
-      for (long ns = 1; ns <= 4096; ns *= 2) {
+      for (long ns : split_counts(make_geometry(L, K, trans, dtype, NT, cw, 1, 1, 1, 1).blocks_x)) {
         Geometry g = make_geometry(L, K, trans, dtype, NT, cw, 1, ns, 1, 1);
-        if (ns > 1 && (g.nsplit < ns || sk / g.nsplit < min_steps)) break;
-        if (ns > 1 && !partials_fit(g, 0.10)) break;
+        const bool p2 = (ns & (ns - 1)) == 0;
+        if (ns > 1 && ((p2 && g.nsplit < ns) || sk / g.nsplit < min_steps)) break;
+        if (!p2 && g.nsplit < ns - ns / 8) continue;
+        if (ns > 1 && !partials_fit(g, share)) break;
         const long waves = g.blocks_x * 4 * g.nsplit;
         if (ns > 1 && waves > 16L * 1024) break;
         if (waves < 2L * ctx->num_cu && ns < 4096) continue;
@@ -2206,14 +2234,17 @@ int pick_geometry(planc_ctx *ctx, int dtype, int trans, int NT, int tm, const St
         sel.push_back(g);
     if (!sel.empty()) cands.swap(sel);
   }
-  // FP32 operands off the 16-byte grid: chains of at most 1024 k per
-  // accumulator where the candidates have them (one 4986-k chain per row of a
-  // 20011 x 9973 product was 12% faster than sixteen of 623, and left NMF-HALS
-  // factors five times as far from FP64 as those did).
+  // FP32 operands off the 16-byte grid: accumulator chains of at most 1024 k,
+  // and an eighth of K where that is shorter (never under 256), if the
+  // candidates have them.  One 4986-k chain per row of a 20011 x 9973 product
+  // was 12% faster than sixteen of 623 and left NMF-HALS factors five times as
+  // far from FP64 (256 everywhere: 11% slower for 1.4e-5 instead of 1.9e-5); on
+  // a 61 x 53 x 47 x 35 tensor chains of 822 left 6.6e-6 where 205 leave 3.0e-6.
   if (dtype == PLANC_F32 && (p.lda % 4 != 0 || (uintptr_t)p.A % 16 != 0)) {
+    const long limit = std::min(1024L, std::max(256L, p.K / 8));
     std::vector<Geometry> sel;
     for (const Geometry &g : cands)
-      if (g.kchunk <= 1024L * g.wk) sel.push_back(g);
+      if (g.kchunk <= limit * g.wk) sel.push_back(g);
     if (!sel.empty()) cands.swap(sel);
   }
   const char *env = getenv("PLANC_AUTOTUNE");
