@@ -231,8 +231,9 @@ __global__ __launch_bounds__(NTHR) void gram_reduce_set_kernel(GramIn in, int k,
 // contracts with is one contiguous row of 16-byte words (uniform address:
 // one LDS broadcast per word for the whole wave).  NTH = blockDim.x: every
 // thread's loads are issued before the first store (one memory round trip).
-template <int KM, int NTH>
-__device__ inline void load_gram(float (&Gt)[KM][KM], const double *G, int k) {
+// With a pitch of 2 KM each row is stored twice over.
+template <int KM, int NTH, int PITCH>
+__device__ inline void load_gram(float (&Gt)[KM][PITCH], const double *G, int k) {
   constexpr int PER = (KM * KM + NTH - 1) / NTH;
   double v[PER];
 #pragma unroll
@@ -243,24 +244,26 @@ __device__ inline void load_gram(float (&Gt)[KM][KM], const double *G, int k) {
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
     const int e = threadIdx.x + NTH * j;
-    if (e < KM * KM) Gt[e / KM][e % KM] = (float)v[j];
+    if (e < KM * KM) {
+      Gt[e / KM][e % KM] = (float)v[j];
+      if constexpr (PITCH == 2 * KM) Gt[e / KM][e % KM + KM] = (float)v[j];
+    }
   }
   __syncthreads();
 }
 
 // s + sum_t h[t] * G(t, x), in t order, from the transposed LDS tile.
+// h . g over KM values of a 16-byte aligned g in LDS, in four chains.
 template <int KM>
-__device__ inline float dot_gcol(const float (&h)[KM], const float (&Gt)[KM][KM], int x, float s) {
-  const floatx4 *g = (const floatx4 *)&Gt[x][0];
+__device__ inline float dot_turned(const float (&h)[KM], const float *g) {
+  floatx4 c = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
   for (int q = 0; q < KM / 4; ++q) {
-    const floatx4 v = g[q];
-    s = fmaf(h[4 * q + 0], v[0], s);
-    s = fmaf(h[4 * q + 1], v[1], s);
-    s = fmaf(h[4 * q + 2], v[2], s);
-    s = fmaf(h[4 * q + 3], v[3], s);
+    const floatx4 v = *(const floatx4 *)(g + 4 * q);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) c[j] = fmaf(h[4 * q + j], v[j], c[j]);
   }
-  return s;
+  return (c[0] + c[1]) + (c[2] + c[3]);
 }
 
 // MU (kind 0: H <- H .* N ./ (H*G + eps)) and HALS rows (kind 1,
@@ -569,24 +572,52 @@ __global__ __launch_bounds__(NTHR * RG) void rows_gram_kernel(float *H, long n, 
 }
 
 // Column-sum exchange of a cooperative launch (all blocks co-resident).
-// Every slot of a column starts as PART_EMPTY (set before the launch); thread
-// 0 of each block writes its partial into its own slot with an agent-scope
-// atomic store.  Wave 0 of every block polls the column's slots with
-// agent-scope atomic loads until none is empty, summing the values of the
-// same poll in a fixed order (identical in every block): the partials
-// travel with the readiness test, one round trip after the last store.  The
-// wait is bounded: on time-out *err is set, later exchanges return at once
-// and the caller reports the failure.
+// Every slot of a column starts as PART_EMPTY (set before the launch); each
+// block writes its partial into its own slot of all EX_COPIES copies with one
+// agent-scope atomic store instruction (publish).  Wave 0 of every block polls
+// one copy's slots with agent-scope atomic loads until none is empty, summing
+// the values of the same poll in a fixed order (identical in every block): the
+// partials travel with the readiness test, one round trip after the last store
+// (collect).  What a block does between the two is hidden in that round trip.
+// The copies keep the polls of many blocks off the lines that others still
+// store to: an exchange of 79 blocks takes 2.42 us with one copy, 1.71 with
+// four, 1.59 with eight, 1.65 with sixteen; of 40 blocks 2.06 and 1.29 (8).
+// The wait is bounded: on time-out *err is set, later exchanges return at once
+// and the caller reports the failure.  LDS is taken in turns (column parity), so
+// a column costs one barrier in each half: the barrier of the other half lies
+// between the last read of a buffer and its next write.
 constexpr unsigned long long PART_EMPTY = ~0ull;  // a NaN no arithmetic produces (all payload bits set)
 
-__device__ inline bool column_exchange(double bs, double *part_col, int *err, double &total) {
-  __shared__ int s_ok;
-  __shared__ double s_tot;
-  unsigned long long *slot = reinterpret_cast<unsigned long long *>(part_col);
-  if (threadIdx.x == 0)
-    __hip_atomic_store(&slot[blockIdx.x], __builtin_bit_cast(unsigned long long, bs), __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
+constexpr int EX_COPIES = 8;
+__host__ __device__ inline long exchange_pitch(long nb) { return (nb + 15) / 16 * 16; }  // whole 128-byte lines
+
+template <int NW>
+struct Exchange {
+  double red[2][NW];
+  double tot[2];
+  int ok[2];
+};
+
+template <int NW>
+__device__ inline void column_publish(Exchange<NW> &ex, int par, double lsum, double *part_col) {
+  lsum = wave_sum(lsum);
+  if ((threadIdx.x & 63) == 0) ex.red[par][threadIdx.x >> 6] = lsum;
+  __syncthreads();
+  if (threadIdx.x < EX_COPIES) {
+    double bs = 0.0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) bs += ex.red[par][w];
+    __hip_atomic_store(reinterpret_cast<unsigned long long *>(part_col) + threadIdx.x * exchange_pitch(gridDim.x) +
+                           blockIdx.x,
+                       __builtin_bit_cast(unsigned long long, bs), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+template <int NW>
+__device__ inline bool column_collect(Exchange<NW> &ex, int par, const double *part_col, int *err, double &total) {
   if (threadIdx.x < 64) {
+    const unsigned long long *slot = reinterpret_cast<const unsigned long long *>(part_col) +
+                                     blockIdx.x % EX_COPIES * exchange_pitch(gridDim.x);
     const int nb = (int)gridDim.x, lane = (int)threadIdx.x;
     int ok = 1;
     double tot = 0.0;
@@ -602,24 +633,23 @@ __device__ inline bool column_exchange(double bs, double *part_col, int *err, do
         tot = t;
         break;
       }
-      if (spin >= (1 << 20) || __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
+      // The flag's load would add its latency to every poll: one in sixteen.
+      if (spin >= (1 << 20) ||
+          ((spin & 15) == 15 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
         if (lane == 0) __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         ok = 0;
         break;
       }
-      __builtin_amdgcn_s_sleep(1);
     }
     tot = wave_sum(tot);
     if (lane == 0) {
-      s_ok = ok;
-      s_tot = tot;
+      ex.ok[par] = ok;
+      ex.tot[par] = tot;
     }
   }
   __syncthreads();
-  total = s_tot;
-  const bool ok = s_ok != 0;
-  __syncthreads();
-  return ok;
+  total = ex.tot[par];
+  return ex.ok[par] != 0;
 }
 
 __global__ void zero_int_kernel(int *p) { *p = 0; }
@@ -630,18 +660,32 @@ __global__ void fill_u64_kernel(unsigned long long *p, long n, unsigned long lon
 
 // HALS over the columns of W with per-column normalisation (nmf/hals.hpp:
 // 89-102).  Persistent cooperative kernel: each thread owns RPT rows of W in
-// registers; one column_exchange per column x publishes the column's sum of
-// squares (block partials summed in the same order by every block, so every
-// block derives the identical norm).  part: k x gridDim.x slots, PART_EMPTY
-// at launch; sync[1] the time-out flag.
-// BS: threads per block; 1024-thread blocks make four times fewer exchange
-// participants.
+// registers; one exchange per column x gives the column's sum of squares
+// (block partials summed in the same order by every block, so every block
+// derives the identical norm).  Bound by that exchange: k round trips between
+// the XCDs, one after the other.  So column x + 1's dot product over all
+// columns but x, which is most of the arithmetic, is formed between publish
+// and collect, and the new column x joins it with one multiply-add.
+// Registers are indexed statically: the column loop is unrolled by four, and
+// after each group the row turns by four places, w[r][t] holding column
+// (x0 + t) mod KM; each Gram column is in LDS twice over, so that the turned
+// row meets it at one offset.  (Selects over a row at a dynamic x took longer
+// than the exchange.)
+// part: k x EX_COPIES x exchange_pitch(gridDim.x) slots, PART_EMPTY at launch;
+// sync[1] the time-out flag.  BS: threads per block; larger blocks make fewer
+// exchange participants.  20011 rows, k = 50: 223 -> 97 us; a call for 20011 x
+// 16 99.5 -> 75.6 us, 65536 x 64 385 -> 167, 600000 x 8 133 -> 118.
+// Wavefronts per SIMD that 256-thread blocks are compiled for: they set how many
+// rows one launch can hold.
+constexpr int coop_waves(int KM, int RPT) {
+  return RPT == 1 ? (KM <= 16 ? 7 : KM <= 32 ? 5 : KM <= 48 ? 4 : 3) : KM <= 16 ? 5 : KM <= 32 ? 3 : 2;
+}
 template <int KM, int RPT, int BS>
-__global__ __launch_bounds__(BS) void hals_cols_coop_kernel(float *W, long m, int k, long ldw,
+__global__ __launch_bounds__(BS, BS > 256 ? BS / 256 : coop_waves(KM, RPT)) void hals_cols_coop_kernel(float *W, long m, int k, long ldw,
                                                             const float *AH, long ldah,
                                                             const double *G, double *part, int *sync) {
-  __shared__ __attribute__((aligned(16))) float Gs[KM][KM];
-  __shared__ double red[BS / 64];
+  __shared__ __attribute__((aligned(16))) float Gs[KM][2 * KM];
+  __shared__ Exchange<BS / 64> ex;
   load_gram<KM, BS>(Gs, G, k);
   const long total = (long)gridDim.x * blockDim.x;
   const long gtid = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -653,50 +697,67 @@ __global__ __launch_bounds__(BS) void hals_cols_coop_kernel(float *W, long m, in
 #pragma unroll
     for (int t = 0; t < KM; ++t) w[r][t] = (i < m && t < k) ? W[i + ldw * t] : 0.0f;
   }
-  // AH(i, x) of the next column is loaded one column ahead, so its latency
-  // hides behind the current column's barrier instead of stalling the
-  // column update.
-  float ahn[RPT];
+  // s: the row's dot with G's column x; ah = AH(i, x), loaded a column ahead,
+  // so its latency hides behind the exchange.
+  float s[RPT], ah[RPT];
 #pragma unroll
   for (int r = 0; r < RPT; ++r) {
     long i = gtid + r * total;
-    ahn[r] = i < m ? AH[i] : 0.0f;
+    ah[r] = i < m ? AH[i] : 0.0f;
+    s[r] = dot_turned<KM>(w[r], &Gs[0][0]);
   }
-  // The column loop is not unrolled (it holds a grid barrier); registers are
-  // only indexed by the unrolled t loops, w[r][x] is read and written through
-  // selects.
-  for (int x = 0; x < k; ++x) {
-    float u[RPT];
-    double lsum = 0.0;
-    const float gxx = Gs[x][x];
+  int x0 = 0;
+#pragma unroll 1
+  for (;; x0 += 4) {
 #pragma unroll
-    for (int r = 0; r < RPT; ++r) {
-      long i = gtid + r * total;
-      u[r] = 0.0f;
-      float wx = 0.0f;
-#pragma unroll
-      for (int t = 0; t < KM; ++t) wx = (t == x) ? w[r][t] : wx;
-      const float s = dot_gcol<KM>(w[r], Gs, x, 0.0f);
-      const float ax = ahn[r];
-      if (i < m && x + 1 < k) ahn[r] = AH[i + ldah * (x + 1)];
-      if (i < m) {
-        float v = (wx * gxx) + (ax - s);
-        v = (v < floor_v) ? floor_v : v;
-        u[r] = v;
-        lsum += (double)v * (double)v;
-      }
-    }
-    double bs = block_sum(lsum, red);
-    double tot = 0.0;
-    if (!column_exchange(bs, part + (size_t)x * gridDim.x, sync + 1, tot)) return;
-    double nrm = sqrt(tot);
-    if (nrm != 0.0) {
+    for (int j = 0; j < 4; ++j) {
+      const int x = x0 + j;
+      if (x >= k) break;
+      float u[RPT], old[RPT];
+      double lsum = 0.0;
+      const float gxx = Gs[x][x];
 #pragma unroll
       for (int r = 0; r < RPT; ++r) {
-        float nv = (float)((double)u[r] / nrm);
-#pragma unroll
-        for (int t = 0; t < KM; ++t) w[r][t] = (t == x) ? nv : w[r][t];
+        long i = gtid + r * total;
+        u[r] = 0.0f;
+        old[r] = w[r][j];
+        if (i < m) {
+          float v = (w[r][j] * gxx) + (ah[r] - s[r]);
+          v = (v < floor_v) ? floor_v : v;
+          u[r] = v;
+          lsum += (double)v * (double)v;
+        }
       }
+      double *col = part + (size_t)x * EX_COPIES * exchange_pitch(gridDim.x);
+      column_publish(ex, j & 1, lsum, col);
+      const int xn = x + 1 < k ? x + 1 : x;
+      const float gn = Gs[xn][x];
+#pragma unroll
+      for (int r = 0; r < RPT; ++r) {
+        long i = gtid + r * total;
+        if (i < m && x + 1 < k) ah[r] = AH[i + ldah * (x + 1)];
+        w[r][j] = 0.0f;
+        s[r] = dot_turned<KM>(w[r], &Gs[xn][x0]);
+      }
+      double tot = 0.0;
+      if (!column_collect(ex, j & 1, col, sync + 1, tot)) return;
+      const double inv = rsqrt(tot);
+#pragma unroll
+      for (int r = 0; r < RPT; ++r) {
+        w[r][j] = tot != 0.0 ? (float)((double)u[r] * inv) : old[r];
+        s[r] = fmaf(w[r][j], gn, s[r]);
+      }
+    }
+    if (x0 + 4 >= k) break;
+#pragma unroll
+    for (int r = 0; r < RPT; ++r) {
+      float head[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) head[t] = w[r][t];
+#pragma unroll
+      for (int t = 0; t < KM - 4; ++t) w[r][t] = w[r][t + 4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) w[r][KM - 4 + t] = head[t];
     }
   }
 #pragma unroll
@@ -704,8 +765,10 @@ __global__ __launch_bounds__(BS) void hals_cols_coop_kernel(float *W, long m, in
     long i = gtid + r * total;
     if (i < m) {
 #pragma unroll
-      for (int t = 0; t < KM; ++t)
-        if (t < k) W[i + ldw * t] = w[r][t];
+      for (int t = 0; t < KM; ++t) {
+        const int c = (x0 + t) % KM;
+        if (c < k) W[i + ldw * c] = w[r][t];
+      }
     }
   }
 }
@@ -1208,10 +1271,10 @@ int try_coop(planc_ctx *ctx, float *W, long m, int k, long ldw, const float *AH,
   long need = (m + (long)BS * RPT - 1) / ((long)BS * RPT);
   if (need > maxblocks || need <= 0) return PLANC_OK;
   unsigned nb = (unsigned)need;
-  double *part = (double *)ws_get(ctx, 2, sizeof(double) * (size_t)KM * nb);
+  const long nslots = (long)k * EX_COPIES * exchange_pitch(nb);
+  double *part = (double *)ws_get(ctx, 2, sizeof(double) * (size_t)nslots);
   int *sync = (int *)ws_get(ctx, 17, 2 * sizeof(int));
   if (!part || !sync) return set_error(ctx, PLANC_ENOMEM, "hals_cols: workspace");
-  const long nslots = (long)k * nb;
   fill_u64_kernel<<<(unsigned)((nslots + 255) / 256), 256, 0, ctx->stream>>>((unsigned long long *)part, nslots,
                                                                              PART_EMPTY);
   PLANC_LAUNCH_CHECK(ctx);
@@ -1234,7 +1297,13 @@ int hals_cols_impl(planc_ctx *ctx, float *W, long m, int k, long ldw, const floa
                    const double *G) {
   bool done = false;
   int rc = PLANC_OK;
-  if constexpr (KM <= 48) {  // at k = 64 a 1024-thread block leaves too few registers per row
+  // The widest block first that has the registers (k > 32 at 1024 threads is
+  // tight, k > 48 impossible): fewest participants.
+  if constexpr (KM > 32) {
+    rc = try_coop<KM, 1, 512>(ctx, W, m, k, ldw, AH, ldah, G, &done);
+    if (rc || done) return rc;
+  }
+  if constexpr (KM <= 48) {
     rc = try_coop<KM, 1, 1024>(ctx, W, m, k, ldw, AH, ldah, G, &done);
     if (rc || done) return rc;
   }
