@@ -1870,9 +1870,10 @@ std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K,
   const double abytes = (double)L * (double)K * esz;
   // K splits: the partial tiles' round trip may be 10% of A's bytes (20% for
   // FP32, whose products are bound by MFMA as much as by reading and gain more
-  // from an even grid), or 8 MB (they stay in L2) where A is small and one pass of its few groups leaves
-  // most CUs idle; each wave keeps 8 k steps, 2 there (2000 x 1000, k = 20:
-  // 37 and 21 us products with one split of 32 waves).
+  // from an even grid: 96^4, k = 48 TN 104 -> 90 us), or 8 MB (they stay in L2)
+  // where A is small and one pass of its few groups leaves most CUs idle; each
+  // wave keeps 8 k steps, 2 there (2000 x 1000, k = 20: 37 and 21 us products
+  // with one split of 32 waves).
   const bool small = abytes <= (double)(64L << 20);
   const long min_steps = small ? 2 : 8;
   const double share = dtype == PLANC_F32 ? 0.20 : 0.10;
@@ -2234,17 +2235,16 @@ int pick_geometry(planc_ctx *ctx, int dtype, int trans, int NT, int tm, const St
         sel.push_back(g);
     if (!sel.empty()) cands.swap(sel);
   }
-  // FP32 operands off the 16-byte grid: accumulator chains of at most 1024 k,
-  // and an eighth of K where that is shorter (never under 256), if the
-  // candidates have them.  One 4986-k chain per row of a 20011 x 9973 product
-  // was 12% faster than sixteen of 623 and left NMF-HALS factors five times as
-  // far from FP64 (256 everywhere: 11% slower for 1.4e-5 instead of 1.9e-5); on
-  // a 61 x 53 x 47 x 35 tensor chains of 822 left 6.6e-6 where 205 leave 3.0e-6.
+  // FP32 operands off the 16-byte grid: accumulator chains of at most 1024 k
+  // where the candidates have them.  One 4986-k chain per row of a 20011 x 9973
+  // product was 12% faster than sixteen of 623 and left NMF-HALS factors five
+  // times as far from FP64; 256 was 11% slower than 1024 and no closer.  (On a
+  // 61 x 53 x 47 x 35 tensor 64, 128 and 1024 leave NTF-BPP factors 4.1, 3.6 and
+  // 3.9e-6 from FP64, means over 32 starts: not the chains' error.)
   if (dtype == PLANC_F32 && (p.lda % 4 != 0 || (uintptr_t)p.A % 16 != 0)) {
-    const long limit = std::min(1024L, std::max(256L, p.K / 8));
     std::vector<Geometry> sel;
     for (const Geometry &g : cands)
-      if (g.kchunk <= limit * g.wk) sel.push_back(g);
+      if (g.kchunk <= 1024L * g.wk) sel.push_back(g);
     if (!sel.empty()) cands.swap(sel);
   }
   const char *env = getenv("PLANC_AUTOTUNE");
