@@ -31,7 +31,7 @@
 // microseconds.  Complete tree of 9 levels, 50000 x 200000, 1.9 M entries, 100
 // iterations: eight launches an iteration, with 16 lanes on every row, took
 // 97 us (41 of them the row kernel) and the power iteration 51 us; these take
-// 46 (22) and 33 us.
+// 41 (20) and 31 us.
 #include <algorithm>
 #include <cstring>
 #include <map>

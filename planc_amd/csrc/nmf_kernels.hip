@@ -673,7 +673,7 @@ __global__ void fill_u64_kernel(unsigned long long *p, long n, unsigned long lon
 // than the exchange.)
 // part: k x EX_COPIES x exchange_pitch(gridDim.x) slots, PART_EMPTY at launch;
 // sync[1] the time-out flag.  BS: threads per block; larger blocks make fewer
-// exchange participants.  20011 rows, k = 50: 223 -> 97 us; a call for 20011 x
+// exchange participants.  20011 rows, k = 50: 223 -> 84 us; a call for 20011 x
 // 16 99.5 -> 75.6 us, 65536 x 64 385 -> 167, 600000 x 8 133 -> 118.
 // Wavefronts per SIMD that 256-thread blocks are compiled for: they set how many
 // rows one launch can hold.
