@@ -1861,8 +1861,11 @@ Geometry make_geometry(long L, long K, int trans, int dtype, int NT, int cw, int
 // partial traffic stays under 10% of A, every wave keeps at least 8 k steps
 // and the grid stays under 16k waves.  The first entry is the static choice
 // used when tuning is off or impossible (graph capture).
+// krp: the thin operand is a Khatri-Rao product (written out or not).
+constexpr long KRP_ONE_CHAIN = 512;  // rows of an FP32 contraction that is not split
+
 std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K, int trans, int dtype,
-                                           int NT, bool shared_ok, bool f32dual_ok, bool fly_ok = false) {
+                                           int NT, bool shared_ok, bool f32dual_ok, bool fly_ok, bool krp) {
   std::vector<Geometry> out;
   const int step = dtype == PLANC_F32 ? 16 : 32;
   const long ksteps = (K + step - 1) / step;
@@ -1877,7 +1880,15 @@ std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K,
   const bool small = abytes <= (double)(64L << 20);
   const long min_steps = small ? 2 : 8;
   const double share = dtype == PLANC_F32 ? 0.20 : 0.10;
+  // A tensor contraction in FP32 over at most KRP_ONE_CHAIN rows is summed in one
+  // chain, whatever the operand's form: these are the smallest calls, where a
+  // split gains nothing (NTF-HALS 20 x 18 x 16, K = 288: 261 us whole, 258 in nine
+  // pieces), and HALS sweeps carry a change of the order of these sums into the
+  // factors (there over 24 starts 4.1e-6 from FP64 on average whole, 1.8e-6 in
+  // pieces, but a single start up to 1.2 times as far, of 20 x 16 x 16 2.8 times).
+  const bool whole = krp && dtype == PLANC_F32 && K <= KRP_ONE_CHAIN;
   auto partials_fit = [&](const Geometry &g, double share) {
+    if (whole) return g.nsplit == 1;
     const double b = 2.0 * g.nsplit * g.groups * g.tile_bytes;
     return b <= share * abytes || (small && b <= (double)(8L << 20));
   };
@@ -2206,7 +2217,7 @@ bool stream_capturing(hipStream_t st) {
 // the other 16-bit candidates read: it runs before the first candidate is
 // timed, and with fly_ok it is timed too and its time charged to every
 // candidate that needs it.
-int pick_geometry(planc_ctx *ctx, int dtype, int trans, int NT, int tm, const StreamParams &p, bool fly_ok,
+int pick_geometry(planc_ctx *ctx, int dtype, int trans, int NT, int tm, const StreamParams &p, bool krp, bool fly_ok,
                   const std::function<int()> &pack, Geometry *out) {
   // PLANC_STREAM_VARIANT restricts the tuner to one kernel family (used to
   // test each path): "plain" (per-wave thin operand, 16/32-k steps), "dual"
@@ -2217,7 +2228,7 @@ int pick_geometry(planc_ctx *ctx, int dtype, int trans, int NT, int tm, const St
   const std::string vs = venv ? venv : "";
   const int smode = vs == "plain" ? 0 : (vs == "shared" ? 1 : (vs == "dual" ? 3 : (vs == "fly" ? 4 : 2)));
   const std::vector<long> key = {dtype, trans, NT, tm, p.L, p.K, p.lda, p.th.k, p.cmajor, smode, p.np,
-                                 fly_ok ? 1 : 0};
+                                 fly_ok ? 1 : 0, krp ? 1 : 0};
   for (const auto &e : ctx->gemm_tuned)
     if (e.first == key) {
       const auto &v = e.second;
@@ -2226,7 +2237,7 @@ int pick_geometry(planc_ctx *ctx, int dtype, int trans, int NT, int tm, const St
     }
   const bool shared_ok = (dtype != PLANC_F32 || tm != THIN_SAFE) && smode != 0 && smode != 3;
   std::vector<Geometry> cands = candidate_geometries(ctx, p.L, p.K, trans, dtype, NT, shared_ok,
-                                                     dtype == PLANC_F32 && tm != THIN_SAFE, fly_ok && shared_ok);
+                                                     dtype == PLANC_F32 && tm != THIN_SAFE, fly_ok && shared_ok, krp);
   if (smode != 2) {
     std::vector<Geometry> sel;
     for (const Geometry &g : cands)
@@ -2508,7 +2519,7 @@ int thin_gemm(planc_ctx *ctx, int dtype, int trans, const void *A, long lda, lon
     if (splits_hint > 0) {
       g = make_geometry(L, K, trans, dtype, NT, trans && dtype == PLANC_F32 ? 2 : 4, 1, splits_hint);
     } else {
-      rc = pick_geometry(ctx, dtype, trans, NT, tm, p, fly_ok, pack, &g);
+      rc = pick_geometry(ctx, dtype, trans, NT, tm, p, krp && krp->nf > 0, fly_ok, pack, &g);
       if (rc) return rc;
     }
     if (!packed && !(g.shared == 2 && !trans && dtype != PLANC_F32)) {
