@@ -15,7 +15,7 @@
 //    smaller of the passive and the complementary system (at most k / 2
 //    variables).  Taken where G's 1-norm condition is at most BPP_COND.
 //  * the passive system itself, for any other G and for columns the pair gives
-//    up.
+//    up (more than 5 k steps, or H b not finite).
 // Bound by FP64 arithmetic and the lane broadcasts of the elimination (two
 // v_readlane per FMA).  One ANLS-BPP iteration at 65536 x 16384, k = 64 (81920
 // columns, BF16 products): 70.8 ms with a masked elimination of all k columns
@@ -275,6 +275,12 @@ __global__ __launch_bounds__(512) void bpp_kernel(const double *G, const double 
     if (!PAIR && usable && iters[col] >= 0) continue;
     const double b = live ? (double)B[col * b_cs + lane * b_rs] : 0.0;
     const double c = PAIR ? times(Hs, b) : 0.0;
+    // H spreads an entry that is no finite number over the whole column; the
+    // passive systems meet it only where its variable is passive.
+    if (PAIR && ballot64(live && !isfinite(c))) {
+      if (lane == 0) iters[col] = -1;
+      continue;
+    }
     double bb = b, cc = c;  // right-hand side of the current solve and H times it
     double x = 0.0, y = -b, xbase = 0.0;
     Exchange ex(k);

@@ -54,3 +54,27 @@ def test_bpp_pair_matches_oracle(ctx, k, nrhs, kind):
     tol = 2e-7 + (2.2e-16 * np.linalg.cond(G) if kind == "ill" else 0.0)
     err = np.abs(X - Xr).max(0) / np.maximum(np.abs(Xr).max(0), 1e-30)
     assert err.max() <= tol, (err.max(), tol)
+
+
+@pytest.mark.parametrize("bad", [float("nan"), -float("inf")])
+@pytest.mark.parametrize("k,nrhs", [(8, 70), (24, 70), (33, 9001), (64, 1030)])
+def test_bpp_entries_that_are_no_finite_number(ctx, k, nrhs, bad):
+    """A right-hand side entry of NaN or -inf is never below zero in y = G x - b,
+    so its variable stays 0 and the others solve the system without it; the
+    columns beside it are what they are alone.  (These columns are the ones that
+    the kernel of the pair leaves to the general one, 9001 of them more than
+    one pass of its grid.)"""
+    print("bpp not finite", k, nrhs, bad, flush=True)
+    G, B = problem(k, nrhs, "plain")
+    X0 = ctx.bpp(P.colmajor(G), P.colmajor(B)).cpu().numpy()
+    i, cols = k // 3, np.arange(nrhs) % 3 == 1
+    Bad = B.copy(order="F")
+    Bad[i, cols] = bad
+    X = ctx.bpp(P.colmajor(G), P.colmajor(Bad)).cpu().numpy()
+    assert np.array_equal(X[:, ~cols], X0[:, ~cols])
+    rest = np.arange(k) != i
+    Xr, it = O.bppnnls(np.asfortranarray(G[np.ix_(rest, rest)]), np.asfortranarray(B[np.ix_(rest, cols)].astype(np.float64)))
+    assert it >= 0
+    assert not X[i, cols].any()
+    err = np.abs(X[np.ix_(rest, cols)] - Xr).max(0) / np.maximum(np.abs(Xr).max(0), 1e-30)
+    assert err.max() <= 2e-7, err.max()
