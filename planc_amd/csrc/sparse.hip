@@ -77,6 +77,7 @@ __global__ void csr_t_gather_kernel(long nnz, long n, const int *ent, const unsi
 
 constexpr int SP_SHORT = 64;
 constexpr int SP_SEG = 512;
+constexpr int SP_WIDE = SP_SEG;
 
 // A piece of a row longer than SP_SHORT: entries part * SP_SEG .. of row
 // `row`; with nseg > 1 its sums go to partial row pslot, the row's pieces in
@@ -116,9 +117,12 @@ __device__ inline void spmm_store4(float *out, long r, int c, int k, long ors, l
 // out(r, c) at out[r * ors + c * ocs], F k-major (element (j, c) at F[j * ldf
 // + c], ldf a multiple of 4).  G lanes (4 G >= k) hold an output row, four
 // columns each.  PLAN: blocks below nsegb walk the pieces, the others the short
-// rows.  Without a plan (nsegb 0: a single product whose entry count the host
-// does not know) a block walks the long ones among its rows afterwards, its
-// four wavefronts together.
+// rows.  Without a plan (a single product whose entry count the host does not
+// know) the first nsegb blocks take four rows at a time: a row of more than SP_SHORT
+// entries is walked by a wavefront, one of more than SP_WIDE by the block's four
+// together.  k = 16, 10000 rows of 100 entries: 14 us, of 1000: 58 (67 and 189
+// where the long ones among a block's rows were walked one after the other by all
+// four, 46 and 417 with a wavefront per row and an entry at a time).
 template <int G, bool PLAN>
 __global__ __launch_bounds__(256) void spmm_kernel(long rows, const long *indptr, const int *indices,
                                                    const float *values, const float *F, long ldf, int k, float *out,
@@ -175,25 +179,40 @@ __global__ __launch_bounds__(256) void spmm_kernel(long rows, const long *indptr
       walk(b, e, 1);
       spmm_store4(out, r, 4 * gl, k, ors, ocs, acc);
     }
-    if constexpr (!PLAN) {
-      __shared__ int nlong, lrow[256 / G];
-      __shared__ floatx4 red[4][G];
-      if (threadIdx.x == 0) nlong = 0;
-      __syncthreads();
-      if (is_long && gl == 0) lrow[atomicAdd(&nlong, 1)] = (int)r;
-      __syncthreads();
-      const int wave = threadIdx.x >> 6;
-      for (int i = 0; i < nlong; ++i) {
-        const long lr = lrow[i];
+    return;
+  }
+  if constexpr (!PLAN) {
+    __shared__ floatx4 red[4][G];
+    const int wave = threadIdx.x >> 6;
+    auto add_groups = [&]() {
+#pragma unroll
+      for (int off = G; off < 64; off <<= 1)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[q] += __shfl_xor(acc[q], off, 64);
+    };
+    for (long r0 = 4L * blockIdx.x; r0 < rows; r0 += 4L * nsegb) {
+      long b[5];
+#pragma unroll
+      for (int i = 0; i < 5; ++i) b[i] = indptr[min(r0 + i, rows)];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const long len = b[i + 1] - b[i];
+        if (len <= SP_WIDE) {
+          if (wave == i && len > SP_SHORT) {
+            acc = floatx4{0.f, 0.f, 0.f, 0.f};
+            walk(b[i] + grp, b[i + 1], NG);
+            add_groups();
+            if (grp == 0) spmm_store4(out, r0 + i, 4 * gl, k, ors, ocs, acc);
+          }
+          continue;
+        }
         acc = floatx4{0.f, 0.f, 0.f, 0.f};
-        walk(indptr[lr] + wave * NG + grp, indptr[lr + 1], 4 * NG);
-#pragma unroll
-        for (int off = G; off < 64; off <<= 1)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) acc[q] += __shfl_xor(acc[q], off, 64);
+        walk(b[i] + wave * NG + grp, b[i + 1], 4 * NG);
+        add_groups();
         if (grp == 0) red[wave][gl] = acc;
         __syncthreads();
-        if (threadIdx.x < G) spmm_store4(out, lr, 4 * gl, k, ors, ocs, (red[0][gl] + red[1][gl]) + (red[2][gl] + red[3][gl]));
+        if (threadIdx.x < G)
+          spmm_store4(out, r0 + i, 4 * gl, k, ors, ocs, (red[0][gl] + red[1][gl]) + (red[2][gl] + red[3][gl]));
         __syncthreads();
       }
     }
@@ -351,8 +370,10 @@ template <int G>
 static int spmm_launch(planc_ctx *ctx, const SpmmPlan &pl, long rows, const long *indptr, const int *indices,
                        const float *values, const float *F, long ldf, int k, float *out, long ors, long ocs) {
   if (!pl.cnt) {
-    spmm_kernel<G, false><<<(unsigned)((rows + 256 / G - 1) / (256 / G)), 256, 0, ctx->stream>>>(
-        rows, indptr, indices, values, F, ldf, k, out, ors, ocs, 0, nullptr, nullptr, nullptr);
+    const int nsegb = (int)std::min<long>((rows + 3) / 4, 1L << 20);
+    const long nb = nsegb + (rows + 256 / G - 1) / (256 / G);
+    spmm_kernel<G, false><<<(unsigned)nb, 256, 0, ctx->stream>>>(rows, indptr, indices, values, F, ldf, k, out, ors, ocs,
+                                                                nsegb, nullptr, nullptr, nullptr);
     PLANC_LAUNCH_CHECK(ctx);
     return PLANC_OK;
   }

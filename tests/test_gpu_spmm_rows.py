@@ -82,6 +82,25 @@ def elapsed(f, reps):
     return best
 
 
+@pytest.mark.parametrize("k", [8, 16])
+def test_spmm_long_rows_run_side_by_side(ctx, k):
+    """Rows just past the short class take no more than twice the time of rows
+    just inside it (10000 rows of 66 and of 64 entries): a wavefront each, not one
+    after the other in a block."""
+    g = torch.Generator(device="cuda").manual_seed(k)
+    F = torch.rand((k, 5000), generator=g, device="cuda").t()
+
+    def run(per):
+        print("spmm rows of", per, k, flush=True)
+        indptr = torch.arange(10001, device="cuda", dtype=torch.int64) * per
+        idx = torch.randint(0, 5000, (10000 * per,), generator=g, device="cuda", dtype=torch.int32)
+        val = torch.rand(10000 * per, generator=g, device="cuda")
+        return elapsed(lambda: ctx.spmm(10000, 5000, indptr, idx, val, F), 50)
+
+    short, long = run(64), run(66)
+    assert long <= 2 * short, (short, long)
+
+
 @pytest.mark.parametrize("where", ["first", "last", "spread", "none"])
 def test_transpose_with_empty_columns(ctx, where):
     """Row pointers of the transpose over long runs of empty columns: right, and
