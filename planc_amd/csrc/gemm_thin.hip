@@ -1857,15 +1857,17 @@ Geometry make_geometry(long L, long K, int trans, int dtype, int NT, int cw, int
   return g;
 }
 
+constexpr long KRP_ONE_CHAIN = 512;  // rows of an FP32 tensor contraction that is not split
+constexpr long MAX_CHAIN = 1024;     // rows that one accumulator takes of an FP32 operand off the 16-byte grid
+
 // Candidate geometries: every (cw, wk) with K splits 1, 2, 4, ... while the
 // partial traffic stays under 10% of A, every wave keeps at least 8 k steps
 // and the grid stays under 16k waves.  The first entry is the static choice
 // used when tuning is off or impossible (graph capture).
 // krp: the thin operand is a Khatri-Rao product (written out or not).
-constexpr long KRP_ONE_CHAIN = 512;  // rows of an FP32 contraction that is not split
-
 std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K, int trans, int dtype,
-                                           int NT, bool shared_ok, bool f32dual_ok, bool fly_ok, bool krp) {
+                                           int NT, bool shared_ok, bool f32dual_ok, bool fly_ok, bool krp,
+                                           bool off_grid) {
   std::vector<Geometry> out;
   const int step = dtype == PLANC_F32 ? 16 : 32;
   const long ksteps = (K + step - 1) / step;
@@ -1887,18 +1889,36 @@ std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K,
   // factors (there over 24 starts 4.1e-6 from FP64 on average whole, 1.8e-6 in
   // pieces, but a single start up to 1.2 times as far, of 20 x 16 x 16 2.8 times).
   const bool whole = krp && dtype == PLANC_F32 && K <= KRP_ONE_CHAIN;
+  // off_grid (an FP32 A whose columns do not all begin on 16 bytes): accumulators
+  // take at most MAX_CHAIN rows of K each.  Every candidate has the splits that
+  // this needs (4096 at most; their partials are up to 2 k / MAX_CHAIN, 12%, of A's
+  // bytes), the bounds below hold for further ones.  The element-wise kernels that
+  // such operands took before had chains of a few hundred rows; one of 4986 per row
+  // of a 20011 x 9973 product was 12% faster than sixteen of 623 and left NMF-HALS
+  // factors five times as far from FP64 (256 was 11% slower than 1024 and no
+  // closer).  Operands on the grid have always been read in chains as long as is
+  // fastest, and the limit would cost them up to a third: 32768 x 16384, k = 32, NN
+  // 348 -> 405 us and TN 371 -> 492; 30000 x 16000, k = 64, both 525 -> 580.  It
+  // would bring NMF-HALS of 20012 x 9976 from 5.3e-5 to 1.6e-5 (8.3e-5 before the
+  // uneven split counts below); an odd leading dimension has that effect.
+  auto least_splits = [&](int st, int wk) -> long {
+    if (!off_grid) return 1;
+    const long most = MAX_CHAIN * wk / st, steps = (K + st - 1) / st;
+    return std::clamp((steps + most - 1) / most, 1L, 4096L);
+  };
   auto partials_fit = [&](const Geometry &g, double share) {
     if (whole) return g.nsplit == 1;
     const double b = 2.0 * g.nsplit * g.groups * g.tile_bytes;
     return b <= share * abytes || (small && b <= (double)(8L << 20));
   };
-  // Split counts tried for a grid of bx blocks: powers of two, and those that
+  // Split counts tried for a grid of bx blocks: least, powers of two, and those that
   // make it 1, 2, 3 or 4 blocks per CU where no power of two comes within 8%
   // below such a whole number (96^4: 36 and 72 blocks a split; 16 splits of 36
   // leave a quarter of the SIMDs idle in the last round).
-  auto split_counts = [&](long bx) {
-    std::vector<long> out;
-    for (long ns = 1; ns <= 4096; ns *= 2) out.push_back(ns);
+  auto split_counts = [&](long bx, long least) {
+    std::vector<long> out = {least};
+    for (long ns = 1; ns <= 4096; ns *= 2)
+      if (ns > least) out.push_back(ns);
     const long cu = ctx->num_cu;
     bool even = false;
     for (long ns = 1; ns <= 4096 && bx * ns <= 4 * cu; ns *= 2) {
@@ -1908,7 +1928,7 @@ std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K,
     if (!even)
       for (long t = 1; t <= 4; ++t) {
         const long ns = t * cu / bx;
-        if (ns > 1 && (ns & (ns - 1)) != 0) out.push_back(ns);
+        if (ns > least && (ns & (ns - 1)) != 0) out.push_back(ns);
       }
     std::sort(out.begin(), out.end());
     out.erase(std::unique(out.begin(), out.end()), out.end());
@@ -1957,7 +1977,8 @@ std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K,
       wk *= 2;
       g = make_geometry(L, K, trans, dtype, NT, cw, wk, 1);
     }
-    long ns = 1;
+    long ns = least_splits(step, wk);
+    g = make_geometry(L, K, trans, dtype, NT, cw, wk, ns);
     while (g.blocks_x * 4 * ns < 4L * ctx->num_cu) {
       Geometry h = make_geometry(L, K, trans, dtype, NT, cw, wk, ns * 2);
       if (!partials_fit(h, 0.06) || ksteps / ((long)h.nsplit * wk) < min_steps) break;
@@ -1972,14 +1993,15 @@ std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K,
   for (int cw : cws)
     for (int wk = 1; wk <= 4; wk *= 2) {
       if (wk > 1 && ksteps < 8L * wk * (dual ? 2 : 1)) break;
-      for (long ns : split_counts(make_geometry(L, K, trans, dtype, NT, cw, wk, 1, dual).blocks_x)) {
+      const long least = least_splits(dtype == PLANC_F32 && dual ? 32 : step, wk);
+      for (long ns : split_counts(make_geometry(L, K, trans, dtype, NT, cw, wk, 1, dual).blocks_x, least)) {
         Geometry g = make_geometry(L, K, trans, dtype, NT, cw, wk, ns, dual);
-        const bool p2 = (ns & (ns - 1)) == 0;
-        if (ns > 1 && ((p2 && g.nsplit < ns) || ksteps / ((long)g.nsplit * wk * (dual ? 2 : 1)) < min_steps)) break;
-        if (!p2 && g.nsplit < ns - ns / 8) continue;
-        if (ns > 1 && !partials_fit(g, share)) break;
+        const bool p2 = (ns & (ns - 1)) == 0, more = ns > least;
+        if (more && ((p2 && g.nsplit < ns) || ksteps / ((long)g.nsplit * wk * (dual ? 2 : 1)) < min_steps)) break;
+        if (more && !p2 && g.nsplit < ns - ns / 8) continue;
+        if (more && !partials_fit(g, share)) break;
         const long waves = g.blocks_x * 4 * g.nsplit;
-        if (ns > 1 && waves > 16L * 1024) break;
+        if (more && waves > 16L * 1024) break;
         if (waves < 2L * ctx->num_cu && ns < 4096) continue;  // too few waves: try more splits
         out.push_back(g);
       }
@@ -1990,14 +2012,15 @@ std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K,
     for (int cw : scws) {
       const int sstep = dtype == PLANC_F32 ? 16 : 64;
       const long sk = (K + sstep - 1) / sstep;
-      for (long ns : split_counts(make_geometry(L, K, trans, dtype, NT, cw, 1, 1, 1, 1).blocks_x)) {
+      const long least = least_splits(sstep, 1);
+      for (long ns : split_counts(make_geometry(L, K, trans, dtype, NT, cw, 1, 1, 1, 1).blocks_x, least)) {
         Geometry g = make_geometry(L, K, trans, dtype, NT, cw, 1, ns, 1, 1);
-        const bool p2 = (ns & (ns - 1)) == 0;
-        if (ns > 1 && ((p2 && g.nsplit < ns) || sk / g.nsplit < min_steps)) break;
-        if (!p2 && g.nsplit < ns - ns / 8) continue;
-        if (ns > 1 && !partials_fit(g, share)) break;
+        const bool p2 = (ns & (ns - 1)) == 0, more = ns > least;
+        if (more && ((p2 && g.nsplit < ns) || sk / g.nsplit < min_steps)) break;
+        if (more && !p2 && g.nsplit < ns - ns / 8) continue;
+        if (more && !partials_fit(g, share)) break;
         const long waves = g.blocks_x * 4 * g.nsplit;
-        if (ns > 1 && waves > 16L * 1024) break;
+        if (more && waves > 16L * 1024) break;
         if (waves < 2L * ctx->num_cu && ns < 4096) continue;
         out.push_back(g);
       }
@@ -2227,8 +2250,9 @@ int pick_geometry(planc_ctx *ctx, int dtype, int trans, int NT, int tm, const St
   const char *venv = getenv("PLANC_STREAM_VARIANT");
   const std::string vs = venv ? venv : "";
   const int smode = vs == "plain" ? 0 : (vs == "shared" ? 1 : (vs == "dual" ? 3 : (vs == "fly" ? 4 : 2)));
+  const bool off_grid = dtype == PLANC_F32 && (p.lda % 4 != 0 || (uintptr_t)p.A % 16 != 0);
   const std::vector<long> key = {dtype, trans, NT, tm, p.L, p.K, p.lda, p.th.k, p.cmajor, smode, p.np,
-                                 fly_ok ? 1 : 0, krp ? 1 : 0};
+                                 fly_ok ? 1 : 0, krp ? 1 : 0, off_grid ? 1 : 0};
   for (const auto &e : ctx->gemm_tuned)
     if (e.first == key) {
       const auto &v = e.second;
@@ -2237,25 +2261,14 @@ int pick_geometry(planc_ctx *ctx, int dtype, int trans, int NT, int tm, const St
     }
   const bool shared_ok = (dtype != PLANC_F32 || tm != THIN_SAFE) && smode != 0 && smode != 3;
   std::vector<Geometry> cands = candidate_geometries(ctx, p.L, p.K, trans, dtype, NT, shared_ok,
-                                                     dtype == PLANC_F32 && tm != THIN_SAFE, fly_ok && shared_ok, krp);
+                                                     dtype == PLANC_F32 && tm != THIN_SAFE, fly_ok && shared_ok, krp,
+                                                     off_grid);
   if (smode != 2) {
     std::vector<Geometry> sel;
     for (const Geometry &g : cands)
       if (smode == 4 ? g.shared == 2
                      : smode == 1 ? g.shared != 0 : (g.shared == 0 && (smode == 3) == (g.dual != 0)))
         sel.push_back(g);
-    if (!sel.empty()) cands.swap(sel);
-  }
-  // FP32 operands off the 16-byte grid: accumulator chains of at most 1024 k
-  // where the candidates have them.  One 4986-k chain per row of a 20011 x 9973
-  // product was 12% faster than sixteen of 623 and left NMF-HALS factors five
-  // times as far from FP64; 256 was 11% slower than 1024 and no closer.  (On a
-  // 61 x 53 x 47 x 35 tensor 64, 128 and 1024 leave NTF-BPP factors 4.1, 3.6 and
-  // 3.9e-6 from FP64, means over 32 starts: not the chains' error.)
-  if (dtype == PLANC_F32 && (p.lda % 4 != 0 || (uintptr_t)p.A % 16 != 0)) {
-    std::vector<Geometry> sel;
-    for (const Geometry &g : cands)
-      if (g.kchunk <= 1024L * g.wk) sel.push_back(g);
     if (!sel.empty()) cands.swap(sel);
   }
   const char *env = getenv("PLANC_AUTOTUNE");
