@@ -15,10 +15,19 @@ int set_error(planc_ctx *ctx, int code, const std::string &msg) {
   return code;
 }
 
+bool stream_capturing(hipStream_t st) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &cs) != hipSuccess) return true;
+  return cs != hipStreamCaptureStatusNone;
+}
+
 void *ws_get(planc_ctx *ctx, int slot, size_t bytes) {
   Workspace &w = ctx->ws[slot];
   if (bytes == 0) bytes = 256;
   if (w.bytes >= bytes) return w.ptr;
+  // PLANC_WS_MAX (bytes) refuses larger buffers, as a device without the room would.
+  const char *most = getenv("PLANC_WS_MAX");
+  if (most && bytes > strtoull(most, nullptr, 10)) return nullptr;
   if (w.ptr) {
     // Queued kernels may still read the old buffer.
     if (hipStreamSynchronize(ctx->stream) != hipSuccess) return nullptr;
@@ -28,11 +37,17 @@ void *ws_get(planc_ctx *ctx, int slot, size_t bytes) {
   }
   size_t b = bytes + bytes / 8;
   if (hipMalloc(&w.ptr, b) != hipSuccess) {
+    (void)hipGetLastError();  // the caller may go on without the buffer
     w.ptr = nullptr;
     return nullptr;
   }
   w.bytes = b;
   return w.ptr;
+}
+
+void *ws_try(planc_ctx *ctx, int slot, size_t bytes) {
+  if (ctx->ws[slot].bytes < bytes && stream_capturing(ctx->stream)) return nullptr;
+  return ws_get(ctx, slot, bytes);
 }
 
 // Dimension-tree split: the s in [0, N-2] minimising the larger of the two

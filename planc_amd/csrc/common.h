@@ -128,6 +128,10 @@ namespace planc {
 // 35 NES iterates, 36 NES factors (centres, previous, accelerated), 37 NES
 // lambdas.
 void *ws_get(planc_ctx *ctx, int slot, size_t bytes);
+// For buffers that the caller can do without: null too where the stream is being
+// captured and the slot would have to grow.
+void *ws_try(planc_ctx *ctx, int slot, size_t bytes);
+bool stream_capturing(hipStream_t st);
 
 // Scoped choice of ctx->thin_planes (restored on exit).
 struct ThinPlanes {

@@ -2143,7 +2143,7 @@ int launch_stream(planc_ctx *ctx, int dtype, int trans, int NT, int tm, StreamPa
   // Partial tiles are indexed by padded group (blocks_x * wgrp >= groups).
   const long gpad = g.blocks_x * g.wgrp;
   if (g.nsplit > 1) {
-    p.part = (float *)ws_get(ctx, 0, (size_t)g.nsplit * gpad * g.tile_bytes);
+    p.part = (float *)ws_try(ctx, 0, (size_t)g.nsplit * gpad * g.tile_bytes);
     if (!p.part) return set_error(ctx, PLANC_ENOMEM, "thin_gemm: workspace");
   }
   dim3 grid((unsigned)g.blocks_x, (unsigned)g.nsplit);
@@ -2224,12 +2224,6 @@ int launch_stream(planc_ctx *ctx, int dtype, int trans, int NT, int tm, StreamPa
   return PLANC_OK;
 }
 
-bool stream_capturing(hipStream_t st) {
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(st, &cs) != hipSuccess) return true;
-  return cs != hipStreamCaptureStatusNone;
-}
-
 // Picks the geometry of a product shape: cached per context; otherwise
 // every candidate is timed on the live operands (one warm-up launch and two
 // or eight timed launches each; the products are idempotent) unless tuning is off
@@ -2302,6 +2296,7 @@ int pick_geometry(planc_ctx *ctx, int dtype, int trans, int NT, int tm, const St
     bool have = false;
     for (const Geometry &g : cands) {
       int rc = launch_stream(ctx, dtype, trans, NT, tm, p, g);  // warm-up (and workspace growth)
+      if (rc == PLANC_ENOMEM) continue;                         // no room for these partials
       if (rc) return rc;
       PLANC_HIP_CHECK(ctx, hipEventRecord(e0, ctx->stream));
       for (int r = 0; r < reps; ++r) {
@@ -2326,6 +2321,7 @@ int pick_geometry(planc_ctx *ctx, int dtype, int trans, int NT, int tm, const St
         have = true;
       }
     }
+    if (!have) best = make_geometry(p.L, p.K, trans, dtype, NT, best.cw, best.wk, 1, best.dual, best.shared);
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
   }
@@ -2477,14 +2473,17 @@ int thin_gemm(planc_ctx *ctx, int dtype, int trans, const void *A, long lda, lon
     p.oscale = oscale;
     // FP32 with a Khatri-Rao operand that the kernels cannot form from one
     // 16-byte load per four rows (three or more factors, a ragged first one,
-    // row scales): the K x k operand is written out once in FP32, while that
-    // stays small beside A (or small outright), and read as a plain one.  Its
-    // entries are the products that the kernels would form element by element
-    // per use (61 x 53 x 47 x 35, k = 17: 205 and 45 us products).
-    if (dtype == PLANC_F32 && thin_mode(th, rowscale) == THIN_SAFE &&
-        (L >= 2L * kc || K * kc <= (4L << 20))) {
-      float *kr = (float *)ws_get(ctx, 6, sizeof(float) * (size_t)K * kc);
-      if (!kr) return set_error(ctx, PLANC_ENOMEM, "thin_gemm: Khatri-Rao operand");
+    // row scales): the K x k operand is written out once in FP32 and read as a
+    // plain one.  Its entries are the products that the kernels would form element
+    // by element per use (61 x 53 x 47 x 35, k = 17: 205 and 45 us products).  It
+    // may take 16 MB, 256 MB where it is at most half of A's bytes, or a sixteenth
+    // of A's bytes; a larger one, or one that there is no room for, is formed by
+    // the element-wise kernels, which need no buffer.
+    const bool write_out = K * kc <= (4L << 20) || (L >= 2L * kc && K * kc <= (64L << 20)) || L >= 16L * kc;
+    float *kr = nullptr;
+    if (dtype == PLANC_F32 && thin_mode(th, rowscale) == THIN_SAFE && write_out)
+      kr = (float *)ws_try(ctx, 6, sizeof(float) * (size_t)K * kc);
+    if (kr) {
       form_thin_kernel<<<dim3((unsigned)std::min<long>((K + 255) / 256, 4096), (unsigned)kc), 256, 0, ctx->stream>>>(
           th, K, kr);
       PLANC_LAUNCH_CHECK(ctx);
@@ -2540,6 +2539,9 @@ int thin_gemm(planc_ctx *ctx, int dtype, int trans, const void *A, long lda, lon
       if (rc) return rc;
     }
     rc = launch_stream(ctx, dtype, trans, NT, tm, p, g);
+    if (rc == PLANC_ENOMEM)  // no room for the partials: the same kernel over all of K
+      rc = launch_stream(ctx, dtype, trans, NT, tm, p,
+                         make_geometry(L, K, trans, dtype, NT, g.cw, g.wk, 1, g.dual, g.shared));
     if (rc) return rc;
   }
   return PLANC_OK;
