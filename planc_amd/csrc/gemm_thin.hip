@@ -1857,6 +1857,8 @@ Geometry make_geometry(long L, long K, int trans, int dtype, int NT, int cw, int
   return g;
 }
 
+size_t partial_bytes(const Geometry &g) { return (size_t)g.nsplit * g.blocks_x * g.wgrp * g.tile_bytes; }
+
 constexpr long KRP_ONE_CHAIN = 512;  // rows of an FP32 tensor contraction that is not split
 constexpr long MAX_CHAIN = 1024;     // rows that one accumulator takes of an FP32 operand off the 16-byte grid
 
@@ -1873,15 +1875,19 @@ std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K,
   const long ksteps = (K + step - 1) / step;
   const int esz = dtype == PLANC_F32 ? 4 : 2;
   const double abytes = (double)L * (double)K * esz;
-  // K splits: the partial tiles' round trip may be 10% of A's bytes (20% for
-  // FP32, whose products are bound by MFMA as much as by reading and gain more
-  // from an even grid: 96^4, k = 48 TN 104 -> 90 us), or 8 MB (they stay in L2)
-  // where A is small and one pass of its few groups leaves most CUs idle; each
-  // wave keeps 8 k steps, 2 there (2000 x 1000, k = 20: 37 and 21 us products
-  // with one split of 32 waves).
+  // K splits: the partial tiles' round trip may be 10% of A's bytes (20% for a
+  // larger FP32 one, whose products are bound by MFMA as much as by reading and
+  // gain more from an even grid: 96^4, k = 48 TN 104 -> 90 us) and each wave keeps
+  // 8 k steps.  The static choice of an A of up to 64 MB (and 16-bit NN's few
+  // candidates) may go further, to 8 MB of partials (they stay in L2) and 2 steps,
+  // since one pass of its few groups leaves most CUs idle (2000 x 1000, k = 20: 37
+  // and 21 us products with one split of 32 waves).  It is not timed against other
+  // counts like it: they differ by less than their timings do, and with them the
+  // first call of five NMF-MU iterations there took 3.2 ms instead of 0.8 (later
+  // ones 0.27 either way), of NTF-HALS 61 x 53 x 47 x 35 5.2 instead of 0.7.
   const bool small = abytes <= (double)(64L << 20);
   const long min_steps = small ? 2 : 8;
-  const double share = dtype == PLANC_F32 ? 0.20 : 0.10;
+  const double share = dtype == PLANC_F32 && !small ? 0.20 : 0.10;
   // A tensor contraction in FP32 over at most KRP_ONE_CHAIN rows is summed in one
   // chain, whatever the operand's form: these are the smallest calls, where a
   // split gains nothing (NTF-HALS 20 x 18 x 16, K = 288: 261 us whole, 258 in nine
@@ -1906,10 +1912,13 @@ std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K,
     const long most = MAX_CHAIN * wk / st, steps = (K + st - 1) / st;
     return std::clamp((steps + most - 1) / most, 1L, 4096L);
   };
-  auto partials_fit = [&](const Geometry &g, double share) {
+  auto partials_fit = [&](const Geometry &g, double share, bool in_l2) {
     if (whole) return g.nsplit == 1;
     const double b = 2.0 * g.nsplit * g.groups * g.tile_bytes;
-    return b <= share * abytes || (small && b <= (double)(8L << 20));
+    return b <= share * abytes || (in_l2 && b <= (double)(8L << 20));
+  };
+  auto same_split = [](const Geometry &a, const Geometry &b) {
+    return a.cw == b.cw && a.wk == b.wk && a.nsplit == b.nsplit;
   };
   // Split counts tried for a grid of bx blocks: least, powers of two, and those that
   // make it 1, 2, 3 or 4 blocks per CU where no power of two comes within 8%
@@ -1946,7 +1955,7 @@ std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K,
       for (long ns = 1; ns <= 4096; ns *= 2) {
         Geometry g = make_geometry(L, K, trans, dtype, NT, 1, 1, ns, 0, sh);
         if (ns > 1 && (g.nsplit < ns || ksteps / g.nsplit < min_steps)) break;
-        if (ns > 1 && !partials_fit(g, share)) break;
+        if (ns > 1 && !partials_fit(g, share, small)) break;
         const long waves = g.blocks_x * 4 * g.nsplit;
         if (ns > 1 && waves > 16L * 1024) break;
         if (!out.empty() && waves < 2L * ctx->num_cu && ns < 4096) {
@@ -1981,7 +1990,7 @@ std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K,
     g = make_geometry(L, K, trans, dtype, NT, cw, wk, ns);
     while (g.blocks_x * 4 * ns < 4L * ctx->num_cu) {
       Geometry h = make_geometry(L, K, trans, dtype, NT, cw, wk, ns * 2);
-      if (!partials_fit(h, 0.06) || ksteps / ((long)h.nsplit * wk) < min_steps) break;
+      if (!partials_fit(h, 0.06, small) || ksteps / ((long)h.nsplit * wk) < min_steps) break;
       ns *= 2;
       g = h;
     }
@@ -1997,13 +2006,13 @@ std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K,
       for (long ns : split_counts(make_geometry(L, K, trans, dtype, NT, cw, wk, 1, dual).blocks_x, least)) {
         Geometry g = make_geometry(L, K, trans, dtype, NT, cw, wk, ns, dual);
         const bool p2 = (ns & (ns - 1)) == 0, more = ns > least;
-        if (more && ((p2 && g.nsplit < ns) || ksteps / ((long)g.nsplit * wk * (dual ? 2 : 1)) < min_steps)) break;
+        if (more && ((p2 && g.nsplit < ns) || ksteps / ((long)g.nsplit * wk * (dual ? 2 : 1)) < 8)) break;
         if (more && !p2 && g.nsplit < ns - ns / 8) continue;
-        if (more && !partials_fit(g, share)) break;
+        if (more && !partials_fit(g, share, false)) break;
         const long waves = g.blocks_x * 4 * g.nsplit;
         if (more && waves > 16L * 1024) break;
         if (waves < 2L * ctx->num_cu && ns < 4096) continue;  // too few waves: try more splits
-        out.push_back(g);
+        if (dual || !same_split(g, out[0])) out.push_back(g);
       }
     }
   // Block-shared thin operand: one k phase, four groups per block.
@@ -2016,9 +2025,9 @@ std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K,
       for (long ns : split_counts(make_geometry(L, K, trans, dtype, NT, cw, 1, 1, 1, 1).blocks_x, least)) {
         Geometry g = make_geometry(L, K, trans, dtype, NT, cw, 1, ns, 1, 1);
         const bool p2 = (ns & (ns - 1)) == 0, more = ns > least;
-        if (more && ((p2 && g.nsplit < ns) || sk / g.nsplit < min_steps)) break;
+        if (more && ((p2 && g.nsplit < ns) || sk / g.nsplit < 8)) break;
         if (more && !p2 && g.nsplit < ns - ns / 8) continue;
-        if (more && !partials_fit(g, share)) break;
+        if (more && !partials_fit(g, share, false)) break;
         const long waves = g.blocks_x * 4 * g.nsplit;
         if (more && waves > 16L * 1024) break;
         if (waves < 2L * ctx->num_cu && ns < 4096) continue;
@@ -2143,7 +2152,7 @@ int launch_stream(planc_ctx *ctx, int dtype, int trans, int NT, int tm, StreamPa
   // Partial tiles are indexed by padded group (blocks_x * wgrp >= groups).
   const long gpad = g.blocks_x * g.wgrp;
   if (g.nsplit > 1) {
-    p.part = (float *)ws_try(ctx, 0, (size_t)g.nsplit * gpad * g.tile_bytes);
+    p.part = (float *)ws_try(ctx, 0, partial_bytes(g));
     if (!p.part) return set_error(ctx, PLANC_ENOMEM, "thin_gemm: workspace");
   }
   dim3 grid((unsigned)g.blocks_x, (unsigned)g.nsplit);
@@ -2226,7 +2235,7 @@ int launch_stream(planc_ctx *ctx, int dtype, int trans, int NT, int tm, StreamPa
 
 // Picks the geometry of a product shape: cached per context; otherwise
 // every candidate is timed on the live operands (one warm-up launch and two
-// or eight timed launches each; the products are idempotent) unless tuning is off
+// timed launches each; the products are idempotent) unless tuning is off
 // (PLANC_AUTOTUNE=0) or the stream is being captured into a graph, where the
 // static choice is used.  PLANC_TUNE_LOG=1 prints each candidate's time.
 // fly_ok: the shared 16-bit NN kernel may form its thin operand on the fly
@@ -2274,9 +2283,10 @@ int pick_geometry(planc_ctx *ctx, int dtype, int trans, int NT, int tm, const St
     hipEvent_t e0, e1;
     PLANC_HIP_CHECK(ctx, hipEventCreate(&e0));
     PLANC_HIP_CHECK(ctx, hipEventCreate(&e1));
-    // Launches timed per candidate: two of a large product, eight of one that
-    // takes microseconds (A up to 64 MB).
-    const int reps = (double)p.L * (double)p.K * (dtype == PLANC_F32 ? 4 : 2) <= (double)(64L << 20) ? 8 : 2;
+    const int reps = 2;    // launches timed per candidate
+    // A large product's warm-up launch is timed too: a candidate that takes a
+    // quarter longer in it than the best so far is not timed further.
+    const bool large = (double)p.L * (double)p.K * (dtype == PLANC_F32 ? 4 : 2) > (double)(64L << 20);
     float pack_ms = 0.0f;  // as many pack launches
     if (dtype != PLANC_F32) {
       int prc = pack();
@@ -2295,9 +2305,17 @@ int pick_geometry(planc_ctx *ctx, int dtype, int trans, int NT, int tm, const St
     float best_ms = 0.0f;
     bool have = false;
     for (const Geometry &g : cands) {
-      int rc = launch_stream(ctx, dtype, trans, NT, tm, p, g);  // warm-up (and workspace growth)
-      if (rc == PLANC_ENOMEM) continue;                         // no room for these partials
+      if (g.nsplit > 1 && !ws_try(ctx, 0, partial_bytes(g))) continue;  // no room for these partials
+      if (large) PLANC_HIP_CHECK(ctx, hipEventRecord(e0, ctx->stream));
+      int rc = launch_stream(ctx, dtype, trans, NT, tm, p, g);  // warm-up
       if (rc) return rc;
+      if (large && have) {
+        float ms = 0.0f;
+        PLANC_HIP_CHECK(ctx, hipEventRecord(e1, ctx->stream));
+        PLANC_HIP_CHECK(ctx, hipEventSynchronize(e1));
+        PLANC_HIP_CHECK(ctx, hipEventElapsedTime(&ms, e0, e1));
+        if (ms * reps > 1.25f * best_ms) continue;
+      }
       PLANC_HIP_CHECK(ctx, hipEventRecord(e0, ctx->stream));
       for (int r = 0; r < reps; ++r) {
         rc = launch_stream(ctx, dtype, trans, NT, tm, p, g);
