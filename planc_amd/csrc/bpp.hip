@@ -14,8 +14,8 @@
 //  * the pair: with H = G^-1 formed once for all columns, a step solves the
 //    smaller of the passive and the complementary system (at most k / 2
 //    variables).  Taken where G's 1-norm condition is at most BPP_COND.
-//  * the passive system itself, for any other G and for columns the pair gives
-//    up (more than 5 k steps, or H b not finite).
+//  * the passive system itself, for any other G, for a few columns of a small G
+//    and for columns the pair gives up (more than 5 k steps, or H b not finite).
 // Bound by FP64 arithmetic and the lane broadcasts of the elimination (two
 // v_readlane per FMA).  One ANLS-BPP iteration at 65536 x 16384, k = 64 (81920
 // columns, BF16 products): 70.8 ms with a masked elimination of all k columns
@@ -229,8 +229,8 @@ __device__ inline double solve_selected(const double *M, int sel, double rhs, in
 // refinement is solved on the same set (at most BPP_REFINE), and the signs are
 // tested again on the final values.
 // PAIR = false is the form for any other G: every step solves the passive system
-// itself, from G, and nothing is refined.  It takes all columns where the inverse
-// is not usable, else only those that the pair gave up (iters < 0), and sets
+// itself, from G, and nothing is refined.  It takes all columns where there is no
+// inverse (info null) or it is not usable, else only those that the pair gave up (iters < 0), and sets
 // *failed_out for a column that needs more than maxit steps.
 constexpr int BPP_REFINE = 3;
 template <int KM, bool PAIR>
@@ -241,7 +241,7 @@ __global__ __launch_bounds__(512) void bpp_kernel(const double *G, const double 
   __shared__ double Gs[KM * LD], Hs[PAIR ? KM * LD : 1];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
   const long stride = (long)gridDim.x * nw;
-  const bool usable = info->ok != 0;
+  const bool usable = info && info->ok != 0;
   if (PAIR && !usable) return;
   if (!PAIR && usable) {
     int any = 0;
@@ -250,7 +250,7 @@ __global__ __launch_bounds__(512) void bpp_kernel(const double *G, const double 
       any |= iters[c] < 0;  // the block's columns, spread over its threads
     if (!__syncthreads_or(any)) return;
   }
-  const double hnorm = info->hnorm;
+  const double hnorm = PAIR ? info->hnorm : 0.0;
   for (int e = threadIdx.x; e < KM * KM; e += blockDim.x) {
     const int r = e % KM, c = e / KM;
     const bool in = r < k && c < k;
@@ -393,10 +393,24 @@ static void bpp_launch(planc_ctx *ctx, const double *G, const double *H, const B
                                                                   x_rs, 5 * k, iters, d_failed);
 }
 
+// A few right-hand sides of a Gram of up to 16 variables are solved by the general
+// kernel alone: its systems are as small as the pair's would be within a step of
+// four, and the call is bound by its launches.  16 variables, 60 columns: 37 us a
+// call, 42 in three launches; 2 variables, 5 columns: 29 and 34 (32 with a masked
+// elimination and a launch that gathered the failures).
+constexpr int BPP_DIRECT_K = 16;
+
 int bpp_solve(planc_ctx *ctx, const double *G, int k, const float *B, long b_cs, long b_rs, long nrhs,
               float *X, long x_cs, long x_rs, int *d_failed) {
   if (k <= 0 || k > 64) return set_error(ctx, PLANC_EUNSUPPORTED, "bpp: k must be 1..64");
   if (nrhs <= 0) return PLANC_OK;
+  if (k <= BPP_DIRECT_K && nrhs <= 4L * ctx->num_cu) {
+    const unsigned nb = (unsigned)((nrhs + 3) / 4);
+    bpp_kernel<16, false><<<nb, 256, 0, ctx->stream>>>(G, nullptr, nullptr, k, B, b_cs, b_rs, nrhs, X, x_cs, x_rs, 5 * k,
+                                                       nullptr, d_failed);
+    PLANC_LAUNCH_CHECK(ctx);
+    return PLANC_OK;
+  }
   // Workspace: H, its description, then the columns' pivot counts.
   double *H = (double *)ws_get(ctx, 10, sizeof(double) * 4096 + sizeof(BppInfo) + sizeof(int) * (size_t)nrhs);
   if (!H) return set_error(ctx, PLANC_ENOMEM, "bpp: workspace");

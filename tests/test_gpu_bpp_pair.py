@@ -1,7 +1,7 @@
 """Batched BPP from the Gram and its shared inverse, against the FP64 oracle,
 at the edges of its compact systems (k / 2 of 4, 8, ... 32 variables) and on
 both sides of the condition limit that selects it (past it the passive systems
-themselves are solved).
+themselves are solved, as for up to 1024 columns of at most 16 variables).
 
 Tolerance per column, relative to the column's largest entry: the results are
 FP32 (2^-24), and the solution is refined to 1e-10 of its largest entry, so
@@ -42,7 +42,7 @@ def problem(k, nrhs, kind):
 
 @pytest.mark.parametrize("kind", ["plain", "graded", "ill", "dead"])
 @pytest.mark.parametrize("k,nrhs", [(1, 5), (2, 70), (8, 33), (9, 64), (16, 70), (17, 1030), (31, 70), (33, 70),
-                                    (48, 1030), (63, 70), (64, 1030)])
+                                    (48, 1030), (63, 70), (64, 1030), (1, 1030), (7, 1024), (7, 1025), (16, 3000)])
 def test_bpp_pair_matches_oracle(ctx, k, nrhs, kind):
     if kind in ("ill", "dead") and k < 3:
         pytest.skip("needs other columns")
