@@ -230,8 +230,8 @@ __device__ inline double solve_selected(const double *M, int sel, double rhs, in
 // tested again on the final values.
 // PAIR = false is the form for any other G: every step solves the passive system
 // itself, from G, and nothing is refined.  It takes all columns where there is no
-// inverse (info null) or it is not usable, else only those that the pair gave up (iters < 0), and sets
-// *failed_out for a column that needs more than maxit steps.
+// inverse (info null) or it is not usable, else only those that the pair gave up
+// (iters < 0), and sets *failed_out for a column that needs more than maxit steps.
 constexpr int BPP_REFINE = 3;
 template <int KM, bool PAIR>
 __global__ __launch_bounds__(512) void bpp_kernel(const double *G, const double *H, const BppInfo *info, int k,
