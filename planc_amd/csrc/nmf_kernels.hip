@@ -633,8 +633,10 @@ __device__ inline bool column_collect(Exchange<NW> &ex, int par, const double *p
         tot = t;
         break;
       }
-      // The flag's load would add its latency to every poll: one in sixteen.
-      if (spin >= (1 << 20) ||
+      // The flag's load would add its latency to every poll: one in sixteen.  (2^21
+      // polls of a load each: over a second, for blocks that wait for another
+      // stream's kernel to leave its CUs.)
+      if (spin >= (1 << 21) ||
           ((spin & 15) == 15 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
         if (lane == 0) __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         ok = 0;
