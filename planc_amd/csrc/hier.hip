@@ -798,7 +798,7 @@ struct Engine {
   // level
   DBuf<long> perm, col_ptr, row_ptr, rstart, bsum, node_col0;
   DBuf<int> colmap, node_of_col, flag, row_node, row_orig, row_len, col_len, csr_col, csc_row,
-      cb_rows, cb_cols, lflag, llist, node_long0, row0, csc2csr, ent, ent_s, rid_of_entry, lcnt, seg_row;
+      cb_cols, lflag, llist, node_long0, row0, csc2csr, ent, ent_s, rid_of_entry, lcnt, seg_row;
   DBuf<long> seg_off, seg_b;
   DBuf<double> seg_part;
   DBuf<unsigned> key, key_s;
@@ -815,8 +815,8 @@ struct Engine {
     cval0.release(); perm.release(); col_ptr.release(); row_ptr.release(); rstart.release();
     bsum.release(); node_col0.release(); colmap.release(); node_of_col.release();
     flag.release(); row_node.release(); row_orig.release(); row_len.release();
-    col_len.release(); csr_col.release(); csc_row.release(); cb_rows.release();
-    cb_cols.release(); lflag.release(); llist.release(); row0.release();
+    col_len.release(); csr_col.release(); csc_row.release(); cb_cols.release();
+    lflag.release(); llist.release(); row0.release();
     csc2csr.release(); ent.release(); ent_s.release(); rid_of_entry.release(); key.release();
     key_s.release(); temp.release(); csr_val.release(); csc_val.release(); W.release();
     H.release(); part.release(); q.release(); z.release();
@@ -1121,12 +1121,10 @@ int planc_hiernmf_run(planc_ctx *ctx, const planc_hier_desc *desc, const long *h
     RC(E.ch_rows.get(ctx, chr.size()));
     RC(E.ch_cols.get(ctx, chc.size()));
     RC(E.ch_init.get(ctx, chi.size()));
-    RC(E.cb_rows.get(ctx, nn + 1));
     RC(E.cb_cols.get(ctx, nn + 1));
     if (!chr.empty()) PLANC_HIP_CHECK(ctx, up(E.ch_rows.p, chr.data(), sizeof(Chunk) * chr.size()));
     if (!chc.empty()) PLANC_HIP_CHECK(ctx, up(E.ch_cols.p, chc.data(), sizeof(Chunk) * chc.size()));
     PLANC_HIP_CHECK(ctx, up(E.ch_init.p, chi.data(), sizeof(Chunk) * chi.size()));
-    PLANC_HIP_CHECK(ctx, up(E.cb_rows.p, cbr.data(), sizeof(int) * (nn + 1)));
     PLANC_HIP_CHECK(ctx, up(E.cb_cols.p, cbc.data(), sizeof(int) * (nn + 1)));
     RC(E.part.get(ctx, 3 * std::max(chr.size(), chi.size()) + 3));
     RC(E.part_h.get(ctx, 3 * chc.size() + 3));

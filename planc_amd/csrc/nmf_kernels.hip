@@ -252,7 +252,6 @@ __device__ inline void load_gram(float (&Gt)[KM][PITCH], const double *G, int k)
   __syncthreads();
 }
 
-// s + sum_t h[t] * G(t, x), in t order, from the transposed LDS tile.
 // h . g over KM values of a 16-byte aligned g in LDS, in four chains.
 template <int KM>
 __device__ inline float dot_turned(const float (&h)[KM], const float *g) {
@@ -660,6 +659,12 @@ __global__ void fill_u64_kernel(unsigned long long *p, long n, unsigned long lon
   if (i < n) p[i] = v;
 }
 
+// Wavefronts per SIMD that the column sweep's 256-thread blocks are compiled for:
+// they set how many rows one launch can hold.
+constexpr int coop_waves(int KM, int RPT) {
+  return RPT == 1 ? (KM <= 16 ? 7 : KM <= 32 ? 5 : KM <= 48 ? 4 : 3) : KM <= 16 ? 5 : KM <= 32 ? 3 : 2;
+}
+
 // HALS over the columns of W with per-column normalisation (nmf/hals.hpp:
 // 89-102).  Persistent cooperative kernel: each thread owns RPT rows of W in
 // registers; one exchange per column x gives the column's sum of squares
@@ -677,15 +682,9 @@ __global__ void fill_u64_kernel(unsigned long long *p, long n, unsigned long lon
 // sync[1] the time-out flag.  BS: threads per block; larger blocks make fewer
 // exchange participants.  20011 rows, k = 50: 223 -> 84 us; a call for 20011 x
 // 16 99.5 -> 75.6 us, 65536 x 64 385 -> 167, 600000 x 8 133 -> 118.
-// Wavefronts per SIMD that 256-thread blocks are compiled for: they set how many
-// rows one launch can hold.
-constexpr int coop_waves(int KM, int RPT) {
-  return RPT == 1 ? (KM <= 16 ? 7 : KM <= 32 ? 5 : KM <= 48 ? 4 : 3) : KM <= 16 ? 5 : KM <= 32 ? 3 : 2;
-}
 template <int KM, int RPT, int BS>
-__global__ __launch_bounds__(BS, BS > 256 ? BS / 256 : coop_waves(KM, RPT)) void hals_cols_coop_kernel(float *W, long m, int k, long ldw,
-                                                            const float *AH, long ldah,
-                                                            const double *G, double *part, int *sync) {
+__global__ __launch_bounds__(BS, BS > 256 ? BS / 256 : coop_waves(KM, RPT)) void hals_cols_coop_kernel(
+    float *W, long m, int k, long ldw, const float *AH, long ldah, const double *G, double *part, int *sync) {
   __shared__ __attribute__((aligned(16))) float Gs[KM][2 * KM];
   __shared__ Exchange<BS / 64> ex;
   load_gram<KM, BS>(Gs, G, k);
@@ -1363,7 +1362,7 @@ static int gram_launch(planc_ctx *ctx, GramIn &in, int n, int k) {
   int nbmax = 1;
   size_t tot = 0;
   for (int i = 0; i < n; ++i) {
-    if (in.rows[i] < 0) return set_error(ctx, PLANC_EINVAL, "gram: k must be 1..64");
+    if (in.rows[i] < 0) return set_error(ctx, PLANC_EINVAL, "gram: negative row count");
     long nchunks = (in.rows[i] + GCR - 1) / GCR;
     if (nchunks == 0) nchunks = 1;
     in.nb[i] = (int)(nchunks < ctx->num_cu ? nchunks : ctx->num_cu);
