@@ -1859,6 +1859,7 @@ Geometry make_geometry(long L, long K, int trans, int dtype, int NT, int cw, int
 
 size_t partial_bytes(const Geometry &g) { return (size_t)g.nsplit * g.blocks_x * g.wgrp * g.tile_bytes; }
 
+constexpr long ONE_CHAIN = 128;      // rows of a product that is not split
 constexpr long KRP_ONE_CHAIN = 512;  // rows of an FP32 tensor contraction that is not split
 constexpr long MAX_CHAIN = 1024;     // rows that one accumulator takes of an FP32 operand off the 16-byte grid
 
@@ -1894,7 +1895,10 @@ std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K,
   // pieces), and HALS sweeps carry a change of the order of these sums into the
   // factors (there over 24 starts 4.1e-6 from FP64 on average whole, 1.8e-6 in
   // pieces, but a single start up to 1.2 times as far, of 20 x 16 x 16 2.8 times).
-  const bool whole = krp && dtype == PLANC_F32 && K <= KRP_ONE_CHAIN;
+  // Nor is any product over at most ONE_CHAIN rows split, whose chain is over
+  // before a second launch would begin (3000 x 100, k = 10, FP32 NN: 9.8 us a call
+  // in a row of them and 21.9 alone, 12.5 and 23.1 in pieces).
+  const bool whole = K <= ONE_CHAIN || (krp && dtype == PLANC_F32 && K <= KRP_ONE_CHAIN);
   // off_grid (an FP32 A whose columns do not all begin on 16 bytes): accumulators
   // take at most MAX_CHAIN rows of K each.  Every candidate has the splits that
   // this needs (4096 at most; their partials are up to 2 k / MAX_CHAIN, 12%, of A's

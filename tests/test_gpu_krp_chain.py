@@ -1,6 +1,6 @@
 """How the sums of FP32 products are cut into accumulator chains: a tensor
-contraction over at most 512 rows not at all, a product of an operand off the
-16-byte grid into at most 1024 rows.
+contraction over at most 512 rows and any product over at most 128 not at all, a
+product of an operand off the 16-byte grid into at most 1024 rows.
 
 The first term of every sum is 2^27 and the others are ones: an FP32
 accumulator that holds 2^27 (unit in the last place 16) takes a matrix step's
@@ -63,6 +63,14 @@ def chain_loss(c, trans, L, K, ld, off):
     B = torch.ones((5, K), device="cuda").t()
     out = (c.gemm_tn if trans else c.gemm_nn)(A, B)
     return (out.double() - 2.0 ** 27).min().item()
+
+
+@pytest.mark.parametrize("trans", [0, 1])
+@pytest.mark.parametrize("L,K", [(60, 50), (3000, 100), (5, 33), (200, 128)])
+def test_short_products_are_not_split(trans, L, K):
+    print("short product", trans, L, K, flush=True)
+    with P.Context(0) as c:
+        assert chain_loss(c, trans, L, K, 0, 0) == 0
 
 
 @pytest.mark.parametrize("tune", ["0", "1"])
