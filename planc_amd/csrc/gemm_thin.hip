@@ -1877,16 +1877,16 @@ std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K,
   const int esz = dtype == PLANC_F32 ? 4 : 2;
   const double abytes = (double)L * (double)K * esz;
   // K splits: the partial tiles' round trip may be 10% of A's bytes (20% for a
-  // larger FP32 one, whose products are bound by MFMA as much as by reading and
-  // gain more from an even grid: 96^4, k = 48 TN 104 -> 90 us) and each wave keeps
-  // 8 k steps.  The static choice of an A of up to 64 MB (and 16-bit NN's few
-  // candidates) may go further, to 8 MB of partials (they stay in L2) and 2 steps,
-  // since one pass of its few groups leaves most CUs idle (2000 x 1000, k = 20: 37
-  // and 21 us products with one split of 32 waves).  It is not timed against other
-  // counts like it: they differ by less than their timings do, and with them the
-  // first call of five NMF-MU iterations there took 3.2 ms instead of 0.8 (later
-  // ones 0.27 either way), of NTF-HALS 61 x 53 x 47 x 35 5.2 instead of 0.7.
-  const bool small = abytes <= (double)(64L << 20);
+  // large FP32 A, whose products are bound by MFMA as much as by reading and gain
+  // more from an even grid: 96^4, k = 48 TN 104 -> 90 us) and each wave keeps 8 k
+  // steps.  Up to 64 MB of A they may be 8 MB (they stay in L2) and a wave keeps 2
+  // steps, since one pass of its few groups leaves most CUs idle (2000 x 1000, k =
+  // 20: 37 and 21 us products with one split of 32 waves): in the static choice
+  // only.  To time such counts against each other made first calls long: five
+  // NMF-MU iterations on 2000 x 1000 3.2 ms instead of 0.5, on 4096 x 4096 12.5
+  // instead of 3.5, later ones no faster.
+  const double mb = abytes / (double)(1L << 20);
+  const bool small = mb <= 64, wide = mb >= 8 && mb < 32 && dtype == PLANC_F32;
   const long min_steps = small ? 2 : 8;
   const double share = dtype == PLANC_F32 && !small ? 0.20 : 0.10;
   // A tensor contraction in FP32 over at most KRP_ONE_CHAIN rows is summed in one
@@ -1981,12 +1981,15 @@ std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K,
     cws = {2, 4};
   else
     cws = {4};
-  // Static choice: one wave per SIMD or more, fewest partials.
+  // Static choice: one wave per SIMD or more, fewest partials.  An FP32 A of 8 to 32
+  // MB, which has few other candidates: at most two k phases and, as near as the
+  // bounds allow, a block per CU (61 x 53 x 47 x 35, k = 17, four phases and a power
+  // of two: NN 15.2 us, TN 17.0; so 13.7 and 14.1).
   {
     const int cw = cws[0];
     int wk = 1;
     Geometry g = make_geometry(L, K, trans, dtype, NT, cw, 1, 1);
-    while (wk < 4 && g.blocks_x * 4 < 4L * ctx->num_cu && ksteps >= 64L * wk) {
+    while (wk < (wide ? 2 : 4) && g.blocks_x * 4 < 4L * ctx->num_cu && ksteps >= 64L * wk) {
       wk *= 2;
       g = make_geometry(L, K, trans, dtype, NT, cw, wk, 1);
     }
@@ -1997,6 +2000,11 @@ std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K,
       if (!partials_fit(h, 0.06, small) || ksteps / ((long)h.nsplit * wk) < min_steps) break;
       ns *= 2;
       g = h;
+    }
+    const long even = ctx->num_cu / g.blocks_x;
+    if (wide && even > least_splits(step, wk) && (even > ns || ns * g.blocks_x > ctx->num_cu)) {
+      const Geometry h = make_geometry(L, K, trans, dtype, NT, cw, wk, even);
+      if (partials_fit(h, 0.06, true) && ksteps / ((long)h.nsplit * wk) >= min_steps) g = h;
     }
     out.push_back(g);
   }

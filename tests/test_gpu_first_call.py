@@ -2,8 +2,7 @@
 against the calls after it.  For a matrix or tensor of a few MB the choice may
 cost a few calls, not tens (a first call of five NMF-MU iterations on 2000 x 1000
 took 2.8 calls when this was written, of NTF-HALS 61 x 53 x 47 x 35 2.1; with every
-split count among the candidates 11 and 16).  The kernels' code is loaded by a
-context before."""
+split count among the candidates 11 and 16)."""
 import time
 
 import pytest
@@ -20,21 +19,22 @@ def rand(g, rows, cols):
 
 
 def first_and_later(make):
-    """Seconds of the first call in a new context and of the best of eight more."""
+    """Seconds of the first call in a new context (the best of three contexts,
+    after one that loads the kernels) and of the best of eight more."""
     if not torch.cuda.is_available():
         pytest.skip("no GPU")
-    times = []
-    for _ in range(2):
+    first, later = [], []
+    for i in range(4):
         with P.Context(0) as c:
             call = make(c)
-            times.clear()
-            for _ in range(9):
+            for j in range(9):
                 torch.cuda.synchronize()
                 t = time.perf_counter()
                 call()
                 torch.cuda.synchronize()
-                times.append(time.perf_counter() - t)
-    return times[0], min(times[1:])
+                if i:
+                    (later if j else first).append(time.perf_counter() - t)
+    return min(first), min(later)
 
 
 @pytest.mark.parametrize("m,n,k", [(2000, 1000, 20), (400, 16384, 16)])
