@@ -115,18 +115,19 @@ namespace planc {
 
 // Returns a device buffer of at least `bytes` for workspace slot `slot`.
 // Slots: 0 split-K partials, 1 Gram partials, 2 column-norm / HALS-sweep
-// partials, 3 dot partials, 4 loop float buffers, 5 loop double buffers,
-// 6 packed 16-bit thin operand, 7 16-bit copy of A / X, 8 column scales of that copy, 9 entry-point norms,
-// 10 BPP per-column iteration counts, 11 BPP failure flag, 12 CP-loss scalar,
-// 13 CP-gradient float buffers, 14 CP-gradient Grams, 15 loop-graph counter,
-// 16 transposed 16-bit copy of A / X, 17 HALS grid-barrier counter and flag,
-// 18 NTF mode-update partials (two-launch form), 19 / 20 the pieces of A's / A^T's long rows and 21 their
-// partial sums (sparse.hip), 22 AO-ADMM factor / partials,
-// 23 GNSym CG vectors, 24..31 sparse path (sparse.hip: k-major factor
-// copies, error partials, transposed CSR, sort keys / entries / temporary
-// storage), 32 NTF AO-ADMM duals, 33 NMF AO-ADMM duals, 34 dual norms,
-// 35 NES iterates, 36 NES factors (centres, previous, accelerated), 37 NES
-// lambdas.
+// partials, 3 dot partials, 4 loop float buffers, 5 loop double buffers, 6 packed
+// 16-bit or written-out FP32 thin operand, 7 16-bit copy of A / X, 8 column scales
+// of that copy, 9 entry-point norms, 10 BPP: the Gram's inverse and the columns'
+// iteration counts, 11 BPP failure flag, 12 CP-loss scalar, 13 CP-gradient float
+// buffers, 14 CP-gradient Grams, 15 loop-graph counter, 16 transposed 16-bit copy
+// of A / X, 17 HALS grid-barrier counter and flag, 18 NTF mode-update partials
+// (two-launch form), 19 / 20 the pieces of A's / A^T's long rows and 21 their
+// partial sums (sparse.hip), 22 AO-ADMM factor / partials, 23 GNSym CG vectors,
+// 24..31 sparse path (sparse.hip: k-major factor copies, error partials,
+// transposed CSR, sort keys / entries / temporary storage), 32 NTF AO-ADMM duals,
+// 33 NMF AO-ADMM duals, 34 dual norms, 35 NES iterates, 36 NES factors (centres,
+// previous, accelerated), 37 NES lambdas, 38 norms of a set of factors.
+// Null where there is no room (or PLANC_WS_MAX forbids the size).
 void *ws_get(planc_ctx *ctx, int slot, size_t bytes);
 // For buffers that the caller can do without: null too where the stream is being
 // captured and the slot would have to grow.

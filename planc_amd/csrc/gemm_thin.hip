@@ -5,9 +5,10 @@
 //
 // A is the big column-major operand (FP32, BF16 or FP16) streamed from HBM
 // exactly once per product; B is the thin K x k operand, either a factor
-// matrix or a Khatri-Rao product of up to six factors generated on the fly
-// (never stored in FP32).  k <= 64 per launch (wider k loops over 64-column
-// slices).
+// matrix or a Khatri-Rao product of up to six factors, generated on the fly
+// where a 16-byte load per four rows gives it and else, for FP32, written out
+// first while that is small (thin_gemm).  k <= 64 per launch (wider k loops over
+// 64-column slices).
 //
 // Streaming kernels (FP32 NN, FP32 TN, 16-bit TN).  The big operand goes
 // straight from HBM into MFMA operand registers, 16 bytes per lane, with no
@@ -39,8 +40,8 @@
 // (whole 128-byte lines per column per step) and the block-shared thin
 // operand (an LDS ring filled once per block).
 //
-// 16-bit NN with rows not in 16-byte groups (L % 8 != 0 or unaligned) uses an
-// LDS-transposing kernel with a separate split-K reduction.
+// 16-bit NN with rows not in groups of eight (L % 8 != 0) uses an LDS-transposing
+// kernel with a separate split-K reduction.
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
