@@ -27,7 +27,7 @@ void *ws_get(planc_ctx *ctx, int slot, size_t bytes) {
   if (w.bytes >= bytes) return w.ptr;
   // PLANC_WS_MAX (bytes) refuses larger buffers, as a device without the room would.
   const char *most = getenv("PLANC_WS_MAX");
-  if (most && bytes > strtoull(most, nullptr, 10)) return nullptr;
+  if (most && *most && bytes > strtoull(most, nullptr, 10)) return nullptr;
   if (w.ptr) {
     // Queued kernels may still read the old buffer.
     if (hipStreamSynchronize(ctx->stream) != hipSuccess) return nullptr;
