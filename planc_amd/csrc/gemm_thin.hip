@@ -1861,7 +1861,7 @@ Geometry make_geometry(long L, long K, int trans, int dtype, int NT, int cw, int
 size_t partial_bytes(const Geometry &g) { return (size_t)g.nsplit * g.blocks_x * g.wgrp * g.tile_bytes; }
 
 constexpr long ONE_CHAIN = 128;      // rows of a product that is not split
-constexpr long KRP_ONE_CHAIN = 512;  // rows of an FP32 tensor contraction that is not split
+constexpr long KRP_ONE_CHAIN = 320;  // rows of an FP32 tensor contraction that is not split
 constexpr long MAX_CHAIN = 1024;     // rows that one accumulator takes of an FP32 operand off the 16-byte grid
 
 // Candidate geometries: every (cw, wk) with K splits 1, 2, 4, ... while the
@@ -1892,10 +1892,11 @@ std::vector<Geometry> candidate_geometries(const planc_ctx *ctx, long L, long K,
   const double share = dtype == PLANC_F32 && !small ? 0.20 : 0.10;
   // A tensor contraction in FP32 over at most KRP_ONE_CHAIN rows is summed in one
   // chain, whatever the operand's form: these are the smallest calls, where a
-  // split gains nothing (NTF-HALS 20 x 18 x 16, K = 288: 261 us whole, 258 in nine
-  // pieces), and HALS sweeps carry a change of the order of these sums into the
-  // factors (there over 24 starts 4.1e-6 from FP64 on average whole, 1.8e-6 in
-  // pieces, but a single start up to 1.2 times as far, of 20 x 16 x 16 2.8 times).
+  // split gains little (NTF-HALS 20 x 18 x 16, K = 288: 261 us whole, 258 in nine
+  // pieces; at K = 480, NTF-BPP 34 x 36 x 15 x 32, k = 25, it is 466 against 441),
+  // and HALS sweeps carry a change of the order of these sums into the factors
+  // (there over 24 starts 4.1e-6 from FP64 on average whole, 1.8e-6 in pieces, but
+  // a single start up to 1.2 times as far, of 20 x 16 x 16 2.8 times).
   // Nor is any product over at most ONE_CHAIN rows split, whose chain is over
   // before a second launch would begin (3000 x 100, k = 10, FP32 NN: 9.8 us a call
   // in a row of them and 21.9 alone, 12.5 and 23.1 in pieces).
